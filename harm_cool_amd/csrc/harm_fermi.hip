@@ -1,6 +1,7 @@
 // harm_fermi.hip -- device batches of the tabulated-EOS generator's gas
 // physics (harm_fermi.hpp): generalized Fermi-Dirac integrals and the
-// per-species equations of state, one element per thread.
+// per-species equations of state, one element per thread, and whole table
+// points (harm_nse.hpp), three wavefronts per point.
 //
 // The 20-point Gauss-Legendre and Gauss-Laguerre rules are computed here once
 // (Newton iteration on P_20 and L_20 in long double, then rounded), not read
@@ -20,6 +21,7 @@
 #include "harm_nse.hpp"
 
 using harm::FermiRules;
+using harm::NseNodes;
 using harm::NseRules;
 
 namespace {
@@ -121,7 +123,6 @@ const NseRules &nse_rules()
             N.lx40[i] = (double)l40x[i];
             N.lw40[i] = (double)l40w[i];
         }
-        R.wave = 0;
     });
     return N;
 }
@@ -129,10 +130,8 @@ const NseRules &nse_rules()
 // The rules on the device, copied once per device before the first launch
 // (kernels read them in place rather than copying a by-value argument to
 // their stack for the noinline routines that take them by reference).
-__constant__ NseRules c_rules;
-__constant__ NseRules c_rules_group;  // the same rules for the lane-group-per-point kernel
-
-constexpr int GEN_G = harm::FD_GROUP;  // lanes per point of k_abundance_group
+__constant__ FermiRules c_rules;
+__constant__ NseNodes c_nodes;
 
 int upload_rules()
 {
@@ -143,11 +142,10 @@ int upload_rules()
     std::lock_guard<std::mutex> lk(mu);
     if (dev < 0 || dev >= 64) return harm_host::set_error("device index out of range", 3);
     if (!done[dev]) {
-        const NseRules &N = nse_rules();
-        FCHK(hipMemcpyToSymbol(HIP_SYMBOL(c_rules), &N, sizeof(NseRules)));
-        NseRules W = N;
-        W.f.wave = 1;
-        FCHK(hipMemcpyToSymbol(HIP_SYMBOL(c_rules_group), &W, sizeof(NseRules)));
+        NseNodes nodes;
+        harm::nse_nodes(nse_rules(), nodes);
+        FCHK(hipMemcpyToSymbol(HIP_SYMBOL(c_rules), &rules(), sizeof(FermiRules)));
+        FCHK(hipMemcpyToSymbol(HIP_SYMBOL(c_nodes), &nodes, sizeof(NseNodes)));
         done[dev] = true;
     }
     return 0;
@@ -161,7 +159,7 @@ __global__ void __launch_bounds__(TPB_F) k_fermi(const double *__restrict__ dk,
     const size_t i = (size_t)blockIdx.x * TPB_F + threadIdx.x;
     if (i >= n) return;
     double a, b, c;
-    harm::dfermi(dk[i], eta[i], theta[i], c_rules.f, a, b, c);
+    harm::dfermi(dk[i], eta[i], theta[i], c_rules, a, b, c);
     fd[i] = a;
     if (fdeta) fdeta[i] = b;
     if (fdtheta) fdtheta[i] = c;
@@ -174,7 +172,7 @@ __global__ void __launch_bounds__(TPB_F) k_eos_species(int kind, const double *_
     const size_t i = (size_t)blockIdx.x * TPB_F + threadIdx.x;
     if (i >= n) return;
     auto I = [&](int k) { return in[(size_t)k * n + i]; };
-    const FermiRules &R = c_rules.f;
+    const FermiRules &R = c_rules;
     double e = 0., p = 0., s = 0.;
     switch (kind) {
     case HARM_EOS_NPE:
@@ -204,25 +202,36 @@ __global__ void __launch_bounds__(64) k_abundance(const double *__restrict__ rho
     const size_t i = (size_t)blockIdx.x * 64 + threadIdx.x;
     if (i >= n) return;
     double v[6];
-    harm::abundance(rho[i], T[i], hdfac[i], c_rules, v[0], v[1], v[2], v[3], v[4], v[5]);
+    harm::abundance(harm::NseSerial(c_nodes), rho[i], T[i], hdfac[i], v);
     for (int k = 0; k < 6; k++) out[(size_t)k * n + i] = v[k];
 }
 
-// One cooling-table point per group of GEN_G lanes (64 / GEN_G points per
-// wavefront): every lane of a group runs its point's chain (the same values,
-// so the same branches) and the group shares each dfermi's quadrature nodes
-// (dfermi_group), which shortens the chain of the slowest points -- the ones
-// whose Newton solves run long -- and spreads the points over the chip.
-__global__ void __launch_bounds__(64) k_abundance_group(const double *__restrict__ rho,
-                                                        const double *__restrict__ T,
-                                                        const double *__restrict__ hdfac, double *__restrict__ out,
-                                                        size_t n)
+// One cooling-table point per block of three wavefronts (NseWave).  Bound by
+// the latency of a point's chain of Newton trials (exp, sqrt and division of
+// ten nodes per lane) where points are few, and by the issue of those 64-bit
+// instructions where they are many.  With eight lanes per point, one integral
+// at a time by pow() with its derivatives, the emissivities formed in each of
+// the ten trapping passes and every solve run to its 200th trial, a 200x200
+// table over rho 1e6-1e13, T 1e9-1e12 took 21.3 s and a 40x40 one over its
+// dense part (rho > 1e10, T 1e10-1e11) 125 ms; now 0.10 s and 3.1 ms.  A single
+// 4x4 patch at T < 3e9 K, whose outer solves cycle, went from 12 s to 4 ms.
+constexpr int TPB_P = 192;
+__global__ void __launch_bounds__(TPB_P) k_abundance_wave(const double *__restrict__ rho,
+                                                          const double *__restrict__ T,
+                                                          const double *__restrict__ hdfac,
+                                                          double *__restrict__ out, size_t n)
 {
-    const size_t i = (size_t)blockIdx.x * (64 / GEN_G) + threadIdx.x / GEN_G;
-    if (i >= n) return;  // whole groups leave together
+    __shared__ double nodes[320], ex[3];
+    for (int k = threadIdx.x; k < 320; k += TPB_P) nodes[k] = (&c_nodes.fd[0][0])[k];
+    __syncthreads();
+    const size_t i = blockIdx.x;
+    harm::NseWave pol;
+    pol.fd = (const double(*)[2])nodes;
+    pol.rate = (const double(*)[2])(nodes + 160);
+    pol.ex = ex;
     double v[6];
-    harm::abundance(rho[i], T[i], hdfac[i], c_rules_group, v[0], v[1], v[2], v[3], v[4], v[5]);
-    if (threadIdx.x % GEN_G == 0)
+    harm::abundance(pol, rho[i], T[i], hdfac[i], v);
+    if (threadIdx.x == 0)
         for (int k = 0; k < 6; k++) out[(size_t)k * n + i] = v[k];
 }
 
@@ -268,9 +277,8 @@ int harm_eos_point_batch(const double *rho, const double *T, const double *hdfac
     hipStream_t s = (hipStream_t)stream;
     int rc = upload_rules();
     if (rc) return rc;
-    const size_t nblk = (n + 64 / GEN_G - 1) / (64 / GEN_G);
-    if (nblk > 0x7fffffffu) return harm_host::set_error("harm_eos_point_batch: too many points for one call", 3);
-    hipLaunchKernelGGL(k_abundance_group, dim3((unsigned)nblk), dim3(64), 0, s, rho, T, hdfac, out, n);
+    if (n > 0x7fffffffu) return harm_host::set_error("harm_eos_point_batch: too many points for one call", 3);
+    hipLaunchKernelGGL(k_abundance_wave, dim3((unsigned)n), dim3(TPB_P), 0, s, rho, T, hdfac, out, n);
     FCHK(hipGetLastError());
     FCHK(hipStreamSynchronize(s));
     return 0;

@@ -421,10 +421,9 @@ int harm_fermi_batch(const double *dk, const double *eta, const double *theta, d
 int harm_fermi_rules(double *out /* 100 */);
 /* One cooling-table point per element (abundance.f90:6-243): rho [g cm^-3], T
  * [K] and the disk-height factor HdFac -> out[6][n]: e, p [erg cm^-3], Qnu
- * [erg cm^-2 s^-1], optical depth tau, n_e-, n_e+ [fm^-3].  The chemical
- * equilibrium solve, the neutrino trapping iteration and all rates of a point
- * run in one group of lanes, which shares each Fermi-Dirac integral's
- * quadrature nodes (the sums in the serial order). */
+ * [erg cm^-2 s^-1], optical depth tau, n_e-, n_e+ [fm^-3].  Three wavefronts
+ * per point: they take the three proton fractions of the equilibrium solve's
+ * central difference, and their lanes the quadrature nodes. */
 int harm_eos_point_batch(const double *rho, const double *T, const double *hdfac, double *out, size_t n,
                          void *stream);
 /* The same with one point per thread (every integral serial); the same bits. */
