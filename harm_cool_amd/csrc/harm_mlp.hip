@@ -7,11 +7,13 @@
 //   loss      L = 1/(2B) sum_b mask_b |O_b - T_b|^2
 //   backward  dO = mask (O - T) / B;  dW_l = dZ_l^T H_{l-1};  db_l = dZ_l^T 1
 //             dZ_{l-1} = (dZ_l W_l) * (1 - H_{l-1}^2)
-// Every product is one launch of k_gemm (v_mfma_f32_16x16x4_f32, one 16x16
-// tile per wavefront, split-K over the batch for the weight gradients with a
-// fixed-order reduction, so a training step is deterministic).
+// One launch (k_train) takes the batch through all of that with the activations
+// in registers and LDS, every product on v_mfma_f32_16x16x4_f32; a second
+// (k_adam_gather) folds the blocks' gradients in a fixed order, so that a training
+// step is deterministic, applies Adam, and draws the next step's rows.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -34,10 +36,14 @@ struct harm_mlp {
     int vsq_from_W;
     float loss_w[2];  // weights of the two outputs in the training loss
     long long adam_t;
-    // training workspace, sized for wsB rows
+    // training workspace: the drawn rows of a batch (wsB of them), the blocks'
+    // gradients, the losses of the steps not yet copied to the host
     int wsB;
-    float *X, *T, *H1, *H2, *H3, *O, *dO, *dZa, *dZb, *ones, *part, *lossp;
+    float *X, *T, *part;
     uint8_t *M;
+    float4 *rec;  // a training set's records, recN of them
+    size_t recN;
+    double *lossd;
     double *normp;
 };
 
@@ -54,110 +60,331 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
                                         2);                                                                \
     } while (0)
 
-constexpr int KCHUNK = 256;  // split-K length of the weight-gradient products
+// k_train: one block of 8 wavefronts per CU, each wavefront on 16 batch rows at a
+// time.  A layer's activations are kept transposed (neurons x rows): with q = lane /
+// 16 and c = lane % 16 the D layout of a 16x16 tile (register r: neuron 4q + r of row
+// c) is the B operand of the next product for the contraction order {4q + r : q}, so
+// the forward and the backward chain run from register to register, the weights
+// coming from LDS (rows of TR_LD floats: 16-byte reads along a row and 4-byte reads
+// across rows both touch every bank once).  A weight gradient contracts over the batch
+// rows, for which D would have to be rows x neurons: each layer's h and dZ pass
+// through LDS once and are read back in that order.  The 8 + 128 accumulator tiles of
+// a wavefront (dW1 with db1 as its ninth column, dW2, dW3) stay in registers over all
+// its rows.
+//
+// Bound by the FP32 matrix cores: 408 MFMA of 32 cycles per 16 rows.  Two wavefronts
+// a SIMD (256 registers each) let one's 48 tanhf a lane run beside the other's
+// products.
+constexpr int TR_WAVES = 8, TR_BLOCKS = 256;
+constexpr int TR_LD = MLP_NH + 4;
+constexpr int TR_W1 = 0, TR_W2 = TR_W1 + MLP_NH * MLP_NIN, TR_W3 = TR_W2 + MLP_NH * TR_LD,
+              TR_BIAS = TR_W3 + MLP_NH * TR_LD, TR_W4 = TR_BIAS + 3 * MLP_NH, TR_B4 = TR_W4 + MLP_NOUT * MLP_NH,
+              TR_SCR = TR_B4 + 4;
+constexpr int TR_TILE = 16 * TR_LD, TR_SCRATCH = 3 * TR_TILE + 2 * 16;  // per wavefront: h1, h2, h3 or dZ; dO
+// A wavefront's gradient as rows of 64 lanes: dW2 64, dW3 64, dW1 16, dW4 8, db2 4,
+// db3 4, db4 2, loss 1.  The block's waves are added 55 rows at a time.
+constexpr int TR_ROWS = 163, TR_FOLD = 55;
+static_assert(TR_WAVES * TR_FOLD * 64 <= TR_SCR + TR_WAVES * TR_SCRATCH && 3 * TR_FOLD >= TR_ROWS, "fold buffer");
+static_assert((TR_SCR + TR_WAVES * TR_SCRATCH) * 4 <= 160 * 1024, "LDS");
 
-// C(m,n) = sum_k A(m,k) B(k,n), strided operands; epilogue:
-//   0: C = acc   1: C = acc + bias[n]   2: C = tanh(acc + bias[n])
-//   3: C = acc * (1 - H(m,n)^2)
-// grid = (ceil(N/16), ceil(M/16), splits), 64 threads; split z covers
-// k in [z*kchunk, min(K, (z+1)*kchunk)) and writes C + z*cz.
-struct GemmArgs {
-    int M, N, K, kchunk, epi;
-    const float *A;
-    long sam, sak;
-    const float *B;
-    long sbk, sbn;
-    float *C;
-    long scm, scn, cz;
-    const float *bias;
-    const float *H;
-    long shm, shn;
-};
-
-__global__ void __launch_bounds__(64) k_gemm(GemmArgs a)
+// LDS written by some lanes of a wavefront and read by others of the same one: its
+// LDS operations complete in order, so only the compiler has to keep it.
+__device__ __forceinline__ void wave_lds_fence()
 {
-    const int lane = threadIdx.x, r = lane & 15, q = lane >> 4;
-    const int m0 = blockIdx.y * 16, n0 = blockIdx.x * 16;
-    const int kb = blockIdx.z * a.kchunk;
-    const int ke = min(a.K, kb + a.kchunk);
-    const int mr = m0 + r, nr = n0 + r;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int k = kb; k < ke; k += 4) {
-        const int kk = k + q;
-        const float av = (mr < a.M && kk < ke) ? a.A[mr * a.sam + kk * a.sak] : 0.f;
-        const float bv = (nr < a.N && kk < ke) ? a.B[kk * a.sbk + nr * a.sbn] : 0.f;
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc, 0, 0, 0);
-    }
-    float *C = a.C + (size_t)blockIdx.z * a.cz;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ f32x4 lds4(const float *p) { return *reinterpret_cast<const f32x4 *>(p); }
+
+// Keeps the scheduler from gathering the loads of several products in registers.
+__device__ __forceinline__ void tr_stage() { __builtin_amdgcn_sched_barrier(0); }
+
+// a = b + W h: a, h in D layout, 64 neurons each.
+__device__ __forceinline__ void tr_dense(const float *W, const float *b, int q, int c, const f32x4 (&h)[4],
+                                         f32x4 (&a)[4])
+{
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int m = m0 + 4 * q + i, n = nr;
-        if (m < a.M && n < a.N) {
-            float v = acc[i];
-            if (a.epi == 1 || a.epi == 2) v += a.bias[n];
-            if (a.epi == 2) v = tanhf(v);
-            if (a.epi == 3) {
-                const float h = a.H[m * a.shm + n * a.shn];
-                v *= (1.f - h * h);
+    for (int t = 0; t < 4; t++) a[t] = lds4(b + 16 * t + 4 * q);
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        if (s == 2) tr_stage();
+        f32x4 w[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) w[t] = lds4(W + (16 * t + c) * TR_LD + 16 * s + 4 * q);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) a[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][r], h[s][r], a[t], 0, 0, 0);
+    }
+}
+
+// a = W^T dz
+__device__ __forceinline__ void tr_dense_t(const float *W, int q, int c, const f32x4 (&dz)[4], f32x4 (&a)[4])
+{
+#pragma unroll
+    for (int t = 0; t < 4; t++) a[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        tr_stage();
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+                a[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(W[(16 * s + 4 * q + r) * TR_LD + 16 * t + c], dz[s][r],
+                                                            a[t], 0, 0, 0);
+    }
+}
+
+// dW += dZ^T h and db += dZ^T 1 over the 16 rows of two LDS tiles.
+__device__ __forceinline__ void tr_wgrad(const float *dz, const float *h, int q, int c, f32x4 (&dW)[4][4],
+                                         float (&db)[4])
+{
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        if (r == 2) tr_stage();
+        float a[4], b[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            a[t] = dz[(4 * q + r) * TR_LD + 16 * t + c];
+            b[t] = h[(4 * q + r) * TR_LD + 16 * t + c];
+            db[t] += a[t];
+        }
+#pragma unroll
+        for (int o = 0; o < 4; o++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                dW[o][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[o], b[i], dW[o][i], 0, 0, 0);
+    }
+}
+
+// tanh without a branch (the library's takes one of two per lane, so a wavefront runs
+// both and the loads around them wait): an odd polynomial below 0.6, fitted there to a
+// relative error of 2e-9, and 1 - 2 / (exp(2|x|) + 1) above.  TANH_MEASURED
+__device__ __forceinline__ float tr_tanhf(float x)
+{
+    const float ax = __builtin_fabsf(x), y = x * x;
+    float p = -0.00589516f;
+    p = __builtin_fmaf(p, y, 0.02079597f);
+    p = __builtin_fmaf(p, y, -0.05378383f);
+    p = __builtin_fmaf(p, y, 0.13331924f);
+    p = __builtin_fmaf(p, y, -0.33333298f);
+    const float lo = __builtin_fmaf(ax * y, p, ax);
+    const float e = __builtin_amdgcn_exp2f(ax * 2.88539008f) + 1.f;  // 2 log2(e)
+    float r = __builtin_amdgcn_rcpf(e);
+    r = e < 1e30f ? __builtin_fmaf(__builtin_fmaf(-e, r, 1.f), r, r) : r;
+    const float hi = __builtin_fmaf(-2.f, r, 1.f);
+    return __builtin_copysignf(ax < 0.6f ? lo : hi, x);
+}
+
+// h = tanh(a), also into the LDS tile (rows x neurons)
+__device__ __forceinline__ void tr_tanh(const f32x4 (&a)[4], f32x4 (&h)[4], float *tile, int q, int c)
+{
+    tr_stage();
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) h[t][r] = tr_tanhf(a[t][r]);
+        if (tile) *reinterpret_cast<f32x4 *>(tile + c * TR_LD + 16 * t + 4 * q) = h[t];
+    }
+}
+
+// dz = a (1 - h^2) with h from its LDS tile, into the tile dzt
+__device__ __forceinline__ void tr_dtanh(const f32x4 (&a)[4], const float *ht, f32x4 (&dz)[4], float *dzt, int q,
+                                         int c)
+{
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const f32x4 h = lds4(ht + c * TR_LD + 16 * t + 4 * q);
+#pragma unroll
+        for (int r = 0; r < 4; r++) dz[t][r] = a[t][r] * (1.f - h[r] * h[r]);
+        *reinterpret_cast<f32x4 *>(dzt + c * TR_LD + 16 * t + 4 * q) = dz[t];
+    }
+}
+
+// GRAD: the blocks' gradients and losses into part[block][TR_ROWS][64]; otherwise the
+// outputs Y[B][2].  Any grid of at most TR_BLOCKS blocks covers the batch.
+template <bool GRAD>
+__global__ void __launch_bounds__(TR_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
+k_train(const float *__restrict__ P, const float *__restrict__ X, const float *__restrict__ T,
+        const uint8_t *__restrict__ M, int B, float lw0, float lw1, float *__restrict__ part, float *__restrict__ Y)
+{
+    __shared__ __attribute__((aligned(16))) float lds[TR_SCR + (GRAD ? TR_WAVES * TR_SCRATCH : 0)];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, c = lane & 15;
+    for (int k = tid; k < MLP_NH * MLP_NH; k += TR_WAVES * 64) {
+        lds[TR_W2 + (k >> 6) * TR_LD + (k & 63)] = P[MLP_W2 + k];
+        lds[TR_W3 + (k >> 6) * TR_LD + (k & 63)] = P[MLP_W3 + k];
+    }
+    for (int k = tid; k < MLP_NH * MLP_NIN; k += TR_WAVES * 64) lds[TR_W1 + k] = P[MLP_W1 + k];
+    if (tid < MLP_NH) {
+        lds[TR_BIAS + tid] = P[MLP_B1 + tid];
+        lds[TR_BIAS + MLP_NH + tid] = P[MLP_B2 + tid];
+        lds[TR_BIAS + 2 * MLP_NH + tid] = P[MLP_B3 + tid];
+    } else if (tid < MLP_NH + MLP_NOUT * MLP_NH + MLP_NOUT) {
+        lds[TR_W4 + tid - MLP_NH] = P[MLP_W4 + tid - MLP_NH];  // W4 and b4 follow each other in both
+    }
+    __syncthreads();
+
+    float *t1 = lds + TR_SCR + (GRAD ? wave * TR_SCRATCH : 0), *t2 = t1 + TR_TILE, *t3 = t2 + TR_TILE,
+          *tdo = t3 + TR_TILE;
+    f32x4 dW1[4], dW2[4][4], dW3[4][4];
+    float dW4[2][4], db2[4], db3[4], db4[2] = {0.f, 0.f}, loss = 0.f;
+#pragma unroll
+    for (int o = 0; o < 4; o++) {
+        dW1[o] = f32x4{0.f, 0.f, 0.f, 0.f};
+        db2[o] = db3[o] = dW4[0][o] = dW4[1][o] = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) dW2[o][i] = dW3[o][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+
+    const int ntile = (B + 15) / 16;
+    for (int tile = blockIdx.x + gridDim.x * wave; tile < ntile; tile += gridDim.x * TR_WAVES) {
+        asm volatile("" ::: "memory");  // weights are read where they are used, not kept in registers over the rows
+        const int z = 16 * tile + c;
+        const bool in = z < B;
+        f32x4 a[4], h[4];
+        {
+            const float x0 = in ? X[(size_t)z * MLP_NIN + 2 * q] : 0.f;
+            const float x1 = in ? X[(size_t)z * MLP_NIN + 2 * q + 1] : 0.f;
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                a[t] = lds4(lds + TR_BIAS + 16 * t + 4 * q);
+                const float *w = lds + TR_W1 + (16 * t + c) * MLP_NIN + 2 * q;
+                a[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[0], x0, a[t], 0, 0, 0);
+                a[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[1], x1, a[t], 0, 0, 0);
             }
-            C[m * a.scm + n * a.scn] = v;
+        }
+        tr_tanh(a, h, GRAD ? t1 : nullptr, q, c);
+        tr_dense(lds + TR_W2, lds + TR_BIAS + MLP_NH, q, c, h, a);
+        tr_tanh(a, h, GRAD ? t2 : nullptr, q, c);
+        tr_dense(lds + TR_W3, lds + TR_BIAS + 2 * MLP_NH, q, c, h, a);
+        tr_tanh(a, h, GRAD ? t3 : nullptr, q, c);
+        float o0 = 0.f, o1 = 0.f;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const f32x4 w0 = lds4(lds + TR_W4 + 16 * t + 4 * q), w1 = lds4(lds + TR_W4 + MLP_NH + 16 * t + 4 * q);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                o0 += w0[r] * h[t][r];
+                o1 += w1[r] * h[t][r];
+            }
+        }
+        o0 += __shfl_xor(o0, 16, 64);
+        o1 += __shfl_xor(o1, 16, 64);
+        o0 += __shfl_xor(o0, 32, 64);
+        o1 += __shfl_xor(o1, 32, 64);
+        o0 += lds[TR_B4];
+        o1 += lds[TR_B4 + 1];
+        if (!GRAD) {
+            if (q == 0 && in) {
+                Y[(size_t)z * MLP_NOUT] = o0;
+                Y[(size_t)z * MLP_NOUT + 1] = o1;
+            }
+            continue;
+        }
+        float d0 = 0.f, d1 = 0.f;
+        if (in) {
+            const float w = M ? (float)M[z] : 1.f;
+            const float e0 = o0 - T[(size_t)z * MLP_NOUT], e1 = o1 - T[(size_t)z * MLP_NOUT + 1];
+            d0 = w * lw0 * e0 / (float)B;
+            d1 = w * lw1 * e1 / (float)B;
+            if (q == 0) {
+                loss += w * (lw0 * e0 * e0 + lw1 * e1 * e1);
+                db4[0] += d0;
+                db4[1] += d1;
+            }
+        }
+        if (q == 0) {
+            tdo[2 * c] = d0;
+            tdo[2 * c + 1] = d1;
+        }
+        wave_lds_fence();
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float e0 = tdo[2 * (4 * q + r)], e1 = tdo[2 * (4 * q + r) + 1];
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const float hz = t3[(4 * q + r) * TR_LD + 16 * t + c];
+                dW4[0][t] += e0 * hz;
+                dW4[1][t] += e1 * hz;
+            }
+        }
+        f32x4 dz[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const f32x4 w0 = lds4(lds + TR_W4 + 16 * t + 4 * q), w1 = lds4(lds + TR_W4 + MLP_NH + 16 * t + 4 * q);
+#pragma unroll
+            for (int r = 0; r < 4; r++) a[t][r] = w0[r] * d0 + w1[r] * d1;
+        }
+        wave_lds_fence();
+        tr_dtanh(a, t3, dz, t3, q, c);
+        wave_lds_fence();
+        tr_wgrad(t3, t2, q, c, dW3, db3);
+        tr_dense_t(lds + TR_W3, q, c, dz, a);
+        wave_lds_fence();
+        tr_dtanh(a, t2, dz, t3, q, c);
+        wave_lds_fence();
+        tr_wgrad(t3, t1, q, c, dW2, db2);
+        tr_dense_t(lds + TR_W2, q, c, dz, a);
+        wave_lds_fence();
+        tr_dtanh(a, t1, dz, t3, q, c);
+        wave_lds_fence();
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int zr = 16 * tile + 4 * q + r;
+            const float x = c < MLP_NIN ? (zr < B ? X[(size_t)zr * MLP_NIN + c] : 0.f) : (c == MLP_NIN ? 1.f : 0.f);
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+                dW1[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(t3[(4 * q + r) * TR_LD + 16 * t + c], x, dW1[t], 0, 0, 0);
+        }
+        wave_lds_fence();  // the next rows write the tiles that were read here
+    }
+    if (!GRAD) return;
+
+    auto over_q = [](float v) {
+        v += __shfl_xor(v, 16, 64);
+        return v + __shfl_xor(v, 32, 64);
+    };
+    auto over_lanes = [](float v) {
+#pragma unroll
+        for (int s = 1; s < 64; s <<= 1) v += __shfl_xor(v, s, 64);
+        return v;
+    };
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        dW4[0][t] = over_q(dW4[0][t]);
+        dW4[1][t] = over_q(dW4[1][t]);
+        db2[t] = over_q(db2[t]);
+        db3[t] = over_q(db3[t]);
+    }
+    db4[0] = over_lanes(db4[0]);
+    db4[1] = over_lanes(db4[1]);
+    loss = over_lanes(loss);
+    auto row = [&](int k) -> float {  // k is a constant after unrolling
+        if (k < 64) return dW2[k >> 4][(k >> 2) & 3][k & 3];
+        if (k < 128) return dW3[(k - 64) >> 4][(k >> 2) & 3][k & 3];
+        if (k < 144) return dW1[(k - 128) >> 2][k & 3];
+        if (k < 152) return dW4[(k - 144) >> 2][k & 3];
+        if (k < 156) return db2[k & 3];
+        if (k < 160) return db3[k & 3];
+        return k == 160 ? db4[0] : k == 161 ? db4[1] : loss;
+    };
+    float *out = part + (size_t)blockIdx.x * (TR_ROWS * 64);
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < TR_FOLD; k++)
+            if (f * TR_FOLD + k < TR_ROWS) lds[(wave * TR_FOLD + k) * 64 + lane] = row(f * TR_FOLD + k);
+        __syncthreads();
+        const int n = (f == 2 ? TR_ROWS - 2 * TR_FOLD : TR_FOLD) * 64;
+        for (int k = tid; k < n; k += TR_WAVES * 64) {
+            float s = 0.f;
+#pragma unroll
+            for (int w = 0; w < TR_WAVES; w++) s += lds[w * TR_FOLD * 64 + k];
+            out[f * TR_FOLD * 64 + k] = s;
         }
     }
-}
-
-// out[i] = sum_z part[z*stride + i], z = 0..nsplit-1 in order.
-__global__ void k_reduce_splits(const float *__restrict__ part, int nsplit, long stride, int count,
-                                float *__restrict__ out)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    float s = 0.f;
-    for (int z = 0; z < nsplit; z++) s += part[(size_t)z * stride + i];
-    out[i] = s;
-}
-
-__global__ void k_fill(float *__restrict__ p, float v, int n)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
-// dO = mask (O - T) / B; per-block partial sums of mask |O - T|^2.
-__global__ void __launch_bounds__(256) k_loss(const float *__restrict__ O, const float *__restrict__ T,
-                                              const uint8_t *__restrict__ M, int B, float lw0, float lw1,
-                                              float *__restrict__ dO, float *__restrict__ lossp)
-{
-    __shared__ float red[256];
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    float l = 0.f;
-    if (b < B) {
-        const float w = M ? (float)M[b] : 1.f;
-        const float e0 = O[2 * b] - T[2 * b], e1 = O[2 * b + 1] - T[2 * b + 1];
-        dO[2 * b] = w * lw0 * e0 / (float)B;
-        dO[2 * b + 1] = w * lw1 * e1 / (float)B;
-        l = w * (lw0 * e0 * e0 + lw1 * e1 * e1);
-    }
-    red[threadIdx.x] = l;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) lossp[blockIdx.x] = red[0];
-}
-
-__global__ void k_adam(float *__restrict__ p, float *__restrict__ m, float *__restrict__ v,
-                       const float *__restrict__ g, int n, float lr, float bc1, float bc2)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = 0.9f * m[i] + 0.1f * gi;
-    const float vi = 0.999f * v[i] + 0.001f * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float mh = mi / bc1, vh = vi / bc2;
-    p[i] -= lr * mh / (sqrtf(vh) + 1e-8f);
 }
 
 // Packs the BF16 A operands and the bias table of harm_mlp.hpp from the
@@ -210,20 +437,129 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long x)
     return x ^ (x >> 31);
 }
 
-__global__ void __launch_bounds__(256) k_gather(const double *__restrict__ feat, const double *__restrict__ targ,
-                                                const uint8_t *__restrict__ valid, size_t n, const double *norm,
-                                                unsigned long long seed, int B, float *__restrict__ X,
-                                                float *__restrict__ T, uint8_t *__restrict__ M)
+// A training set and the draw of one batch from it.  A row lies in eleven arrays, and
+// at random rows each of its numbers costs a cache line: where a call draws enough of
+// them (see harm_mlp_train) the set is first written as records of the very floats
+// that a draw forms, 8 inputs, 2 targets and the mask in 48 bytes.
+struct Draw {
+    const double *feat, *targ;
+    const uint8_t *valid;
+    const float4 *rec;  // the records, or null
+    size_t n;
+    int B;
+    unsigned long long seed;
+};
+
+__device__ __forceinline__ void row_floats(const Draw &d, const double *__restrict__ norm, size_t r, float (&x)[12])
 {
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    if (b >= B) return;
-    const size_t r = (size_t)(mix64(seed ^ mix64((unsigned long long)b)) % n);
+    const size_t n = d.n;
 #pragma unroll
-    for (int k = 0; k < MLP_NIN; k++) X[b * MLP_NIN + k] = (float)((feat[k * n + r] - norm[k]) * norm[8 + k]);
-    const bool ok = valid ? valid[r] != 0 : true;
-    T[2 * b] = ok ? (float)((targ[r] - norm[16]) / norm[18]) : 0.f;
-    T[2 * b + 1] = ok ? (float)((targ[n + r] - norm[17]) / norm[19]) : 0.f;
-    M[b] = ok ? 1 : 0;
+    for (int k = 0; k < MLP_NIN; k++) x[k] = (float)((d.feat[k * n + r] - norm[k]) * norm[8 + k]);
+    const bool ok = d.valid ? d.valid[r] != 0 : true;
+    x[8] = ok ? (float)((d.targ[r] - norm[16]) / norm[18]) : 0.f;
+    x[9] = ok ? (float)((d.targ[n + r] - norm[17]) / norm[19]) : 0.f;
+    x[10] = ok ? 1.f : 0.f;
+    x[11] = 0.f;
+}
+
+__global__ void __launch_bounds__(256) k_records(Draw d, const double *__restrict__ norm, float4 *__restrict__ rec)
+{
+    const size_t r = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (r >= d.n) return;
+    float x[12];
+    row_floats(d, norm, r, x);
+#pragma unroll
+    for (int k = 0; k < 3; k++) rec[3 * r + k] = make_float4(x[4 * k], x[4 * k + 1], x[4 * k + 2], x[4 * k + 3]);
+}
+
+__device__ __forceinline__ void draw_row(const Draw &d, const double *__restrict__ norm, int b, float *__restrict__ X,
+                                         float *__restrict__ T, uint8_t *__restrict__ M)
+{
+    const size_t r = (size_t)(mix64(d.seed ^ mix64((unsigned long long)b)) % d.n);
+    float x[12];
+    if (d.rec) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const float4 v = d.rec[3 * r + k];
+            x[4 * k] = v.x;
+            x[4 * k + 1] = v.y;
+            x[4 * k + 2] = v.z;
+            x[4 * k + 3] = v.w;
+        }
+    } else {
+        row_floats(d, norm, r, x);
+    }
+#pragma unroll
+    for (int k = 0; k < MLP_NIN; k++) X[(size_t)b * MLP_NIN + k] = x[k];
+    T[(size_t)b * MLP_NOUT] = x[8];
+    T[(size_t)b * MLP_NOUT + 1] = x[9];
+    M[b] = x[10] != 0.f ? 1 : 0;
+}
+
+// Parameter of row/lane of k_train's gradients; -1 where there is none.
+__device__ __forceinline__ int tr_param(int row, int lane)
+{
+    const int q = lane >> 4, c = lane & 15;
+    if (row < 128) {
+        const int o = (row >> 4) & 3, i = (row >> 2) & 3, r = row & 3;
+        return (row < 64 ? MLP_W2 : MLP_W3) + (16 * o + 4 * q + r) * MLP_NH + 16 * i + c;
+    }
+    if (row < 144) {
+        const int n = 16 * ((row - 128) >> 2) + 4 * q + (row & 3);
+        return c < MLP_NIN ? MLP_W1 + n * MLP_NIN + c : c == MLP_NIN ? MLP_B1 + n : -1;
+    }
+    if (row < 160) {
+        if (q) return -1;
+        const int t = row & 3;
+        if (row < 152) return MLP_W4 + ((row - 144) >> 2) * MLP_NH + 16 * t + c;
+        return (row < 156 ? MLP_B2 : MLP_B3) + 16 * t + c;
+    }
+    return lane == 0 && row < 162 ? MLP_B4 + row - 160 : -1;
+}
+
+// Blocks [0, nfold): one row of k_train's gradients each, the nb blocks' values added
+// in 64 bits in a fixed order (8 wavefronts a share each, then those), into grad, and
+// an Adam step where asked; row 162 is the loss.  The other blocks draw the rows of
+// the next step's batch, which does not depend on the parameters: its scattered
+// 8-byte loads run beside the fold, and a step is two launches.
+constexpr int AG_THREADS = 512;
+__global__ void __launch_bounds__(AG_THREADS)
+k_adam_gather(const float *__restrict__ part, int nfold, int nb, int B, float *__restrict__ p, float *__restrict__ m,
+              float *__restrict__ v, float *__restrict__ grad, double *__restrict__ loss, int step, float lr, float bc1,
+              float bc2, Draw d, const double *__restrict__ norm, float *__restrict__ X, float *__restrict__ T,
+              uint8_t *__restrict__ M)
+{
+    const int row = blockIdx.x;
+    if (row >= nfold) {
+        const long long b = (long long)(row - nfold) * AG_THREADS + threadIdx.x;
+        if (b < d.B) draw_row(d, norm, (int)b, X, T, M);
+        return;
+    }
+    __shared__ double red[AG_THREADS / 64][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    double s = 0.;
+#pragma unroll 8
+    for (int z = w; z < nb; z += AG_THREADS / 64) s += (double)part[((size_t)z * TR_ROWS + row) * 64 + lane];
+    red[w][lane] = s;
+    __syncthreads();
+    if (w) return;
+#pragma unroll
+    for (int k = 1; k < AG_THREADS / 64; k++) s += red[k][lane];
+    if (row == TR_ROWS - 1) {
+        if (lane == 0) *loss = s / (2. * B);
+        return;
+    }
+    const int i = tr_param(row, lane);
+    if (i < 0) return;
+    const float gi = (float)s;
+    grad[i] = gi;
+    if (!step) return;
+    const float mi = 0.9f * m[i] + 0.1f * gi;
+    const float vi = 0.999f * v[i] + 0.001f * gi * gi;
+    m[i] = mi;
+    v[i] = vi;
+    const float mh = mi / bc1, vh = vi / bc2;
+    p[i] -= lr * mh / (sqrtf(vh) + 1e-8f);
 }
 
 // Partial sums over valid rows for the normalization: pass 0 sums x, pass 1
@@ -398,150 +734,89 @@ int dalloc(T **p, size_t n)
     return 0;
 }
 
-int launch_gemm(harm_mlp *m, const GemmArgs &a, int splits)
-{
-    hipLaunchKernelGGL(k_gemm, dim3(cdiv(a.N, 16), cdiv(a.M, 16), splits), dim3(64), 0, m->stream, a);
-    MCHK(hipGetLastError());
-    return 0;
-}
+// Training sets of at most REC_MAX rows (0.8 GB of records, kept with the network) are
+// drawn from records where a call draws more than one row in REC_ROWS of the set.
+constexpr size_t REC_MAX = (size_t)1 << 24, REC_ROWS = 8;
 
-GemmArgs gemm(int M, int N, int K, const float *A, long sam, long sak, const float *B, long sbk, long sbn, float *C,
-              long scm, long scn)
-{
-    GemmArgs a;
-    std::memset(&a, 0, sizeof(a));
-    a.M = M;
-    a.N = N;
-    a.K = K;
-    a.kchunk = K;
-    a.A = A;
-    a.sam = sam;
-    a.sak = sak;
-    a.B = B;
-    a.sbk = sbk;
-    a.sbn = sbn;
-    a.C = C;
-    a.scm = scm;
-    a.scn = scn;
-    return a;
-}
-
-// Weight gradient dW[Mo][Ni] = dZ^T H over B rows (dZ [B][Mo], H [B][Ni]) and
-// bias gradient db[Mo] = dZ^T 1, split-K then a fixed-order reduction.
-int weight_grad(harm_mlp *m, int B, int Mo, int Ni, const float *dZ, const float *H, float *dW, float *db)
-{
-    const int splits = (int)cdiv(B, KCHUNK);
-    GemmArgs a = gemm(Mo, Ni, B, dZ, 1, Mo, H, Ni, 1, m->part, Ni, 1);
-    a.kchunk = KCHUNK;
-    a.cz = (long)Mo * Ni;
-    int rc;
-    if ((rc = launch_gemm(m, a, splits))) return rc;
-    hipLaunchKernelGGL(k_reduce_splits, dim3(cdiv(Mo * Ni, 256)), dim3(256), 0, m->stream, m->part, splits,
-                       (long)Mo * Ni, Mo * Ni, dW);
-    MCHK(hipGetLastError());
-    GemmArgs b = gemm(Mo, 1, B, dZ, 1, Mo, m->ones, 1, 0, m->part, 1, 1);
-    b.kchunk = KCHUNK;
-    b.cz = Mo;
-    if ((rc = launch_gemm(m, b, splits))) return rc;
-    hipLaunchKernelGGL(k_reduce_splits, dim3(1), dim3(256), 0, m->stream, m->part, splits, (long)Mo, Mo, db);
-    MCHK(hipGetLastError());
-    return 0;
-}
+// Steps whose losses wait on the device for one copy.
+constexpr int LOSS_KEEP = 1024;
 
 int ensure_ws(harm_mlp *m, int B)
 {
     if (B <= m->wsB) return 0;
-    float **bufs[] = {&m->X, &m->T, &m->H1, &m->H2, &m->H3, &m->O, &m->dO, &m->dZa, &m->dZb, &m->ones, &m->part,
-                      &m->lossp};
+    m->wsB = 0;
+    void **bufs[] = {(void **)&m->X, (void **)&m->T, (void **)&m->M};
     for (auto p : bufs) {
         if (*p) (void)hipFree(*p);
         *p = nullptr;
     }
-    if (m->M) (void)hipFree(m->M);
-    m->M = nullptr;
     const size_t b = (size_t)B;
     int rc;
-    if ((rc = dalloc(&m->X, b * MLP_NIN)) || (rc = dalloc(&m->T, b * MLP_NOUT)) || (rc = dalloc(&m->H1, b * MLP_NH)) ||
-        (rc = dalloc(&m->H2, b * MLP_NH)) || (rc = dalloc(&m->H3, b * MLP_NH)) || (rc = dalloc(&m->O, b * MLP_NOUT)) ||
-        (rc = dalloc(&m->dO, b * MLP_NOUT)) || (rc = dalloc(&m->dZa, b * MLP_NH)) ||
-        (rc = dalloc(&m->dZb, b * MLP_NH)) || (rc = dalloc(&m->ones, b)) ||
-        (rc = dalloc(&m->part, (size_t)cdiv(b, KCHUNK) * MLP_NH * MLP_NH)) || (rc = dalloc(&m->lossp, cdiv(b, 256))) ||
-        (rc = dalloc(&m->M, b)))
-        return rc;
-    hipLaunchKernelGGL(k_fill, dim3(cdiv(b, 256)), dim3(256), 0, m->stream, m->ones, 1.f, B);
-    MCHK(hipGetLastError());
+    if ((rc = dalloc(&m->X, b * MLP_NIN)) || (rc = dalloc(&m->T, b * MLP_NOUT)) || (rc = dalloc(&m->M, b))) return rc;
     m->wsB = B;
     return 0;
 }
 
-// Forward of the FP32 training path on X [B][8] into H1..H3, O.
-int forward_f32(harm_mlp *m, const float *X, int B)
+// Room for a training set of n rows as records; false where there is none.
+bool ensure_records(harm_mlp *m, size_t n)
 {
-    const float *P = m->params;
-    int rc;
-    GemmArgs a = gemm(B, MLP_NH, MLP_NIN, X, MLP_NIN, 1, P + MLP_W1, 1, MLP_NIN, m->H1, MLP_NH, 1);
-    a.epi = 2;
-    a.bias = P + MLP_B1;
-    if ((rc = launch_gemm(m, a, 1))) return rc;
-    a = gemm(B, MLP_NH, MLP_NH, m->H1, MLP_NH, 1, P + MLP_W2, 1, MLP_NH, m->H2, MLP_NH, 1);
-    a.epi = 2;
-    a.bias = P + MLP_B2;
-    if ((rc = launch_gemm(m, a, 1))) return rc;
-    a = gemm(B, MLP_NH, MLP_NH, m->H2, MLP_NH, 1, P + MLP_W3, 1, MLP_NH, m->H3, MLP_NH, 1);
-    a.epi = 2;
-    a.bias = P + MLP_B3;
-    if ((rc = launch_gemm(m, a, 1))) return rc;
-    a = gemm(B, MLP_NOUT, MLP_NH, m->H3, MLP_NH, 1, P + MLP_W4, 1, MLP_NH, m->O, MLP_NOUT, 1);
-    a.epi = 1;
-    a.bias = P + MLP_B4;
-    return launch_gemm(m, a, 1);
+    if (n <= m->recN) return true;
+    if (m->rec) (void)hipFree(m->rec);
+    m->rec = nullptr;
+    m->recN = 0;
+    if (hipMalloc((void **)&m->rec, n * 3 * sizeof(float4)) != hipSuccess) {
+        (void)hipGetLastError();
+        m->rec = nullptr;
+        return false;
+    }
+    m->recN = n;
+    return true;
 }
 
-// Forward, loss and gradient into m->grad for B standardized rows.
-int loss_grad(harm_mlp *m, const float *X, const float *T, const uint8_t *M, int B)
+// A batch's 16-row tiles go to the blocks in turn, so a small one takes a wavefront
+// on each of as many CUs as it has tiles.
+int train_blocks(int B) { return (int)std::min<unsigned>(TR_BLOCKS, cdiv(B, 16)); }
+
+int launch_forward(harm_mlp *m, const float *X, float *Y, int B)
 {
-    int rc;
-    if ((rc = forward_f32(m, X, B))) return rc;
-    hipLaunchKernelGGL(k_loss, dim3(cdiv(B, 256)), dim3(256), 0, m->stream, m->O, T, M, B, m->loss_w[0],
-                       m->loss_w[1], m->dO, m->lossp);
+    hipLaunchKernelGGL(k_train<false>, dim3(train_blocks(B)), dim3(TR_WAVES * 64), 0, m->stream, m->params, X,
+                       (const float *)nullptr, (const uint8_t *)nullptr, B, 0.f, 0.f, (float *)nullptr, Y);
     MCHK(hipGetLastError());
-    const float *P = m->params;
-    float *G = m->grad;
-    // layer 4
-    if ((rc = weight_grad(m, B, MLP_NOUT, MLP_NH, m->dO, m->H3, G + MLP_W4, G + MLP_B4))) return rc;
-    GemmArgs a = gemm(B, MLP_NH, MLP_NOUT, m->dO, MLP_NOUT, 1, P + MLP_W4, MLP_NH, 1, m->dZa, MLP_NH, 1);
-    a.epi = 3;
-    a.H = m->H3;
-    a.shm = MLP_NH;
-    a.shn = 1;
-    if ((rc = launch_gemm(m, a, 1))) return rc;
-    // layer 3
-    if ((rc = weight_grad(m, B, MLP_NH, MLP_NH, m->dZa, m->H2, G + MLP_W3, G + MLP_B3))) return rc;
-    a = gemm(B, MLP_NH, MLP_NH, m->dZa, MLP_NH, 1, P + MLP_W3, MLP_NH, 1, m->dZb, MLP_NH, 1);
-    a.epi = 3;
-    a.H = m->H2;
-    a.shm = MLP_NH;
-    a.shn = 1;
-    if ((rc = launch_gemm(m, a, 1))) return rc;
-    // layer 2
-    if ((rc = weight_grad(m, B, MLP_NH, MLP_NH, m->dZb, m->H1, G + MLP_W2, G + MLP_B2))) return rc;
-    a = gemm(B, MLP_NH, MLP_NH, m->dZb, MLP_NH, 1, P + MLP_W2, MLP_NH, 1, m->dZa, MLP_NH, 1);
-    a.epi = 3;
-    a.H = m->H1;
-    a.shm = MLP_NH;
-    a.shn = 1;
-    if ((rc = launch_gemm(m, a, 1))) return rc;
-    // layer 1
-    return weight_grad(m, B, MLP_NH, MLP_NIN, m->dZa, X, G + MLP_W1, G + MLP_B1);
+    return 0;
 }
 
-int adam_step(harm_mlp *m, float lr)
+// Forward, loss and gradient of B standardized rows into m->part.
+int launch_train(harm_mlp *m, const float *X, const float *T, const uint8_t *M, int B)
 {
-    m->adam_t++;
-    const float bc1 = (float)(1. - std::pow(0.9, (double)m->adam_t));
-    const float bc2 = (float)(1. - std::pow(0.999, (double)m->adam_t));
-    hipLaunchKernelGGL(k_adam, dim3(cdiv(MLP_NPARAMS, 256)), dim3(256), 0, m->stream, m->params, m->adam_m, m->adam_v,
-                       m->grad, MLP_NPARAMS, lr, bc1, bc2);
+    hipLaunchKernelGGL(k_train<true>, dim3(train_blocks(B)), dim3(TR_WAVES * 64), 0, m->stream, m->params, X, T, M, B,
+                       m->loss_w[0], m->loss_w[1], m->part, (float *)nullptr);
+    MCHK(hipGetLastError());
+    return 0;
+}
+
+int launch_draw(harm_mlp *m, const Draw &d)
+{
+    hipLaunchKernelGGL(k_adam_gather, dim3(cdiv(d.B, AG_THREADS)), dim3(AG_THREADS), 0, m->stream, m->part, 0, 0, 0,
+                       m->params, m->adam_m, m->adam_v, m->grad, m->lossd, 0, 0.f, 1.f, 1.f, d, m->norm, m->X, m->T, m->M);
+    MCHK(hipGetLastError());
+    return 0;
+}
+
+// The gradient of launch_train's batch into m->grad and its loss into *loss (m->lossd
+// if null); an Adam step where loss is given; the rows of *next drawn where that is.
+int launch_adam(harm_mlp *m, int B, double *loss, float lr, const Draw *next)
+{
+    float bc1 = 1.f, bc2 = 1.f;
+    const bool step = loss != nullptr;
+    if (step) {
+        m->adam_t++;
+        bc1 = (float)(1. - std::pow(0.9, (double)m->adam_t));
+        bc2 = (float)(1. - std::pow(0.999, (double)m->adam_t));
+    }
+    const Draw d = next ? *next : Draw{};
+    hipLaunchKernelGGL(k_adam_gather, dim3(TR_ROWS + cdiv(d.B, AG_THREADS)), dim3(AG_THREADS), 0, m->stream, m->part,
+                       TR_ROWS, train_blocks(B), B, m->params, m->adam_m, m->adam_v, m->grad,
+                       step ? loss : m->lossd, (int)step, lr, bc1, bc2, d, m->norm, m->X, m->T, m->M);
     MCHK(hipGetLastError());
     return 0;
 }
@@ -552,21 +827,6 @@ int repack(harm_mlp *m)
                        m->bias);
     MCHK(hipGetLastError());
     return 0;
-}
-
-double sum_loss(harm_mlp *m, int B, int &rc)
-{
-    std::vector<float> lp(cdiv(B, 256));
-    rc = 0;
-    if (hipMemcpyAsync(lp.data(), m->lossp, lp.size() * sizeof(float), hipMemcpyDeviceToHost, m->stream) !=
-            hipSuccess ||
-        hipStreamSynchronize(m->stream) != hipSuccess) {
-        rc = harm_host::set_error("loss copy failed", 2);
-        return 0.;
-    }
-    double s = 0.;
-    for (float v : lp) s += v;
-    return s / (2. * B);
 }
 
 struct DevGuard {
@@ -623,7 +883,8 @@ harm_mlp *harm_mlp_create(int device)
     bool ok = hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) == hipSuccess;
     ok = ok && !dalloc(&m->params, MLP_NPARAMS) && !dalloc(&m->adam_m, MLP_NPARAMS) &&
          !dalloc(&m->adam_v, MLP_NPARAMS) && !dalloc(&m->grad, MLP_NPARAMS) && !dalloc(&m->wpack, MLP_CHUNKS * 64) &&
-         !dalloc(&m->bias, MLP_BIAS_LEN) && !dalloc(&m->norm, MLP_NORM_LEN) && !dalloc(&m->normp, NORM_BLOCKS * 11 + 16);
+         !dalloc(&m->bias, MLP_BIAS_LEN) && !dalloc(&m->norm, MLP_NORM_LEN) && !dalloc(&m->normp, NORM_BLOCKS * 11 + 16) &&
+         !dalloc(&m->part, (size_t)TR_BLOCKS * TR_ROWS * 64) && !dalloc(&m->lossd, LOSS_KEEP);
     if (!ok) {
         harm_mlp_destroy(m);
         return nullptr;
@@ -644,8 +905,7 @@ void harm_mlp_destroy(harm_mlp *m)
     DevGuard dg(m->device);
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     void *bufs[] = {m->params, m->adam_m, m->adam_v, m->grad, m->wpack, m->bias, m->norm, m->normp,
-                    m->X,      m->T,      m->H1,     m->H2,   m->H3,    m->O,    m->dO,   m->dZa,
-                    m->dZb,    m->ones,   m->part,   m->lossp, m->M};
+                    m->X,      m->T,      m->M,      m->part, m->lossd, m->rec};
     for (void *p : bufs)
         if (p) (void)hipFree(p);
     if (m->stream) (void)hipStreamDestroy(m->stream);
@@ -757,15 +1017,12 @@ int harm_mlp_grad(harm_mlp *m, const float *X, const float *T, const uint8_t *ma
     int rc;
     if ((rc = check_batch(n))) return rc;
     DevGuard dg(m->device);
-    if ((rc = ensure_ws(m, n))) return rc;
-    if ((rc = loss_grad(m, X, T, mask, n))) return rc;
-    const double l = sum_loss(m, n, rc);
-    if (rc) return rc;
+    if ((rc = launch_train(m, X, T, mask, n)) || (rc = launch_adam(m, n, nullptr, 0.f, nullptr))) return rc;
+    double l = 0.;
+    MCHK(hipMemcpyAsync(&l, m->lossd, sizeof(l), hipMemcpyDeviceToHost, m->stream));
+    if (grad) MCHK(hipMemcpyAsync(grad, m->grad, MLP_NPARAMS * sizeof(float), hipMemcpyDeviceToHost, m->stream));
+    MCHK(hipStreamSynchronize(m->stream));
     if (loss) *loss = l;
-    if (grad) {
-        MCHK(hipMemcpyAsync(grad, m->grad, MLP_NPARAMS * sizeof(float), hipMemcpyDeviceToHost, m->stream));
-        MCHK(hipStreamSynchronize(m->stream));
-    }
     return 0;
 }
 
@@ -775,7 +1032,7 @@ int harm_mlp_train_batch(harm_mlp *m, const float *X, const float *T, const uint
     int rc;
     if ((rc = check_batch(n))) return rc;
     DevGuard dg(m->device);
-    if ((rc = ensure_ws(m, n)) || (rc = loss_grad(m, X, T, mask, n)) || (rc = adam_step(m, lr)) || (rc = repack(m)))
+    if ((rc = launch_train(m, X, T, mask, n)) || (rc = launch_adam(m, n, m->lossd, lr, nullptr)) || (rc = repack(m)))
         return rc;
     MCHK(hipStreamSynchronize(m->stream));
     return 0;
@@ -791,18 +1048,28 @@ int harm_mlp_train(harm_mlp *m, const double *feat, const double *targ, const ui
     if (steps < 0 || !(lr0 > 0.f) || !(lr1 > 0.f)) return harm_host::set_error("bad training schedule", 4);
     DevGuard dg(m->device);
     if ((rc = ensure_ws(m, batch))) return rc;
-    std::vector<float> lp;
+    Draw d = {feat, targ, valid, nullptr, n, batch, 0};
+    if (n <= REC_MAX && (size_t)steps * batch >= n / REC_ROWS && ensure_records(m, n)) {
+        hipLaunchKernelGGL(k_records, dim3(cdiv(n, 256)), dim3(256), 0, m->stream, d, m->norm, m->rec);
+        MCHK(hipGetLastError());
+        d.rec = m->rec;
+    }
+    auto draw_seed = [&](int s) { return (unsigned long long)seed * 0x100000001B3ull + (unsigned long long)s; };
+    std::vector<double> lp(LOSS_KEEP);
+    d.seed = draw_seed(0);
+    if (steps > 0 && (rc = launch_draw(m, d))) return rc;
     for (int s = 0; s < steps; s++) {
         const double fr = steps > 1 ? (double)s / (steps - 1) : 0.;
         const float lr = (float)(lr0 * std::pow((double)lr1 / lr0, fr));
-        const unsigned long long sd = (unsigned long long)seed * 0x100000001B3ull + (unsigned long long)s;
-        hipLaunchKernelGGL(k_gather, dim3(cdiv(batch, 256)), dim3(256), 0, m->stream, feat, targ, valid, n, m->norm,
-                           sd, batch, m->X, m->T, m->M);
-        MCHK(hipGetLastError());
-        if ((rc = loss_grad(m, m->X, m->T, m->M, batch)) || (rc = adam_step(m, lr))) return rc;
-        if (loss_trace) {
-            loss_trace[s] = (float)sum_loss(m, batch, rc);
-            if (rc) return rc;
+        d.seed = draw_seed(s + 1);
+        const int k = s % LOSS_KEEP;
+        if ((rc = launch_train(m, m->X, m->T, m->M, batch)) ||
+            (rc = launch_adam(m, batch, m->lossd + k, lr, s + 1 < steps ? &d : nullptr)))
+            return rc;
+        if (loss_trace && (k == LOSS_KEEP - 1 || s == steps - 1)) {
+            MCHK(hipMemcpyAsync(lp.data(), m->lossd, (k + 1) * sizeof(double), hipMemcpyDeviceToHost, m->stream));
+            MCHK(hipStreamSynchronize(m->stream));
+            for (int i = 0; i <= k; i++) loss_trace[s - k + i] = (float)lp[i];
         }
     }
     if ((rc = repack(m))) return rc;
@@ -820,8 +1087,7 @@ int harm_mlp_forward(harm_mlp *m, const float *X, float *Y, int n, int bf16)
         hipLaunchKernelGGL(k_forward_bf16, dim3(cdiv(n, 256)), dim3(256), 0, m->stream, harm_mlp_view(m), X, Y, n);
         MCHK(hipGetLastError());
     } else {
-        if ((rc = ensure_ws(m, n)) || (rc = forward_f32(m, X, n))) return rc;
-        MCHK(hipMemcpyAsync(Y, m->O, (size_t)n * MLP_NOUT * sizeof(float), hipMemcpyDeviceToDevice, m->stream));
+        if ((rc = launch_forward(m, X, Y, n))) return rc;
     }
     MCHK(hipStreamSynchronize(m->stream));
     return 0;
