@@ -25,6 +25,7 @@ struct harm_cache {
     int whole;
     double *vx = nullptr, *vy = nullptr, *vz = nullptr, *values = nullptr;
     uint8_t *counted = nullptr;
+    double *tab = nullptr;  // the splines along y of every component (harm_cache.hpp), or null
     int device = 0;
 };
 
@@ -51,15 +52,19 @@ int check_desc(const harm_cache_desc &d)
 
 bool is_v1(const harm_cache_desc &d) { return std::strncmp(d.ver, "AGACACHE_1.0", 13) == 0; }
 
+// A lookup in z plane zindex >= 0 takes the splines along y from the table; these two
+// kernels are the rest: no table, the linear rule, interpolation in z.  plane_too: also
+// the points that have a z plane.
 __global__ void __launch_bounds__(TPB_C) k_cache_lookup(harm::CacheView c, int mode, uint64_t mask,
                                                         const double *__restrict__ x, const double *__restrict__ y,
                                                         const double *__restrict__ z, const int *__restrict__ zindex,
                                                         double *__restrict__ out, double *__restrict__ dery,
-                                                        int *__restrict__ status, size_t n)
+                                                        int *__restrict__ status, size_t n, bool plane_too)
 {
     const size_t i = (size_t)blockIdx.x * TPB_C + threadIdx.x;
     if (i >= n) return;
     const int zi = zindex ? zindex[i] : -1;
+    if (zi != -1 && !plane_too) return;
     const double zv = z ? z[i] : 0.0;
     const int s = harm::cache_lookup(c, x[i], y[i], zv, zi, mode, mask, out + i, dery ? dery + i : nullptr, n);
     if (status) status[i] = s;
@@ -69,15 +74,152 @@ __global__ void __launch_bounds__(TPB_C) k_cache_solve_T(harm::CacheView c, cons
                                                          const double *__restrict__ e,
                                                          const int *__restrict__ zindex, double *__restrict__ T,
                                                          double lo, double hi, int ntrial, double tolf,
-                                                         double *__restrict__ berr, int *__restrict__ ret, size_t n)
+                                                         double *__restrict__ berr, int *__restrict__ ret, size_t n,
+                                                         bool plane_too)
 {
     const size_t i = (size_t)blockIdx.x * TPB_C + threadIdx.x;
     if (i >= n) return;
+    const int zi = zindex ? zindex[i] : 0;
+    if (zi != -1 && !plane_too) return;
     double t, b;
-    const int r = harm::cache_solve_T(c, rho[i], e[i], zindex ? zindex[i] : 0, T[i], lo, hi, ntrial, tolf, t, b);
+    const int r = harm::cache_newton_T(e[i], T[i], lo, hi, ntrial, tolf, t, b, [&](double xt, double &v, double &dv) {
+        return harm::cache_lookup1<true>(c, rho[i], xt, zi, 0, v, dv) == harm::CACHE_OK;
+    });
     T[i] = t;
     if (berr) berr[i] = b;
     if (ret) ret[i] = r;
+}
+
+// One (x row, bracket) of component and plane blockIdx.y per thread.
+__global__ void __launch_bounds__(TPB_C) k_cache_table(harm::CacheView c, double *__restrict__ tab)
+{
+    const size_t r = (size_t)blockIdx.x * TPB_C + threadIdx.x;
+    const int left = (int)(r / c.X), ix = (int)(r % c.X);
+    if (left < 1 || left >= c.Y) return;
+    const int zp = (int)blockIdx.y / c.D, k = (int)blockIdx.y % c.D;
+    harm::cache_tab_fill(c, zp, k, ix, left, tab + harm::cache_tab_plane(c.X, c.Y) * blockIdx.y);
+}
+
+// The axes in LDS (AX: they fit), where a bisection's steps cost a tenth of a global
+// read each.
+template <bool AX>
+__device__ __forceinline__ void stage_axes(const harm::CacheView &c, double *ax, const double *&vx, const double *&vy)
+{
+    vx = c.vx;
+    vy = c.vy;
+    if (!AX) return;
+    for (int k = threadIdx.x; k < c.X; k += TPB_C) ax[k] = c.vx[k];
+    for (int k = threadIdx.x; k < c.Y; k += TPB_C) ax[c.X + k] = c.vy[k];
+    __syncthreads();
+    vx = ax;
+    vy = ax + c.X;
+}
+
+// One query per thread, its windows found once and then the components one after
+// another.  Bound by the FP64 VALU: 22 divisions and about 300 other operations a
+// component with the derivative (2^21 points of a 200x200 table, six values and their
+// derivatives: 418 us a call; with every spline fitted per query, 4300 us).
+template <bool DER, bool AX>
+__global__ void __launch_bounds__(TPB_C) k_lookup_tab(harm::CacheView c, const double *__restrict__ tab, uint64_t mask,
+                                                      const double *__restrict__ x, const double *__restrict__ y,
+                                                      const double *__restrict__ z, const int *__restrict__ zindex,
+                                                      double *__restrict__ out, double *__restrict__ dery,
+                                                      int *__restrict__ status, size_t n)
+{
+    extern __shared__ double ax[];
+    const double *vx, *vy;
+    stage_axes<AX>(c, ax, vx, vy);
+    const size_t i = (size_t)blockIdx.x * TPB_C + threadIdx.x;
+    if (i >= n) return;
+    const int zi = zindex[i];
+    if (zi == -1 && c.Z >= 3) return;  // k_cache_lookup's
+    const double xv = x[i], yv = y[i];
+    const int lx = harm::cache_bracket(c.X, vx, xv), ly = harm::cache_bracket(c.Y, vy, yv);
+    const int s = harm::cache_lookup_status(c, vx, vy, xv, yv, z ? z[i] : 0.0, zi, lx, ly);
+    if (status) status[i] = s;
+    if (s != harm::CACHE_OK) return;
+    const harm::CacheXWin w = harm::cache_xwin(c.X, vx, lx, xv);
+    const harm::CacheYWin u = harm::cache_ywin<DER>(c.Y, vy, ly, yv);
+    const size_t plane = harm::cache_tab_plane(c.X, c.Y);
+    const double *t = tab + plane * c.D * zi;
+    for (int k = 0; k < c.D; k++, t += plane) {
+        if (!((mask >> k) & 1)) continue;
+        double v, dv;
+        harm::cache_spline_tab<DER>(c.X, c.Y, t, w, u, v, dv);
+        out[k * n + i] = v;
+        if (DER) dery[k * n + i] = dv;
+    }
+}
+
+// One solve per thread, about four trials each (2^21 solves from starts 5% off: 290 us a
+// call; with every spline fitted per trial, 1350 us).
+template <bool AX>
+__global__ void __launch_bounds__(TPB_C) k_solve_tab(harm::CacheView c, const double *__restrict__ tab,
+                                                     const double *__restrict__ rho, const double *__restrict__ e,
+                                                     const int *__restrict__ zindex, double *__restrict__ T, double lo,
+                                                     double hi, int ntrial, double tolf, double *__restrict__ berr,
+                                                     int *__restrict__ ret, size_t n)
+{
+    extern __shared__ double ax[];
+    const double *vx, *vy;
+    stage_axes<AX>(c, ax, vx, vy);
+    const size_t i = (size_t)blockIdx.x * TPB_C + threadIdx.x;
+    if (i >= n) return;
+    const int zi = zindex ? zindex[i] : 0;
+    if (zi == -1 && c.Z >= 3) return;  // k_cache_solve_T's
+    const double rv = rho[i];
+    const int lx = harm::cache_bracket(c.X, vx, rv);
+    const harm::CacheXWin w = harm::cache_xwin(c.X, vx, lx, rv);
+    const double *t = tab + harm::cache_tab_plane(c.X, c.Y) * c.D * (zi < 0 || zi >= c.Z ? 0 : zi);
+    int ly = 0;
+    double tn, b;
+    const int r = harm::cache_newton_T(e[i], T[i], lo, hi, ntrial, tolf, tn, b, [&](double xt, double &v, double &dv) {
+        // the bracket of the trial before, where it still holds this one
+        if (ly == 0 || (ly > 1 && xt < vy[ly - 1]) || (ly < c.Y - 1 && !(xt < vy[ly])))
+            ly = harm::cache_bracket(c.Y, vy, xt);
+        if (harm::cache_lookup_status(c, vx, vy, rv, xt, 0.0, zi, lx, ly) != harm::CACHE_OK) return false;
+        harm::cache_spline_tab<true>(c.X, c.Y, t, w, harm::cache_ywin<true>(c.Y, vy, ly, xt), v, dv);
+        return true;
+    });
+    T[i] = tn;
+    if (berr) berr[i] = b;
+    if (ret) ret[i] = r;
+}
+
+harm::CacheView view_of(const harm_cache *c)
+{
+    return harm::CacheView{c->desc.x, c->desc.y, c->desc.z, c->desc.d, c->desc.xtype, c->desc.ytype, c->desc.ztype,
+                           c->whole,  c->vx,     c->vy,     c->vz,     c->values,     c->counted};
+}
+
+// Bytes of LDS that both axes take, 0 where they would hold back the occupancy: at
+// 16 KiB a block all 8 blocks of 256 threads still fit a CU.
+size_t axes_lds(const harm_cache_desc &d)
+{
+    const size_t b = ((size_t)d.x + d.y) * sizeof(double);
+    return b <= 16 * 1024 ? b : 0;
+}
+
+// Tables of at most 1 GiB (12 times the values' size); larger caches, and those whose
+// table finds no memory, are looked up from their values.
+constexpr size_t TAB_MAX = (size_t)1 << 30;
+
+int build_table(harm_cache *c)
+{
+    const harm_cache_desc &d = c->desc;
+    const size_t planes = (size_t)d.z * d.d, bytes = planes * harm::cache_tab_plane(d.x, d.y) * sizeof(double);
+    if (bytes > TAB_MAX || planes > 65535) return 0;
+    if (hipMalloc(&c->tab, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        c->tab = nullptr;
+        return 0;
+    }
+    const size_t per = (size_t)d.x * d.y;
+    hipLaunchKernelGGL(k_cache_table, dim3((unsigned)((per + TPB_C - 1) / TPB_C), (unsigned)planes), dim3(TPB_C), 0, 0,
+                       view_of(c), c->tab);
+    CCHK(hipGetLastError());
+    CCHK(hipStreamSynchronize(0));
+    return 0;
 }
 
 }  // namespace
@@ -192,6 +334,7 @@ void harm_cache_free(harm_cache *c)
         (void)hipFree(c->vz);
         (void)hipFree(c->values);
         (void)hipFree(c->counted);
+        (void)hipFree(c->tab);
         (void)hipSetDevice(prev);
     }
     delete c;
@@ -249,7 +392,7 @@ harm_cache *harm_cache_create(const harm_cache_desc *desc, const double *vx, con
     for (size_t i = 0; i < np; i++) ones += counted[i] == 1;
     // a file that says it is whole is taken at its word, as the reference does
     c->whole = d.wholecachecalculated || ones == np;
-    if (cache_upload(c, vx, vy, vz, values, counted)) {
+    if (cache_upload(c, vx, vy, vz, values, counted) || build_table(c)) {
         harm_cache_free(c);
         return nullptr;
     }
@@ -273,8 +416,7 @@ harm_cache *harm_cache_open(const char *path)
 int harm_cache_view_of(const harm_cache *c, harm::CacheView &v, harm_cache_desc &d, int &device)
 {
     if (!c) return harm_host::set_error("null cache", 1);
-    v = harm::CacheView{c->desc.x,     c->desc.y,  c->desc.z,  c->desc.d,  c->desc.xtype, c->desc.ytype, c->desc.ztype,
-                        c->whole,      c->vx,      c->vy,      c->vz,      c->values,     c->counted};
+    v = view_of(c);
     d = c->desc;
     device = c->device;
     return 0;
@@ -302,11 +444,21 @@ int harm_cache_lookup(const harm_cache *c, int mode, const int *dimmask, const d
     uint64_t mask = 0;
     for (int k = 0; k < c->desc.d; k++)
         if (!dimmask || dimmask[k]) mask |= 1ull << k;
-    harm::CacheView v{c->desc.x, c->desc.y, c->desc.z, c->desc.d, c->desc.xtype, c->desc.ytype, c->desc.ztype,
-                      c->whole, c->vx, c->vy, c->vz, c->values, c->counted};
+    const harm::CacheView v = view_of(c);
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_cache_lookup, dim3((unsigned)((n + TPB_C - 1) / TPB_C)), dim3(TPB_C), 0, s, v, mode, mask, x,
-                       y, z, zindex, out, dery, status, n);
+    const dim3 grid((unsigned)((n + TPB_C - 1) / TPB_C)), block(TPB_C);
+    const bool tab = c->tab && mode == HARM_INTERP_SPLINE && zindex;
+    if (tab) {
+        const size_t lds = axes_lds(c->desc);
+        auto *k = dery ? (lds ? k_lookup_tab<true, true> : k_lookup_tab<true, false>)
+                       : (lds ? k_lookup_tab<false, true> : k_lookup_tab<false, false>);
+        hipLaunchKernelGGL(k, grid, block, lds, s, v, c->tab, mask, x, y, z, zindex, out, dery, status, n);
+        CCHK(hipGetLastError());
+    }
+    if (!tab || c->desc.z >= 3) {
+        hipLaunchKernelGGL(k_cache_lookup, grid, block, 0, s, v, mode, mask, x, y, z, zindex, out, dery, status, n,
+                           !tab);
+    }
     CCHK(hipGetLastError());
     CCHK(hipStreamSynchronize(s));
     return 0;
@@ -329,11 +481,19 @@ int harm_cache_solve_T(const harm_cache *c, const double *rho, const double *e, 
         Thi = ends[1] * (1. - 1.e-6);
     }
     if (!(Tlo < Thi)) return harm_host::set_error("harm_cache_solve_T: needs Tlo < Thi", 3);
-    harm::CacheView v{c->desc.x, c->desc.y, c->desc.z, c->desc.d, c->desc.xtype, c->desc.ytype, c->desc.ztype,
-                      c->whole, c->vx, c->vy, c->vz, c->values, c->counted};
+    const harm::CacheView v = view_of(c);
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_cache_solve_T, dim3((unsigned)((n + TPB_C - 1) / TPB_C)), dim3(TPB_C), 0, s, v, rho, e,
-                       zindex, T, Tlo, Thi, ntrial, tolf, berr, ret, n);
+    const dim3 grid((unsigned)((n + TPB_C - 1) / TPB_C)), block(TPB_C);
+    if (c->tab) {
+        const size_t lds = axes_lds(c->desc);
+        hipLaunchKernelGGL(lds ? k_solve_tab<true> : k_solve_tab<false>, grid, block, lds, s, v, c->tab, rho, e, zindex,
+                           T, Tlo, Thi, ntrial, tolf, berr, ret, n);
+        CCHK(hipGetLastError());
+    }
+    if (!c->tab || (zindex && c->desc.z >= 3)) {
+        hipLaunchKernelGGL(k_cache_solve_T, grid, block, 0, s, v, rho, e, zindex, T, Tlo, Thi, ntrial, tolf, berr, ret,
+                           n, !c->tab);
+    }
     CCHK(hipGetLastError());
     CCHK(hipStreamSynchronize(s));
     return 0;

@@ -519,16 +519,217 @@ HC_HD void cache_spline_win_co(const CacheView &c, const double *yco, int x0, in
     if (DER) ok &= cache_akima_m<NX, 1>(xs, xd, &x, &dv);
 }
 
+// ---------------------------------------------------------------------------
+// Lookups with the splines along y read from a table.
+//
+// The spline along y of a window depends on the cache alone, so its four numbers
+// (cache_akima_coefs: y_i, g_i, p1_i, p2_i) are formed once per cache for every
+// component, x row and y bracket (left = 1..Y-1, left 0 unused) and each of the
+// window's intervals: per z plane and component [3 intervals][Y][X][4] doubles.  x is
+// fastest, so the four rows of a lookup's window are 128 consecutive bytes, and nearly
+// every lookup reads the plane of interval 1 alone.  What is left per component is the
+// spline along x (twice with the y derivative), of which one lookup needs one
+// interval: 9 divisions instead of the 14 of all of them.  Same operations in the same
+// order as cache_akima for every number that reaches the result, so the same bits.
+// ---------------------------------------------------------------------------
+HC_HD size_t cache_tab_plane(int X, int Y) { return (size_t)3 * X * Y * 4; }
+
+// Two doubles at p (16-byte aligned); on the device through the global address
+// space, also where the pointer came out of a structure.
+struct CacheD2 {
+    double a, b;
+};
+HC_HD CacheD2 cache_ld2(const double *p)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    const d2 v = *(const __attribute__((address_space(1))) d2 *)p;
+    return CacheD2{v.x, v.y};
+#else
+    return CacheD2{p[0], p[1]};
+#endif
+}
+
+// Table entries of x row ix and bracket left of component k of z plane zp; tab: that
+// plane's and component's part of the table.
+HC_HD void cache_tab_fill(const CacheView &c, int zp, int k, int ix, int left, double *tab)
+{
+    const int lo = left - 2 < 0 ? 0 : left - 2;
+    const int hi = left + 1 >= c.Y ? c.Y - 1 : left + 1;
+    const int m = hi - lo + 1;
+    const double *row = c.values + ((size_t)zp * c.X * c.Y + (size_t)ix * c.Y + lo) * c.D + k;
+    double yv[4], co[12];
+    for (int q = 0; q < m; q++) yv[q] = row[(size_t)q * c.D];
+    if (m == 4)
+        cache_akima_coefs<4>(c.vy + lo, yv, co);
+    else
+        cache_akima_coefs<3>(c.vy + lo, yv, co);
+    for (int i = 0; i < m - 1; i++)
+        for (int q = 0; q < 4; q++) tab[(((size_t)i * c.Y + left) * c.X + ix) * 4 + q] = co[4 * i + q];
+}
+
+// The spline along x at one query: its window's rows x0, x0+1, x0+2 and, with w4, x0+3,
+// the interval i1 (0 or 1: a query in its own bracket never lies in the third) and the
+// denominators.  In cache_akima's numbering S[0..M+2] the interval needs S[i..i+4]:
+//   i = 0: L0 L1 R0 R1 F      i = 1: L1 R0 R1 F G
+// R0, R1 the first two secants, L1, L0 those extrapolated on the left; F is the third
+// secant of four rows or the first extrapolated one on the right of three, G the one
+// after it.  One of L0, G is ever needed, so both take the same division.
+struct CacheXWin {
+    int x0;
+    bool w4, i1;
+    double dx0, dx1, eL0, eL1, e2, denF, denG, d0, d00, t1;
+};
+
+HC_HD CacheXWin cache_xwin(int n, const double *v, int left, double x)
+{
+    CacheXWin w;
+    w.x0 = left - 2 < 0 ? 0 : left - 2;
+    const int hi = left + 1 >= n ? n - 1 : left + 1;
+    w.w4 = hi - w.x0 == 3;
+    const double a = v[w.x0], b = v[w.x0 + 1], c = v[w.x0 + 2], d = v[w.w4 ? w.x0 + 3 : w.x0 + 2];
+    w.i1 = x > b;
+    w.dx0 = b - a;
+    w.dx1 = c - b;
+    const double xl1 = a + b - c, xl0 = xl1 + a - b;
+    w.eL1 = a - xl1;
+    w.eL0 = xl1 - xl0;
+    const double xm = w.w4 ? b : a, xa = w.w4 ? c : b, xb = w.w4 ? d : c;
+    const double xr2 = xb + xa - xm, xr3 = xr2 + xb - xa;
+    w.e2 = xr2 - xb;
+    w.denF = w.w4 ? d - c : w.e2;
+    w.denG = w.i1 ? (w.w4 ? w.e2 : xr3 - xr2) : w.eL0;
+    w.d0 = w.i1 ? w.dx1 : w.dx0;
+    w.d00 = w.d0 * w.d0;
+    w.t1 = x - (w.i1 ? b : a);
+    return w;
+}
+
+HC_HD double cache_node_slope(double a, double b, double c, double d)
+{
+    const double d0 = fabs(d - c), d1 = fabs(b - a);
+    return (d0 + d1) < 1e-9 ? 0.5 * (b + c) : (d0 * b + d1 * c) / (d0 + d1);
+}
+
+// Value at the query of the spline along x through the rows' values (y3 is read with
+// w4 alone).
+HC_HD double cache_xspline(const CacheXWin &w, double y0, double y1, double y2, double y3)
+{
+    const double R0 = (y1 - y0) / w.dx0, R1 = (y2 - y1) / w.dx1;
+    const double yl1 = w.eL1 * (R1 - 2.0 * R0) + y0;
+    const double L1 = (y0 - yl1) / w.eL1;
+    const double yr = (2.0 * R1 - R0) * w.e2 + y2;
+    const double F = ((w.w4 ? y3 : yr) - y2) / w.denF;
+    const double base = w.i1 ? (w.w4 ? y3 : yr) : yl1;
+    const double yn = (w.i1 ? 2.0 * F - R1 : R0 - 2.0 * L1) * w.denG + base;
+    const double G = (w.i1 ? yn - base : base - yn) / w.denG;
+    const double s0 = w.i1 ? L1 : G, s1 = w.i1 ? R0 : L1, s2 = w.i1 ? R1 : R0, s3 = w.i1 ? F : R1, s4 = w.i1 ? G : F;
+    const double g0 = cache_node_slope(s0, s1, s2, s3), g1 = cache_node_slope(s1, s2, s3, s4);
+    const double p1 = (3.0 * s2 - 2.0 * g0 - g1) / w.d0;
+    const double p2 = (g0 + g1 - 2.0 * s2) / w.d00;
+    return (w.i1 ? y1 : y0) + g0 * w.t1 + p1 * w.t1 * w.t1 + p2 * w.t1 * w.t1 * w.t1;
+}
+
+// The splines along y at one query: the window's first row lo of the axis, four its
+// size, the intervals (cache_akima's forward search over the points y - h, y, y + h)
+// and the distances into them.
+struct CacheYWin {
+    int left, im, i, ip;
+    double tm, t, tp, h2;
+};
+
+template <bool DER>
+HC_HD CacheYWin cache_ywin(int n, const double *v, int left, double y)
+{
+    CacheYWin u;
+    u.left = left;
+    const int lo = left - 2 < 0 ? 0 : left - 2;
+    const bool four = (left + 1 >= n ? n - 1 : left + 1) - lo == 3;
+    const double a = v[lo], b = v[lo + 1], c = v[lo + 2];
+    auto from = [&](int i, double t) {
+        if (i == 0 && t > b) i = 1;
+        return four && i == 1 && t > c ? 2 : i;
+    };
+    auto at = [&](int i) { return i == 0 ? a : i == 1 ? b : c; };
+    if (DER) {
+        const double h = y * 1.0E-6;
+        u.im = from(0, y - h);
+        u.i = from(u.im, y);
+        u.ip = from(u.i, y + h);
+        u.tm = (y - h) - at(u.im);
+        u.tp = (y + h) - at(u.ip);
+        u.h2 = 2.0 * h;
+    } else {
+        u.im = u.i = u.ip = from(0, y);
+        u.tm = u.tp = u.h2 = 0.0;
+    }
+    u.t = y - at(u.i);
+    return u;
+}
+
+// Value and, with DER, y derivative of the component and z plane whose part of the
+// table is tab.
+template <bool DER>
+HC_HD void cache_spline_tab(int X, int Y, const double *tab, const CacheXWin &w, const CacheYWin &u, double &v,
+                            double &dv)
+{
+    const size_t is = (size_t)X * Y * 4;
+    const double *p = tab + ((size_t)u.left * X + w.x0) * 4;
+    double q[4], d[4];
+#pragma unroll
+    for (int b = 0; b < 4; b++) {
+        const double *r = p + 4 * (b == 3 && !w.w4 ? 2 : b);  // (a row that the axis does not have is not read)
+        const CacheD2 lo = cache_ld2(r + u.i * is), hi = cache_ld2(r + u.i * is + 2);
+        q[b] = lo.a + lo.b * u.t + hi.a * u.t * u.t + hi.b * u.t * u.t * u.t;
+        if (DER) {
+            CacheD2 l = lo, g = hi;
+            if (u.im != u.i) l = cache_ld2(r + u.im * is), g = cache_ld2(r + u.im * is + 2);
+            const double om = l.a + l.b * u.tm + g.a * u.tm * u.tm + g.b * u.tm * u.tm * u.tm;
+            l = lo, g = hi;
+            if (u.ip != u.i) l = cache_ld2(r + u.ip * is), g = cache_ld2(r + u.ip * is + 2);
+            const double op = l.a + l.b * u.tp + g.a * u.tp * u.tp + g.b * u.tp * u.tp * u.tp;
+            d[b] = (op - om) / u.h2;
+        }
+    }
+    v = cache_xspline(w, q[0], q[1], q[2], q[3]);
+    if (DER) dv = cache_xspline(w, d[0], d[1], d[2], d[3]);
+}
+
+// cache_lookup's status of (x, y) in z plane zindex, or for the plane -1 of a cache
+// with too few planes to interpolate in, before anything is read but the flags.
+HC_HD int cache_lookup_status(const CacheView &c, const double *vx, const double *vy, double x, double y, double z,
+                              int zindex, int lx, int ly)
+{
+    int rolling = 0;
+    int s = cache_axis_check(c.xtype, c.X, vx, x, true);
+    if (s == CACHE_OUT_OF_RANGE) return s;
+    rolling |= s == CACHE_NEEDS_RECENTRE;
+    s = cache_axis_check(c.ytype, c.Y, vy, y, true);
+    if (s == CACHE_OUT_OF_RANGE) return s;
+    rolling |= s == CACHE_NEEDS_RECENTRE;
+    s = cache_axis_check(c.ztype, c.Z, c.vz, z, zindex == -1);
+    if (s == CACHE_OUT_OF_RANGE) return s;
+    rolling |= s == CACHE_NEEDS_RECENTRE;
+    if (rolling) return CACHE_NEEDS_RECENTRE;
+    if (zindex < 0 || zindex >= c.Z) return CACHE_BAD_ZINDEX;
+    if (!c.whole) {
+        const int x0 = lx - 2 < 0 ? 0 : lx - 2, x1 = lx + 1 >= c.X ? c.X - 1 : lx + 1;
+        const int y0 = ly - 2 < 0 ? 0 : ly - 2, y1 = ly + 1 >= c.Y ? c.Y - 1 : ly + 1;
+        const long XY = (long)c.X * c.Y;
+        for (int ix = x0; ix <= x1; ix++)
+            for (int iy = y0; iy <= y1; iy++) {
+                const uint8_t f = c.counted[zindex * XY + (long)ix * c.Y + iy];
+                if (f == 0) return CACHE_MISSING;
+                if (f != 1) return CACHE_OUT_OF_RANGE;
+            }
+    }
+    return CACHE_OK;
+}
+
 // cache_lookup for one component k of a z plane (zindex >= 0) in spline mode:
 // the same status and bits, with the window's size fixed per call.
-HC_HD int cache_lookup(const CacheView &c, double x, double y, double z, int zindex, int mode, uint64_t mask,
-                       double *out, double *dery, size_t ostride);
-
-// With yco (the coefficient table of component k, plane zindex, of a cache
-// whose axes were checked when it was built) the y splines are read from it.
 template <bool DER>
-HC_HD int cache_lookup1(const CacheView &c, double x, double y, int zindex, int k, double &v, double &dv,
-                        const double *yco = nullptr)
+HC_HD int cache_lookup1(const CacheView &c, double x, double y, int zindex, int k, double &v, double &dv)
 {
     if (zindex == -1) {
         // interpolation in z (at z = 0): the general lookup
@@ -565,18 +766,6 @@ HC_HD int cache_lookup1(const CacheView &c, double x, double y, int zindex, int 
     }
     const int nx = x1 - x0 + 1, ny = y1 - y0 + 1;
     bool ok = true;
-    if (yco) {
-        const int left = cache_bracket(c.Y, c.vy, y);
-        if (nx == 4 && ny == 4)
-            cache_spline_win_co<4, 4, DER>(c, yco, x0, y0, left, x, y, v, dv, ok);
-        else if (nx == 4)
-            cache_spline_win_co<4, 3, DER>(c, yco, x0, y0, left, x, y, v, dv, ok);
-        else if (ny == 4)
-            cache_spline_win_co<3, 4, DER>(c, yco, x0, y0, left, x, y, v, dv, ok);
-        else
-            cache_spline_win_co<3, 3, DER>(c, yco, x0, y0, left, x, y, v, dv, ok);
-        return ok ? CACHE_OK : CACHE_OUT_OF_RANGE;
-    }
     if (nx == 4 && ny == 4)
         ok = cache_spline_win<4, 4, DER>(c, x0, y0, zindex, k, x, y, v, dv);
     else if (nx == 4)
@@ -598,14 +787,17 @@ HC_HD int cache_lookup1(const CacheView &c, double x, double y, int zindex, int 
 // reference's code (1 converged, errf <= tolf, T the last iterate; 2 or 0 not
 // converged, T the iterate of least error) or -1 when a lookup fails (the
 // reference reads values it did not get).
-HC_HD int cache_solve_T(const CacheView &c, double rho, double e, int zindex, double T0, double lo, double hi,
-                        int ntrial, double tolf, double &T, double &berr, const double *yco = nullptr)
+//
+// lookup(x, val, der) is one trial's lookup, false where it fails.
+template <class Fn>
+HC_HD int cache_newton_T(double e, double T0, double lo, double hi, int ntrial, double tolf, double &T, double &berr,
+                         Fn &&lookup)
 {
     double x = T0, best = T0, besterr = 1.0E100;
     int ret = 0;
     for (int k = 1; k <= ntrial; k++) {
         double val = 0.0, der = 0.0;
-        if (cache_lookup1<true>(c, rho, x, zindex, 0, val, der, yco) != CACHE_OK) {
+        if (!lookup(x, val, der)) {
             T = x;
             berr = besterr;
             return -1;

@@ -113,3 +113,42 @@ def test_temperature_solve_matches_oracle():
     counts = np.bincount(ret + 1, minlength=4)
     assert counts[2] > 1500 and counts[0] == 1, counts  # converged, and the one failed lookup
     c.close()
+
+
+@pytest.mark.parametrize("X,Y,Z,whole", [(3, 3, 1, True), (4, 5, 1, False), (5, 4, 3, True), (7, 3, 4, False)])
+def test_small_windows_and_grid_points_match_oracle(X, Y, Z, whole):
+    """The shortest axes, where every lookup's window touches an end (three rows on
+    either side, four with the query in the first or second interval), at grid points,
+    between them and at the axes' ends, with z planes and interpolation mixed."""
+    rng = np.random.default_rng(X * 100 + Y * 10 + Z)
+    types = (hc.AXIS_LOG, hc.AXIS_LOG, hc.AXIS_CUSTOM if Z == 1 else hc.AXIS_LINEAR)
+    desc, vx, vy, vz, values, counted = random_cache(rng, X=X, Y=Y, Z=Z, D=3, types=types)
+    if not whole:
+        counted[0, X - 1, Y - 1] = 0
+    c = hc.Cache.create(desc, vx, vy, vz, values, counted)
+    o = OracleCache(desc, vx, vy, vz, values, counted)
+    at = lambda v: sorted(set(list(v) + list(0.5 * (v[1:] + v[:-1])) +
+                              [v[0] * (1 - 1e-9), v[-1] * (1 + 1e-9), np.nextafter(v[1], 0), np.nextafter(v[1], 1e99),
+                               v[1] * (1 + 5e-7), v[1] * (1 - 5e-7)]))
+    pts, zidx = [], []
+    for x in at(vx):
+        for y in at(vy):
+            for q in range(-1, Z + 1):
+                pts.append((x, y, vz[0] if Z == 1 else 0.5 * (vz[0] + vz[1])))
+                zidx.append(q)
+    for der in (False, True):
+        st = _check(c, o, pts, zidx, True, None, der)
+    assert (st == hc.CACHE_OK).sum() > 50
+    c.close()
+
+
+def test_table_bracket_search_covers_both_axis_stores():
+    """Axes longer than the block's LDS share of them, against the same axes in it."""
+    rng = np.random.default_rng(77)
+    desc, vx, vy, vz, values, counted = random_cache(rng, X=2100, Y=5, Z=1, D=1,
+                                                      types=(hc.AXIS_LOG, hc.AXIS_LOG, hc.AXIS_CUSTOM))
+    c = hc.Cache.create(desc, vx, vy, vz, values, counted)
+    o = OracleCache(desc, vx, vy, vz, values, counted)
+    pts = query_points(rng, vx, vy, vz, 300)
+    _check(c, o, pts, [0] * len(pts), True, None, True)
+    c.close()
