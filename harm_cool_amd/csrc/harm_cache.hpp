@@ -269,45 +269,6 @@ HC_HD bool cache_akima_coefs(const double *xs, const double *ys, double *co)
     return true;
 }
 
-// The first three abscissae of a window (every window has at least three
-// points), read together and handed to the device code that follows as
-// register values (an empty asm takes them): their reads go out at once ahead
-// of the first comparison, and a pick among them stays a select.
-struct CacheAbsc {
-    double a0, a1, a2;
-};
-
-HC_HD CacheAbsc cache_absc(const double *ys)
-{
-    CacheAbsc w{ys[0], ys[1], ys[2]};
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+v"(w.a0), "+v"(w.a1), "+v"(w.a2));
-#endif
-    return w;
-}
-
-HC_HD double cache_absc_at(const CacheAbsc &w, int s) { return s == 0 ? w.a0 : (s == 1 ? w.a1 : w.a2); }
-
-// cache_akima_m's output points from those numbers: the same interval search
-// and the same cubic.  The search's abscissae are read together, ahead of it.
-template <int M, int NT>
-HC_HD void cache_akima_eval(const double *xs, const double *co, const double *ts, double *out)
-{
-    const CacheAbsc xv = cache_absc(xs);
-    int i = -1;
-#pragma unroll
-    for (int q = 0; q < NT; q++) {
-        const double t = ts[q];
-#pragma unroll
-        for (int s = 0; s <= M - 2; s++)
-            if ((i == s - 1) & (t > cache_absc_at(xv, s))) i = s;
-        if (i < 0) i = 0;
-        const double *ci = co + 4 * i;
-        const double t1 = t - cache_absc_at(xv, i);
-        out[q] = ci[0] + ci[1] * t1 + ci[2] * t1 * t1 + ci[3] * t1 * t1 * t1;
-    }
-}
-
 struct CacheView {
     int X, Y, Z, D;
     int xtype, ytype, ztype;
@@ -438,85 +399,6 @@ HC_HD bool cache_spline_win(const CacheView &c, int x0, int y0, int zp, int k, d
     ok &= cache_akima_m<NX, 1>(xs, xt, &x, &v);
     if (DER) ok &= cache_akima_m<NX, 1>(xs, xd, &x, &dv);
     return ok;
-}
-
-// Coefficient table of the splines along y of one component of one z plane:
-// for x row ix and bracket left = 1..Y-1 (the y window of a query in that
-// bracket, cache_window) the window's intervals' numbers (cache_akima_coefs),
-// [X][Y][3][4] doubles (left 0 unused; a 3-point window fills 2 intervals).
-constexpr int CACHE_YCO = 12;
-
-HC_HD void cache_ycoef_one(const CacheView &c, int zp, int k, int ix, int left, double *co)
-{
-    const int lo = left - 2 < 0 ? 0 : left - 2;
-    const int hi = left + 1 >= c.Y ? c.Y - 1 : left + 1;
-    const int m = hi - lo + 1;
-    const double *row = c.values + ((size_t)zp * c.X * c.Y + (size_t)ix * c.Y + lo) * c.D + k;
-    double yv[4];
-    for (int q = 0; q < m; q++) yv[q] = row[(size_t)q * c.D];
-    if (m == 4)
-        cache_akima_coefs<4>(c.vy + lo, yv, co);
-    else
-        cache_akima_coefs<3>(c.vy + lo, yv, co);
-}
-
-// cache_spline_win with the y splines read from a coefficient table.
-template <int NX, int NY, bool DER>
-HC_HD void cache_spline_win_co(const CacheView &c, const double *yco, int x0, int y0, int left, double x, double y,
-                               double &v, double &dv, bool &ok)
-{
-    const double *xs = c.vx + x0, *ys = c.vy + y0;
-    double xt[NX], xd[NX];
-    if (DER) {
-        // cache_akima_eval's intervals of the three points, shared by every row
-        // (the window's abscissae are the same); they almost always coincide, and
-        // then each row reads one interval's numbers
-        const double h = y * 1.0E-6;
-        const double ts[3] = {y - h, y, y + h};
-        const CacheAbsc yv = cache_absc(ys);
-        int iq[3], i = -1;
-#pragma unroll
-        for (int q = 0; q < 3; q++) {
-#pragma unroll
-            for (int s = 0; s <= NY - 2; s++)
-                if ((i == s - 1) & (ts[q] > cache_absc_at(yv, s))) i = s;
-            if (i < 0) i = 0;
-            iq[q] = i;
-        }
-        if (iq[0] == iq[2]) {
-            const int i0 = iq[0];
-            const double y0v = cache_absc_at(yv, i0);
-            const double t1[3] = {ts[0] - y0v, ts[1] - y0v, ts[2] - y0v};
-#pragma unroll
-            for (int b = 0; b < NX; b++) {
-                const double *ci = yco + ((size_t)(x0 + b) * c.Y + left) * CACHE_YCO + 4 * i0;
-                const double a0 = ci[0], a1 = ci[1], a2 = ci[2], a3 = ci[3];
-                double o3[3];
-#pragma unroll
-                for (int q = 0; q < 3; q++)
-                    o3[q] = a0 + a1 * t1[q] + a2 * t1[q] * t1[q] + a3 * t1[q] * t1[q] * t1[q];
-                xt[b] = o3[1];
-                xd[b] = (o3[2] - o3[0]) / (2.0 * h);
-            }
-        } else {
-#pragma unroll
-            for (int b = 0; b < NX; b++) {
-                const double *co = yco + ((size_t)(x0 + b) * c.Y + left) * CACHE_YCO;
-                double o3[3];
-                cache_akima_eval<NY, 3>(ys, co, ts, o3);
-                xt[b] = o3[1];
-                xd[b] = (o3[2] - o3[0]) / (2.0 * h);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int b = 0; b < NX; b++) {
-            const double *co = yco + ((size_t)(x0 + b) * c.Y + left) * CACHE_YCO;
-            cache_akima_eval<NY, 1>(ys, co, &y, &xt[b]);
-        }
-    }
-    ok &= cache_akima_m<NX, 1>(xs, xt, &x, &v);
-    if (DER) ok &= cache_akima_m<NX, 1>(xs, xd, &x, &dv);
 }
 
 // ---------------------------------------------------------------------------

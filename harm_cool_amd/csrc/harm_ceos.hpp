@@ -51,7 +51,7 @@ struct CeosHint {
 struct CeosParams {
     CacheView view;                // axes, sizes, types; view.values is unused
     const double *const *values;   // device array of n value pointers ([1][X][Y][D] each)
-    const double *const *yco;      // n coefficient tables of e and p along T ([2][X][Y][12] each)
+    const double *const *tab;      // n tables of the splines of e and p along T (cache_tab_plane each)
     int n;
     double rho_unit, u_unit, p_unit, gam;
     double rho_min, rho_max;       // rhoMin, rhoMax (g/cm^3)
@@ -114,30 +114,11 @@ __device__ __forceinline__ int ceos_hint_start(const CeosHint &h, double t)
     return ceos_ld(h.idx, d >= (unsigned long long)h.nk ? h.nk - 1 : (int)d);
 }
 
-template <bool DER>
-__device__ __forceinline__ bool ceos_win(const CacheView &c, const double *yco, int x0, int nx, int yb, double rho,
-                                         double t, double &v, double &dv)
-{
-    const int y0 = yb - 2 < 0 ? 0 : yb - 2;
-    const int y1 = yb + 1 >= c.Y ? c.Y - 1 : yb + 1;
-    const int ny = y1 - y0 + 1;
-    bool ok = true;
-    if (nx == 4 && ny == 4)
-        cache_spline_win_co<4, 4, DER>(c, yco, x0, y0, yb, rho, t, v, dv, ok);
-    else if (nx == 4)
-        cache_spline_win_co<4, 3, DER>(c, yco, x0, y0, yb, rho, t, v, dv, ok);
-    else if (ny == 4)
-        cache_spline_win_co<3, 4, DER>(c, yco, x0, y0, yb, rho, t, v, dv, ok);
-    else
-        cache_spline_win_co<3, 3, DER>(c, yco, x0, y0, yb, rho, t, v, dv, ok);
-    return ok;
-}
-
-// cache_solve_T on component 0 of plane 0 of a whole, non-rolling cache with
-// its coefficient tables (yco: e, then p), and at convergence p = P(rho, T):
-// every trial's lookup as cache_lookup1 makes it, with the density's window
-// formed once and the temperature's bracket walked from the trial before.
-__device__ inline int ceos_solve_Tp(const CacheView &c, const CeosHint &hx, const CeosHint &hy, const double *yco,
+// cache_newton_T on component 0 of plane 0 of a whole, non-rolling cache with the
+// tables of its splines along T (tab: e, then p), and at convergence p = P(rho, T):
+// the density's window is formed once, the temperature's bracket walked from the
+// trial before.
+__device__ inline int ceos_solve_Tp(const CacheView &c, const CeosHint &hx, const CeosHint &hy, const double *tab,
                                     double rho, double e, double T0, double lo, double hi, double &T, double &berr,
                                     double &pv)
 {
@@ -164,16 +145,13 @@ __device__ inline int ceos_solve_Tp(const CacheView &c, const CeosHint &hx, cons
         yb = cache_bracket(c.Y, c.vy, x);
     }
     const bool rho_in = !((rho < xlo) | (rho > xhi));
-    // cache_window's spline window around rho's bracket
-    const int x0 = left - 2 < 0 ? 0 : left - 2;
-    const int x1 = left + 1 >= c.X ? c.X - 1 : left + 1;
-    const int nx = x1 - x0 + 1;
+    const CacheXWin w = cache_xwin(c.X, c.vx, left, rho);
     for (int k = 1; k <= CEOS_NTRIAL; k++) {
         double val = 0.0, der = 0.0;
-        bool ok = rho_in & !((x < ylo) | (x > yhi));
+        const bool ok = rho_in & !((x < ylo) | (x > yhi));
         if (ok) {
             if (k > 1) yb = ceos_walk(c.Y, c.vy, x, yb);  // the first trial's T is T0, bracketed above
-            ok = ceos_win<true>(c, yco, x0, nx, yb, rho, x, val, der);
+            cache_spline_tab<true>(c.X, c.Y, tab, w, cache_ywin<true>(c.Y, c.vy, yb, x), val, der);
         }
         if (!ok) {
             T = x;
@@ -188,7 +166,8 @@ __device__ inline int ceos_solve_Tp(const CacheView &c, const CeosHint &hx, cons
             T = x;
             berr = errf;
             double unused;
-            ceos_win<false>(c, yco + (size_t)c.X * c.Y * CACHE_YCO, x0, nx, yb, rho, x, pv, unused);
+            cache_spline_tab<false>(c.X, c.Y, tab + cache_tab_plane(c.X, c.Y), w, cache_ywin<false>(c.Y, c.vy, yb, x),
+                                    pv, unused);
             return 1;
         }
         if (errf < besterr) {
@@ -218,7 +197,7 @@ __device__ __noinline__ CeosOut ceos_solve(const CeosParams *P, int r, double T,
     const double rho_min = P->rho_min, rho_max = P->rho_max, T_lo = P->T_lo, T_hi = P->T_hi;
     const CacheView c = P->view;
     const CeosHint hx = P->hx, hy = P->hy;
-    const double *yco = P->yco[r];
+    const double *tab = P->tab[r];
     CeosOut o{0., T, 0};
     const double rho = rho0 * rho_unit;
     const double e = u * u_unit;
@@ -233,7 +212,7 @@ __device__ __noinline__ CeosOut ceos_solve(const CeosParams *P, int r, double T,
     if (e < 0.0) return o;
     o.solved = 1;
     double Tn, berr, pv = 0.;
-    ceos_solve_Tp(c, hx, hy, yco, rho, e, o.T, T_lo, T_hi, Tn, berr, pv);
+    ceos_solve_Tp(c, hx, hy, tab, rho, e, o.T, T_lo, T_hi, Tn, berr, pv);
     if (berr > CEOS_TOL) {
         o.p = (gam - 1.) * u;
         return o;

@@ -1236,21 +1236,20 @@ k_update(DGrid g, const double *__restrict__ pi, const double *__restrict__ pb, 
 #define CEOS_EOS_WPE 2
 #endif
 
-// The coefficient tables of the splines along T of e and p of cache blockIdx.y
-// (cache_ycoef_one): one (component, x row, bracket) per thread.
-__global__ void __launch_bounds__(TPB) k_ceos_ycoef(CacheView v, const double *const *values,
-                                                   double *const *yco)
+// The tables of the splines along T of e and p of cache blockIdx.y (cache_tab_fill): one
+// (component, x row, bracket) per thread.
+__global__ void __launch_bounds__(TPB) k_ceos_table(CacheView v, const double *const *values, double *const *tab)
 {
     const size_t per = (size_t)v.X * v.Y;
     const size_t idx = (size_t)blockIdx.x * TPB + threadIdx.x;
     if (idx >= 2 * per) return;
     const int comp = (int)(idx / per);
     const size_t r = idx - (size_t)comp * per;
-    const int ix = (int)(r / (size_t)v.Y), left = (int)(r % (size_t)v.Y);
+    const int left = (int)(r / (size_t)v.X), ix = (int)(r % (size_t)v.X);
     if (left < 1) return;
     CacheView c = v;
     c.values = values[blockIdx.y];
-    cache_ycoef_one(c, 0, comp, ix, left, yco[blockIdx.y] + idx * CACHE_YCO);
+    cache_tab_fill(c, 0, comp, ix, left, tab[blockIdx.y] + comp * cache_tab_plane(v.X, v.Y));
 }
 
 // The stencil of a face along DIR: zones m-2, m-1 (left of the face), m, m+1.
@@ -3097,8 +3096,8 @@ struct harm_ctx {
     CeosParams ceos;
     double *lastT;
     const double **ceos_vals;
-    std::vector<double *> ceos_ycoef;  // per cache: the splines along T of e and p
-    double **ceos_yco;                 // device array of ceos_ycoef
+    std::vector<double *> ceos_tabs;  // per cache: the tables of its splines along T of e and p
+    double **ceos_tab;                 // device array of ceos_tabs
     double *ceos_fe;                   // [4][nz]: each face's p_l, cs2_l, p_r, cs2_r (k_face_eos)
     bool ceos_vanish;                  // the units make dp/drho, dp/du repeat calls (ceos_vanishing_steps)
     unsigned long long *ceos_solves;
@@ -3686,9 +3685,9 @@ void ctx_free(harm_ctx *c)
                     (void *)c->part, (void *)c->fix_bits, (void *)c->fix_pcount, (void *)c->fix_err, (void *)c->font.count, (void *)c->font.zone, (void *)c->font.U,
                     (void *)c->d_cblk, (void *)c->d_fblk, (void *)c->seeds.count, (void *)c->seeds.zone,
                     (void *)c->seeds.U, (void *)c->lastT, (void *)c->ceos_vals, (void *)c->ceos_solves,
-                    (void *)c->ceos_yco, (void *)c->ceos_fe, (void *)c->ceos_hint})
+                    (void *)c->ceos_tab, (void *)c->ceos_fe, (void *)c->ceos_hint})
         if (q) (void)hipFree(q);
-    for (double *q : c->ceos_ycoef) (void)hipFree(q);
+    for (double *q : c->ceos_tabs) (void)hipFree(q);
     for (int l = 0; l < 5; l++)
         if (c->d_geom[l]) (void)hipFree(c->d_geom[l]);
     for (auto &e : c->ev_pool) {
@@ -4318,16 +4317,16 @@ int harm_set_eos_cache(harm_ctx *c, const harm_cache *const *caches, int n, cons
     HIPCHK(hipMemcpy((void *)c->ceos_vals, vals.data(), (size_t)n * sizeof(double *), hipMemcpyHostToDevice));
     P.values = c->ceos_vals;
     // the splines along T of e and p, formed once per cache
-    const size_t nco = 2 * (size_t)v0.X * v0.Y * CACHE_YCO;
-    for (double *q : c->ceos_ycoef) (void)hipFree(q);
-    c->ceos_ycoef.assign((size_t)n, nullptr);
+    const size_t nco = 2 * cache_tab_plane(v0.X, v0.Y);
+    for (double *q : c->ceos_tabs) (void)hipFree(q);
+    c->ceos_tabs.assign((size_t)n, nullptr);
     for (int k = 0; k < n; k++)
-        if ((rc = dalloc(&c->ceos_ycoef[(size_t)k], nco))) return rc;
-    if (c->ceos_yco) (void)hipFree((void *)c->ceos_yco);
-    c->ceos_yco = nullptr;
-    if ((rc = dalloc(&c->ceos_yco, (size_t)n))) return rc;
-    HIPCHK(hipMemcpy((void *)c->ceos_yco, c->ceos_ycoef.data(), (size_t)n * sizeof(double *), hipMemcpyHostToDevice));
-    P.yco = c->ceos_yco;
+        if ((rc = dalloc(&c->ceos_tabs[(size_t)k], nco))) return rc;
+    if (c->ceos_tab) (void)hipFree((void *)c->ceos_tab);
+    c->ceos_tab = nullptr;
+    if ((rc = dalloc(&c->ceos_tab, (size_t)n))) return rc;
+    HIPCHK(hipMemcpy((void *)c->ceos_tab, c->ceos_tabs.data(), (size_t)n * sizeof(double *), hipMemcpyHostToDevice));
+    P.tab = c->ceos_tab;
     std::vector<int> hx, hy;
     P.hx = ceos_hint_table(ax0, hx);
     P.hy = ceos_hint_table(ay0, hy);
@@ -4340,8 +4339,8 @@ int harm_set_eos_cache(harm_ctx *c, const harm_cache *const *caches, int n, cons
         HIPCHK(hipMemcpy(c->ceos_hint + hx.size(), hy.data(), hy.size() * sizeof(int), hipMemcpyHostToDevice));
     P.hx.idx = c->ceos_hint;
     P.hy.idx = c->ceos_hint + hx.size();
-    hipLaunchKernelGGL(k_ceos_ycoef, dim3(nblocks(2 * (size_t)v0.X * v0.Y), (unsigned)n), dim3(TPB), 0, c->stream, v0,
-                       P.values, c->ceos_yco);
+    hipLaunchKernelGGL(k_ceos_table, dim3(nblocks(2 * (size_t)v0.X * v0.Y), (unsigned)n), dim3(TPB), 0, c->stream, v0,
+                       P.values, c->ceos_tab);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
     if (!c->lastT && (rc = dalloc(&c->lastT, c->nz))) return rc;
