@@ -250,16 +250,13 @@ struct EosCacheT {
         z->p = o.p;
         return o.p;
     }
-    // dpdrho_calc_CoolEOS (cooleos.c:704-741)
-    __device__ double dpdrho(double rho0, double u) const
+    // dpdrho_calc_CoolEOS (cooleos.c:704-741); p: the pressure call before it, at (rho0, u)
+    __device__ double dpdrho(double rho0, double u, double p) const
     {
         const double h = rho0 * CEOS_HH / P->rho_unit;
         const double rhoP = rho0 + h;
         double rhoM = rho0 - h;
-        if (V) {
-            const double p = pres(rho0, u);
-            return (rhoM > 0) ? (p - p) / (2.0 * h) : (p - p) / (h);
-        }
+        if (V) return (rhoM > 0) ? (p - p) / (2.0 * h) : (p - p) / (h);
         if (rhoM > 0) {
             const double pP = pres(rhoP, u);
             const double pM = pres(rhoM, u);
@@ -270,16 +267,13 @@ struct EosCacheT {
         const double pM = pres(rhoM, u);
         return (pP - pM) / (h);
     }
-    // dpdu_calc_CoolEOS (cooleos.c:667-701)
-    __device__ double dpdu(double rho0, double u) const
+    // dpdu_calc_CoolEOS (cooleos.c:667-701); p as for dpdrho
+    __device__ double dpdu(double rho0, double u, double p) const
     {
         const double h = u * CEOS_HH / P->u_unit;
         const double uP = u + h;
         double uM = u - h;
-        if (V) {
-            const double p = pres(rho0, u);
-            return (uM > 0) ? (p - p) / (2.0 * h) : (p - p) / (h);
-        }
+        if (V) return (uM > 0) ? (p - p) / (2.0 * h) : (p - p) / (h);
         if (uM > 0) {
             const double pP = pres(rho0, uP);
             const double pM = pres(rho0, uM);
@@ -295,8 +289,8 @@ struct EosCacheT {
     {
         const double e = u / rho;
         const double enthalpy = 1.0 + e + p / rho;
-        const double dpdr = dpdrho(rho, u);
-        const double dpde = dpdu(rho, u) * rho;
+        const double dpdr = dpdrho(rho, u, p);
+        const double dpde = dpdu(rho, u, p) * rho;
         return (dpdr + p / rho / rho * dpde) / enthalpy;
     }
 };
@@ -308,12 +302,11 @@ struct Eos5CacheT {
     EosCacheT<V> e;
     double gam;
     __device__ static constexpr bool tabulated() { return true; }
-    __device__ double p(double rho, double u) const { return e.pres(rho, u); }
-    __device__ void p_derivs(double rho, double u, double &p, double &dpdrho, double &dpdu) const
+    __device__ Eos5Pt at(double rho, double u) const { return Eos5Pt{e.pres(rho, u), 0., 0.}; }
+    __device__ void derivs(double rho, double u, Eos5Pt &pt) const
     {
-        p = e.pres(rho, u);
-        dpdrho = e.dpdrho(rho, u);
-        dpdu = e.dpdu(rho, u);
+        pt.dpdrho = e.dpdrho(rho, u, pt.p);
+        pt.dpdu = e.dpdu(rho, u, pt.p);
     }
 };
 

@@ -79,99 +79,57 @@ __device__ inline int eos_table_p(const EosTab &t, double rho, double u, double 
     return 1;
 }
 
-// The 5D solver's view of the EOS: tab == nullptr is the Gamma-law pressure.
+// The pressure at one iterate and, where the EOS forms them with it, its derivatives.
+struct Eos5Pt {
+    double p, dpdrho, dpdu;
+};
+
+// The 5D solver's view of the EOS: tab == nullptr is the Gamma-law pressure.  at() is
+// called once per iterate: its pressure serves the residual, the Jacobian and the
+// step's W, where each searched the table again (three times an iterate).
 struct Eos5 {
     const EosTab *tab;
     double gam;
     __device__ bool tabulated() const { return tab != nullptr; }
-    __device__ double p(double rho, double u) const
+    __device__ Eos5Pt at(double rho, double u) const
     {
-        if (!tab) return (gam - 1.) * u;
-        double pp, a, b;
-        eos_table_p(*tab, rho, u, pp, a, b);
-        return pp;
+        Eos5Pt e{(gam - 1.) * u, 0., 0.};
+        if (tab) eos_table_p(*tab, rho, u, e.p, e.dpdrho, e.dpdu);
+        return e;
     }
-    __device__ void p_derivs(double rho, double u, double &p, double &dpdrho, double &dpdu) const
-    {
-        eos_table_p(*tab, rho, u, p, dpdrho, dpdu);
-    }
+    __device__ void derivs(double, double, Eos5Pt &) const {}
 };
 
 // ---- utoprim_5d.c, restated for one zone -----------------------------------
 constexpr int N5 = 5;
 
-// ucon_calc_g / bcon_calc_g / lower_g / ncov_calc (u2p_util.c:204-300)
-__device__ __forceinline__ void ucon_calc_g5(const double *pr, const Geom &g, double *ucon)
+// The numbers of one zone's metric and field that every iterate uses.
+struct Zone5 {
+    double lapse;          // sqrt(-1 / g^tt) (ncov_calc, u2p_util.c:204-210; n_t = -lapse)
+    double alpha, ralpha;  // 1 / sqrt(-g^tt) (u2p_util.c:95) and its reciprocal
+    double boa[4];         // beta^j / alpha, beta^j = g^tj alpha alpha
+};
+
+__device__ __forceinline__ Zone5 zone5(const Geom &g)
 {
-    const double ut[4] = {0., pr[U1], pr[U2], pr[U3]};
-    double utsq = 0.;
+    Zone5 z;
+    z.lapse = sqrt(-1. / g.gcon[0][0]);
+    z.alpha = 1.0 / sqrt(-g.gcon[0][0]);
+    z.ralpha = 1.0 / z.alpha;
+    z.boa[0] = 0.;
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) utsq += g.gcov[i][j] * ut[i] * ut[j];
-    utsq = fabs(utsq);
-    const double gamma = sqrt(1. + utsq);
-    const double lapse = sqrt(-1. / g.gcon[0][0]);
-#pragma unroll
-    for (int i = 0; i < 4; i++) ucon[i] = ut[i] - lapse * gamma * g.gcon[0][i];
+    for (int j = 1; j < 4; j++) z.boa[j] = g.gcon[0][j] * z.alpha * z.alpha / z.alpha;
+    return z;
 }
+
 __device__ __forceinline__ void lower_g5(const double *vcon, const Geom &g, double *vcov)
 {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        vcov[i] = 0.;
+        vcov[i] = g.gcov[i][0] * vcon[0];
 #pragma unroll
-        for (int j = 0; j < 4; j++) vcov[i] += g.gcov[i][j] * vcon[j];
+        for (int j = 1; j < 4; j++) vcov[i] += g.gcov[i][j] * vcon[j];
     }
-}
-__device__ __forceinline__ void bcon_calc_g5(const double *pr, const double *ucon, const double *ucov,
-                                             const double *ncov, double *bcon)
-{
-    double Bcon[4];
-    Bcon[0] = 0.;
-#pragma unroll
-    for (int i = 1; i < 4; i++) Bcon[i] = -ncov[0] * pr[B1 + i - 1];
-    double u_dot_B = 0.;
-#pragma unroll
-    for (int i = 0; i < 4; i++) u_dot_B += ucov[i] * Bcon[i];
-    const double gamma = -ucon[0] * ncov[0];
-#pragma unroll
-    for (int i = 0; i < 4; i++) bcon[i] = (Bcon[i] + ucon[i] * u_dot_B) / gamma;
-}
-
-// primtoU_g (u2p_util.c:84-145) with the solver's EOS.
-template <class E5>
-__device__ inline void primtoU_g5(const E5 &eos, const double *pr, const Geom &g, double *U)
-{
-    double ucon[4], ucov[4], bcon[4], bcov[4], ncov[4];
-    const double alpha = 1.0 / sqrt(-g.gcon[0][0]);
-    ucon_calc_g5(pr, g, ucon);
-    lower_g5(ucon, g, ucov);
-    ncov[0] = -sqrt(-1. / g.gcon[0][0]);
-    ncov[1] = ncov[2] = ncov[3] = 0.;
-    const double gamma = -ncov[0] * ucon[0];
-    bcon_calc_g5(pr, ucon, ucov, ncov, bcon);
-    lower_g5(bcon, g, bcov);
-    double n_dot_b = 0., bsq = 0.;
-#pragma unroll
-    for (int i = 0; i < 4; i++) n_dot_b += ncov[i] * bcon[i];
-#pragma unroll
-    for (int i = 0; i < 4; i++) bsq += bcov[i] * bcon[i];
-    const double rho0 = pr[RHO], u = pr[UU];
-    const double p = eos.p(rho0, u);
-    const double w = rho0 + u + p;
-    U[RHO] = ucon[0] * rho0;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        U[1 + i] = gamma * (w + bsq) * ucov[i] - (p + bsq / 2.) * ncov[i] + n_dot_b * bcov[i];
-        U[1 + i] /= alpha;
-    }
-    U[1] = U[1] + U[RHO];
-    U[B1] = pr[B1];
-    U[B2] = pr[B2];
-    U[B3] = pr[B3];
-#pragma unroll
-    for (int i = 0; i < NPR; i++) U[i] *= g.g;
 }
 
 // gamma_calc_g (u2p_util.c:319-341); on failure gamma = sqrt(1 + |utsq|).
@@ -189,218 +147,82 @@ __device__ __forceinline__ int gamma_calc_g5(const double *pr, const Geom &g, do
     return bad;
 }
 
-// dudp_calc_g (utoprim_5d.c:409-529) with its helpers (utoprim_5d.c:531-640).
-template <class E5>
-__device__ inline void dudp_calc_g5(const E5 &eos, const double *pr, const Geom &g, double (&Am)[N5][N5])
-{
-    double dutdui[4], dbtdui[4], dbsqdui[4], dbiduj[4][4], dgdvi[4], duidvj[4][4];
-    double dudduu[4][4], dbdiduj[4][4], tempA[N5][N5];
-    double bcon[4], bcov[4], ucov[4], ucon[4], ncov[4], B[4], Bcov[4];
-#pragma unroll
-    for (int j = 0; j < N5; j++)
-#pragma unroll
-        for (int k = 0; k < N5; k++) tempA[j][k] = Am[j][k] = 0.;
-    ucon_calc_g5(pr, g, ucon);
-    lower_g5(ucon, g, ucov);
-    ncov[0] = -sqrt(-1. / g.gcon[0][0]);
-    ncov[1] = ncov[2] = ncov[3] = 0.;
-    bcon_calc_g5(pr, ucon, ucov, ncov, bcon);
-    lower_g5(bcon, g, bcov);
-    const double bsq = bcon[0] * bcov[0] + bcon[1] * bcov[1] + bcon[2] * bcov[2] + bcon[3] * bcov[3];
-#pragma unroll
-    for (int j = 1; j < 4; j++) dutdui[j] = -ucov[j] / ucov[0];
-    B[0] = 0.;
-#pragma unroll
-    for (int j = 1; j < 4; j++) B[j] = pr[j + B1 - 1];
-    lower_g5(B, g, Bcov);
-#pragma unroll
-    for (int j = 1; j < 4; j++) dbtdui[j] = Bcov[j] + Bcov[0] * dutdui[j];
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int k = 0; k < 4; k++) dbiduj[j][k] = 0.;
-#pragma unroll
-    for (int j = 1; j < 4; j++)
-#pragma unroll
-        for (int k = 1; k < 4; k++) dbiduj[j][k] = -bcon[j] * dutdui[k] / ucon[0] + ucon[j] * dbtdui[k] / ucon[0];
-#pragma unroll
-    for (int j = 1; j < 4; j++) dbiduj[j][j] += bcon[0] / ucon[0];
-#pragma unroll
-    for (int j = 1; j < 4; j++) dbiduj[0][j] = dbtdui[j];
-#pragma unroll
-    for (int j = 0; j < 4; j++) dbsqdui[j] = 0.;
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int k = 0; k < 4; k++) dbsqdui[j] += 2. * bcov[k] * dbiduj[k][j];
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int k = 1; k < 4; k++) dudduu[j][k] = g.gcov[j][k] + g.gcov[j][0] * dutdui[k];
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int k = 1; k < 4; k++) {
-            dbdiduj[j][k] = 0.0;
-#pragma unroll
-            for (int l = 0; l < 4; l++) dbdiduj[j][k] += g.gcov[j][l] * dbiduj[l][k];
-        }
-    double eta;
-    if (eos.tabulated()) {
-        double p, dpdrho, dpdu;
-        eos.p_derivs(pr[RHO], pr[UU], p, dpdrho, dpdu);
-        eta = pr[RHO] + pr[UU] + p + bsq;
-        Am[RHO][RHO] = ucon[0];
-#pragma unroll
-        for (int j = 0; j < 4; j++) Am[UU + j][RHO] = (1.0 + dpdrho) * ucon[0] * ucov[j] + (j == 0 ? 1. : 0.) * dpdrho;
-        Am[RHO][UU] = 0.0;
-#pragma unroll
-        for (int j = 0; j < 4; j++) Am[UU + j][UU] = (1.0 + dpdu) * ucon[0] * ucov[j] + (j == 0 ? 1. : 0.) * dpdu;
-    } else {
-        const double GAMMA = eos.gam;
-        eta = pr[RHO] + GAMMA * pr[UU] + bsq;
-        Am[RHO][RHO] = ucon[0];
-#pragma unroll
-        for (int j = 0; j < 4; j++) Am[UU + j][RHO] = ucon[0] * ucov[j];
-        Am[RHO][UU] = 0.0;
-#pragma unroll
-        for (int j = 0; j < 4; j++) Am[UU + j][UU] = GAMMA * ucon[0] * ucov[j] + (j == 0 ? 1. : 0.) * (GAMMA - 1.0);
-    }
-#pragma unroll
-    for (int j = 1; j < 4; j++) Am[RHO][U1 + j - 1] = pr[RHO] * dutdui[j];
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int k = 1; k < 4; k++)
-            Am[UU + j][U1 + k - 1] = dbsqdui[k] * ucon[0] * ucov[j] +
-                                    eta * (dutdui[k] * ucov[j] + ucon[0] * dudduu[j][k]) +
-                                    (j == 0 ? 1. : 0.) * 0.5 * dbsqdui[k] -
-                                    (dbtdui[k] * bcov[j] + bcon[0] * dbdiduj[j][k]);
-#pragma unroll
-    for (int k = 0; k < N5; k++) Am[UU][k] += Am[RHO][k];
-    double gamma;
-    gamma_calc_g5(pr, g, gamma);
-#pragma unroll
-    for (int j = 1; j < 4; j++) dgdvi[j] = 0.0;
-#pragma unroll
-    for (int j = 1; j < 4; j++)
-#pragma unroll
-        for (int k = 1; k < 4; k++) dgdvi[j] += 1.0 / gamma * g.gcov[j][k] * pr[U1 + k - 1];
-    const double alpha = 1.0 / sqrt(-g.gcon[0][0]);
-    double betacon[4];
-#pragma unroll
-    for (int j = 1; j < 4; j++) betacon[j] = g.gcon[0][j] * alpha * alpha;
-#pragma unroll
-    for (int j = 1; j < 4; j++) duidvj[0][j] = dgdvi[j] / alpha;
-#pragma unroll
-    for (int j = 1; j < 4; j++)
-#pragma unroll
-        for (int k = 1; k < 4; k++) duidvj[j][k] = (j == k ? 1. : 0.) - betacon[j] / alpha * dgdvi[k];
-#pragma unroll
-    for (int i = 0; i < N5; i++)
-#pragma unroll
-        for (int j = RHO; j <= UU; j++) tempA[i][j] = Am[i][j];
-#pragma unroll
-    for (int i = 0; i < N5; i++)
-#pragma unroll
-        for (int j = 1; j < 4; j++)
-#pragma unroll
-            for (int l = 1; l <= 3; l++) tempA[RHO + i][U1 + j - 1] += Am[RHO + i][U1 + l - 1] * duidvj[l][j];
-#pragma unroll
-    for (int j = 0; j < N5; j++)
-#pragma unroll
-        for (int k = 0; k < N5; k++) Am[j][k] = tempA[j][k] * g.g;
-}
-
-// LU_decompose / LU_substitution (utoprim_5d.c:672-874).
+// The linear solve of one Newton step (LU_decompose / LU_substitution,
+// utoprim_5d.c:672-874), B its right-hand side and result.  The row swaps act on B as
+// on A's columns: the reference swaps B during the forward substitution, at step i only
+// among rows i and below, which that substitution has not reached.
 __device__ inline void lu5_solve(double (&A)[N5][N5], double (&B)[N5])
 {
     const double absmin = 1e-30;
     double row_norm[N5];
-    int permute[N5];
-    int max_row = 0;
     const int n = N5;
+    bool zero = false;
 #pragma unroll
     for (int i = 0; i < n; i++) {
         double absmax = 0.;
 #pragma unroll
-        for (int j = 0; j < n; j++) {
-            const double m = fabs(A[i][j]);
-            if (m > absmax) absmax = m;
-        }
-        // a zero row: the reference returns before factorizing and then
-        // substitutes with the unfactorized matrix and a zero permutation
-        if (absmax == 0.) {
-#pragma unroll
-            for (int q = 0; q < n; q++) permute[q] = 0;
-            goto subst;
-        }
+        for (int j = 0; j < n; j++) absmax = fmax(absmax, fabs(A[i][j]));
+        zero |= absmax == 0.;
         row_norm[i] = 1. / absmax;
     }
+    if (zero) {
+        // the reference returns before factorizing and then substitutes with the
+        // unfactorized matrix and a zero permutation
 #pragma unroll
-    for (int j = 0; j < n; j++) {
+        for (int i = 0; i < n; i++) {
+            double tmpvar = B[0];
+            B[0] = B[i];
 #pragma unroll
-        for (int i = 0; i < j; i++)
-#pragma unroll
-            for (int k = 0; k < i; k++) A[i][j] -= A[i][k] * A[k][j];
-        double absmax = 0.0;
-#pragma unroll
-        for (int i = j; i < n; i++) {
-#pragma unroll
-            for (int k = 0; k < j; k++) A[i][j] -= A[i][k] * A[k][j];
-            const double m = fabs(A[i][j]) * row_norm[i];
-            if (m >= absmax) {
-                absmax = m;
-                max_row = i;
-            }
+            for (int j = i - 1; j >= 0; j--) tmpvar -= A[i][j] * B[j];
+            B[i] = tmpvar;
         }
-        if (max_row != j) {
-            if ((j == (n - 2)) && (A[j][j + 1] == 0.)) {
-                max_row = j;
-            } else {
+    } else {
 #pragma unroll
-                for (int k = 0; k < n; k++) {
-                    // rows j and max_row swapped with register-resident
-                    // arrays: select instead of dynamic indexing
-                    double aj = A[j][k], am = 0.;
+        for (int j = 0; j < n; j++) {
 #pragma unroll
-                    for (int r = 0; r < n; r++)
-                        if (r == max_row) am = A[r][k];
+            for (int i = 0; i < j; i++)
 #pragma unroll
-                    for (int r = 0; r < n; r++)
-                        if (r == max_row) A[r][k] = aj;
-                    A[j][k] = am;
+                for (int k = 0; k < i; k++) A[i][j] -= A[i][k] * A[k][j];
+            double absmax = 0.0;
+            int max_row = j;
+#pragma unroll
+            for (int i = j; i < n; i++) {
+#pragma unroll
+                for (int k = 0; k < j; k++) A[i][j] -= A[i][k] * A[k][j];
+                const double m = fabs(A[i][j]) * row_norm[i];
+                if (m >= absmax) {
+                    absmax = m;
+                    max_row = i;
                 }
-                double rn = 0.;
+            }
+            if (max_row != j && !((j == (n - 2)) && (A[j][j + 1 < n ? j + 1 : j] == 0.))) {
+                // rows j and max_row by selects: the rows are registers
 #pragma unroll
-                for (int r = 0; r < n; r++)
-                    if (r == j) rn = row_norm[r];
+                for (int r = j + 1; r < n; r++) {
+                    const bool sw = r == max_row;
 #pragma unroll
-                for (int r = 0; r < n; r++)
-                    if (r == max_row) row_norm[r] = rn;
+                    for (int k = 0; k < n; k++) {
+                        const double a = A[j][k], b = A[r][k];
+                        A[j][k] = sw ? b : a;
+                        A[r][k] = sw ? a : b;
+                    }
+                    const double a = B[j], b = B[r];
+                    B[j] = sw ? b : a;
+                    B[r] = sw ? a : b;
+                    row_norm[r] = sw ? row_norm[j] : row_norm[r];
+                }
+            }
+            if (A[j][j] == 0.) A[j][j] = absmin;
+            if (j != (n - 1)) {
+                const double inv = 1. / A[j][j];
+#pragma unroll
+                for (int i = j + 1; i < n; i++) A[i][j] *= inv;
             }
         }
-        permute[j] = max_row;
-        if (A[j][j] == 0.) A[j][j] = absmin;
-        if (j != (n - 1)) {
-            const double inv = 1. / A[j][j];
 #pragma unroll
-            for (int i = j + 1; i < n; i++) A[i][j] *= inv;
-        }
-    }
-subst:
+        for (int i = 0; i < n; i++)
 #pragma unroll
-    for (int i = 0; i < n; i++) {
-        double tmpvar = 0., bi = B[i];
-#pragma unroll
-        for (int r = 0; r < n; r++)
-            if (r == permute[i]) tmpvar = B[r];
-#pragma unroll
-        for (int r = 0; r < n; r++)
-            if (r == permute[i]) B[r] = bi;
-#pragma unroll
-        for (int j = i - 1; j >= 0; j--) tmpvar -= A[i][j] * B[j];
-        B[i] = tmpvar;
+            for (int j = i - 1; j >= 0; j--) B[i] -= A[i][j] * B[j];
     }
 #pragma unroll
     for (int i = n - 1; i >= 0; i--) {
@@ -410,18 +232,163 @@ subst:
     }
 }
 
-// func_5d (utoprim_5d.c:250-359), NORMMETHOD 1.
+// func_5d (utoprim_5d.c:250-359), NORMMETHOD 1, with primtoU_g (u2p_util.c:84-145) and
+// dudp_calc_g (utoprim_5d.c:409-529, its helpers 531-640): the Newton step dx, f and df
+// at the iterate x with the EOS numbers e.  The two share the four-velocity and the
+// field's four-vector; quotients by one denominator (u^t, alpha, u_t, the field's
+// gamma) go through its reciprocal (div_r, correctly rounded); the reference's sums
+// start from 0 and carry terms with the zero components, which change no value.
 template <class E5>
-__device__ inline void func_5d(const E5 &eos, const double *U_target, const Geom &g, const double *x,
-                               double (&dx)[N5], double &f, double &df)
+__device__ inline void func_5d(const E5 &eos, const double *U_target, const Geom &g, const Zone5 &z, const double *x,
+                               const double *Bf, Eos5Pt e, double (&dx)[N5], double &f, double &df)
 {
-    double pr[NPR], U_curr[NPR], Am[N5][N5];
+    double ucon[4], ucov[4], bcon[4], bcov[4], Bcov[4], resid[N5], Am[N5][N5];
+    {
+        double utsq = 0.;
 #pragma unroll
-    for (int i = 0; i < B1; i++) pr[i] = x[i];
+        for (int i = 1; i < 4; i++)
 #pragma unroll
-    for (int i = B1; i <= B3; i++) pr[i] = U_target[i] / g.g;
-    primtoU_g5(eos, pr, g, U_curr);
-    dudp_calc_g5(eos, pr, g, Am);
+            for (int j = 1; j < 4; j++) utsq += g.gcov[i][j] * x[UU + i] * x[UU + j];
+        const double gamma = sqrt(1. + fabs(utsq));
+        const double lg = z.lapse * gamma;
+        ucon[0] = 0. - lg * g.gcon[0][0];
+#pragma unroll
+        for (int i = 1; i < 4; i++) ucon[i] = x[UU + i] - lg * g.gcon[0][i];
+    }
+    lower_g5(ucon, g, ucov);
+    const double gb = ucon[0] * z.lapse;
+    {
+        double Bn[4], u_dot_B = 0.;
+        Bn[0] = 0.;
+#pragma unroll
+        for (int i = 1; i < 4; i++) {
+            Bn[i] = z.lapse * Bf[i - 1];
+            u_dot_B += ucov[i] * Bn[i];
+        }
+        const double rgb = 1. / gb;
+#pragma unroll
+        for (int i = 0; i < 4; i++) bcon[i] = div_r(Bn[i] + ucon[i] * u_dot_B, gb, rgb);
+    }
+    lower_g5(bcon, g, bcov);
+    const double bsq = bcon[0] * bcov[0] + bcon[1] * bcov[1] + bcon[2] * bcov[2] + bcon[3] * bcov[3];
+    df = 0.;
+    {
+        const double w = x[RHO] + x[UU] + e.p;
+        const double ndb = -z.lapse * bcon[0];
+        double Uc[N5];
+        Uc[RHO] = ucon[0] * x[RHO];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            double t = gb * (w + bsq) * ucov[i];
+            if (i == 0) t -= (e.p + bsq / 2.) * -z.lapse;
+            Uc[1 + i] = div_r(t + ndb * bcov[i], z.alpha, z.ralpha);
+        }
+        Uc[1] = Uc[1] + Uc[RHO];
+#pragma unroll
+        for (int k = 0; k < N5; k++) {
+            const double u = Uc[k] * g.g;
+            resid[k] = u - U_target[k];
+            double residnorm = 0.5 * (fabs(u) + fabs(U_target[k]));
+            residnorm = (residnorm == 0.) ? 1. : 1. / residnorm;
+            df -= residnorm * resid[k] * resid[k];
+        }
+    }
+    f = -0.5 * df;
+
+    const double ru = 1. / ucon[0], rut = 1. / ucov[0];
+    const double bu = div_r(bcon[0], ucon[0], ru);
+    Bcov[0] = 0.;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        Bcov[j] = g.gcov[j][1] * Bf[0];
+        Bcov[j] += g.gcov[j][2] * Bf[1];
+        Bcov[j] += g.gcov[j][3] * Bf[2];
+    }
+    if (eos.tabulated()) {
+        eos.derivs(x[RHO], x[UU], e);
+        Am[RHO][RHO] = ucon[0];
+        Am[RHO][UU] = 0.0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            Am[UU + j][RHO] = (1.0 + e.dpdrho) * ucon[0] * ucov[j];
+            Am[UU + j][UU] = (1.0 + e.dpdu) * ucon[0] * ucov[j];
+        }
+        Am[UU][RHO] += e.dpdrho;
+        Am[UU][UU] += e.dpdu;
+    } else {
+        const double GAMMA = eos.gam;
+        Am[RHO][RHO] = ucon[0];
+        Am[RHO][UU] = 0.0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            Am[UU + j][RHO] = ucon[0] * ucov[j];
+            Am[UU + j][UU] = GAMMA * ucon[0] * ucov[j];
+        }
+        Am[UU][UU] += GAMMA - 1.0;
+    }
+    const double eta = eos.tabulated() ? x[RHO] + x[UU] + e.p + bsq : x[RHO] + eos.gam * x[UU] + bsq;
+    // dU/du^k
+    double At[N5][3];
+#pragma unroll
+    for (int k = 1; k < 4; k++) {
+        const double dut = div_r(-ucov[k], ucov[0], rut);
+        const double dbt = Bcov[k] + Bcov[0] * dut;
+        double dbi[4], dbsq;
+        dbi[0] = dbt;
+#pragma unroll
+        for (int j = 1; j < 4; j++) {
+            dbi[j] = div_r(-bcon[j] * dut, ucon[0], ru) + div_r(ucon[j] * dbt, ucon[0], ru);
+            if (j == k) dbi[j] += bu;
+        }
+        dbsq = 2. * bcov[0] * dbi[0];
+#pragma unroll
+        for (int j = 1; j < 4; j++) dbsq += 2. * bcov[j] * dbi[j];
+        At[RHO][k - 1] = x[RHO] * dut;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const double dud = g.gcov[j][k] + g.gcov[j][0] * dut;
+            double dbd = g.gcov[j][0] * dbi[0];
+#pragma unroll
+            for (int l = 1; l < 4; l++) dbd += g.gcov[j][l] * dbi[l];
+            double a = dbsq * ucon[0] * ucov[j] + eta * (dut * ucov[j] + ucon[0] * dud);
+            if (j == 0) a += 0.5 * dbsq;
+            At[UU + j][k - 1] = a - (dbt * bcov[j] + bcon[0] * dbd);
+        }
+    }
+    Am[UU][RHO] += Am[RHO][RHO];
+    Am[UU][UU] += Am[RHO][UU];
+#pragma unroll
+    for (int k = 0; k < 3; k++) At[UU][k] += At[RHO][k];
+    // du^l/dv^j, l = 1..3 (the reference's product leaves l = 0 out)
+    double dg[4];
+    {
+        double gamma;
+        gamma_calc_g5(x, g, gamma);
+        const double ig = 1.0 / gamma;
+#pragma unroll
+        for (int j = 1; j < 4; j++) {
+            dg[j] = ig * g.gcov[j][1] * x[U1];
+            dg[j] += ig * g.gcov[j][2] * x[U2];
+            dg[j] += ig * g.gcov[j][3] * x[U3];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < N5; i++)
+#pragma unroll
+        for (int j = 1; j < 4; j++) {
+            double a = 0.;
+#pragma unroll
+            for (int l = 1; l <= 3; l++) {
+                const double d = (j == l ? 1. : 0.) - z.boa[l] * dg[j];
+                a = l == 1 ? At[i][0] * d : a + At[i][l - 1] * d;
+            }
+            Am[i][U1 + j - 1] = a * g.g;
+        }
+#pragma unroll
+    for (int i = 0; i < N5; i++) {
+        Am[i][RHO] *= g.g;
+        Am[i][UU] *= g.g;
+    }
     double norm = 0.0;
     int numnormterms = 0;
 #pragma unroll
@@ -437,16 +404,8 @@ __device__ inline void func_5d(const E5 &eos, const double *U_target, const Geom
     for (int j = 0; j < N5; j++)
 #pragma unroll
         for (int k = 0; k < N5; k++) Am[j][k] *= (norm);
-    df = 0.;
 #pragma unroll
-    for (int k = 0; k < N5; k++) {
-        const double resid = U_curr[k] - U_target[k];
-        dx[k] = -resid * (norm);
-        double residnorm = 0.5 * (fabs(U_curr[k]) + fabs(U_target[k]));
-        residnorm = (residnorm == 0.) ? 1. : 1. / residnorm;
-        df -= residnorm * resid * resid;
-    }
-    f = -0.5 * df;
+    for (int k = 0; k < N5; k++) dx[k] = -resid[k] * (norm);
     lu5_solve(Am, dx);
 }
 
@@ -460,12 +419,14 @@ __device__ inline int utoprim_5d(const double *U, const Geom &g, const E5 &eos, 
     double x[N5];
 #pragma unroll
     for (int k = 0; k < N5; k++) x[k] = prim[k];
+    const Zone5 z5 = zone5(g);
+    Eos5Pt e = eos.at(x[RHO], x[UU]);
     double f = 1., df = 1., errx = 1., W = 0.;
     int n_iter = 0, i_extra = 0, doing_extra = 0;
     bool keep = true;
     while (keep) {
         double dx[N5];
-        func_5d(eos, U, g, x, dx, f, df);
+        func_5d(eos, U, g, z5, x, prim + B1, e, dx, f, df);
 #pragma unroll
         for (int id = 0; id < N5; id++) x[id] += dx[id];
         const double W_old = W;
@@ -475,8 +436,9 @@ __device__ inline int utoprim_5d(const double *U, const Geom &g, const E5 &eos, 
 #pragma unroll
             for (int jd = 1; jd < 4; jd++) vsq += g.gcov[id][jd] * x[U1 + id - 1] * x[U1 + jd - 1];
         const double gsqtmp = 1. + vsq;
+        e = eos.at(x[RHO], x[UU]);
         if (eos.tabulated())
-            W = gsqtmp * (x[UU] + x[RHO] + eos.p(x[RHO], x[UU]));
+            W = gsqtmp * (x[UU] + x[RHO] + e.p);
         else
             W = gsqtmp * (eos.gam * x[UU] + x[RHO]);
         errx = (W == 0.) ? fabs(W - W_old) : fabs((W - W_old) / W);
