@@ -284,9 +284,11 @@ struct EosCacheT {
         const double pM = pres(rho0, uM);
         return (pP - pM) / (h);
     }
+    __device__ EosPt at(double rho0, double u) const { return EosPt{pres(rho0, u), 0., 0.}; }
     // vchar's COOL_EOS sound speed (phys.c:365-377), after its pressure call
-    __device__ double cs2(double rho, double u, double p) const
+    __device__ double cs2(double rho, double u, const EosPt &pt) const
     {
+        const double p = pt.p;
         const double e = u / rho;
         const double enthalpy = 1.0 + e + p / rho;
         const double dpdr = dpdrho(rho, u, p);
@@ -302,8 +304,8 @@ struct Eos5CacheT {
     EosCacheT<V> e;
     double gam;
     __device__ static constexpr bool tabulated() { return true; }
-    __device__ Eos5Pt at(double rho, double u) const { return Eos5Pt{e.pres(rho, u), 0., 0.}; }
-    __device__ void derivs(double rho, double u, Eos5Pt &pt) const
+    __device__ EosPt at(double rho, double u) const { return e.at(rho, u); }
+    __device__ void derivs(double rho, double u, EosPt &pt) const
     {
         pt.dpdrho = e.dpdrho(rho, u, pt.p);
         pt.dpdu = e.dpdu(rho, u, pt.p);

@@ -1058,6 +1058,7 @@ k_update(DGrid g, const double *__restrict__ pi, const double *__restrict__ pb, 
     Geom geom;
     const double *blk = nullptr;
     double piz[NPR], U[NPR];
+    EosPt epi{};  // the EOS at piz
     if (active) {
         const unsigned rest = (unsigned)idx / (unsigned)g.N3;
         h = (int)((unsigned)idx - rest * (unsigned)g.N3);
@@ -1079,26 +1080,25 @@ k_update(DGrid g, const double *__restrict__ pi, const double *__restrict__ pb, 
 #pragma unroll
             for (int k = 0; k < NPR; k++) pbz[k] = FUSED ? at32(pb + k * nz, (unsigned)z) : pb[k * nz + z];
             State q;
-            if constexpr (TAB) {
-                const EosTable eos{g.tab, g.ref_derivs};
-                if (UNI)
-                    source(pbz, geom, blk + CENT_CONN, 1, 0, eos, dU, q, fatal);
-                else
-                    source(pbz, geom, g.conn, g.ncol, col, eos, dU, q, fatal);
-            } else {
-                if (UNI)
-                    source(pbz, geom, blk + CENT_CONN, 1, 0, g.gam, dU, q, fatal);
-                else
-                    source(pbz, geom, g.conn, g.ncol, col, g.gam, dU, q, fatal);
-            }
+            if constexpr (TAB)
+                epi = EosTable{g.tab, g.ref_derivs}.at(pbz[RHO], pbz[UU]);
+            else
+                epi = EosGamma{g.gam}.at(pbz[RHO], pbz[UU]);
+            if (UNI)
+                source(pbz, geom, blk + CENT_CONN, 1, 0, epi.p, dU, q, fatal);
+            else
+                source(pbz, geom, g.conn, g.ncol, col, epi.p, dU, q, fatal);
 #pragma unroll
             for (int k = 0; k < NPR; k++)
                 piz[k] = pi_is_pb ? pbz[k] : (FUSED ? at32(pi + k * nz, (unsigned)z) : pi[k * nz + z]);
-            if (!pi_is_pb) get_state(piz, geom, q, fatal);
-            if constexpr (TAB)
-                primtoflux(piz, q, 0, geom, EosTable{g.tab, g.ref_derivs}, U);
-            else
-                primtoflux(piz, q, 0, geom, g.gam, U);
+            if (!pi_is_pb) {
+                get_state(piz, geom, q, fatal);
+                if constexpr (TAB)
+                    epi = EosTable{g.tab, g.ref_derivs}.at(piz[RHO], piz[UU]);
+                else
+                    epi = EosGamma{g.gam}.at(piz[RHO], piz[UU]);
+            }
+            primtoflux_P(piz, q, 0, geom, epi.p, U);
         }
         if constexpr (FUSED) {
             double d[NPR];
@@ -1121,7 +1121,7 @@ k_update(DGrid g, const double *__restrict__ pi, const double *__restrict__ pb, 
             Eos5 e5;
             e5.tab = &g.tab;
             e5.gam = g.gam;
-            ret = utoprim_5d(U, geom, e5, pr, niter);
+            ret = utoprim_5d(U, geom, e5, epi, pr, niter);
             kconv = niter;
         }
     } else if constexpr (MODE == UPD_GATED) {
@@ -1330,15 +1330,15 @@ k_face_eos(DGrid g, CeosParams ce, double *__restrict__ lastT, const double *__r
         zs.T = lastT[z];
         if (chain && zs.T == 0.0 && j > g.js) zs.T = lastT[z - g.N3];
         const EosCacheT<V> eos{&ce, ceos_radius(ce, i), &zs};
-        const double pl = eos.pres(rl, ul);
-        const double cl = eos.cs2(rl, ul, pl);
-        const double pr = eos.pres(rr, ur);
-        const double cr = eos.cs2(rr, ur, pr);
+        const EosPt el = eos.at(rl, ul);
+        const double cl = eos.cs2(rl, ul, el);
+        const EosPt er = eos.at(rr, ur);
+        const double cr = eos.cs2(rr, ur, er);
         lastT[z] = zs.T;
         nsolve += zs.nsolve;
-        fe[0 * nz + z] = pl;
+        fe[0 * nz + z] = el.p;
         fe[1 * nz + z] = cl;
-        fe[2 * nz + z] = pr;
+        fe[2 * nz + z] = er.p;
         fe[3 * nz + z] = cr;
     });
     add_counter(solves, 0, nsolve);
@@ -1353,8 +1353,8 @@ struct EosGiven {
     {
         return __double_as_longlong(rho) == __double_as_longlong(rl) && __double_as_longlong(u) == __double_as_longlong(ul);
     }
-    __device__ double pres(double rho, double u) const { return left(rho, u) ? pl : pr; }
-    __device__ double cs2(double rho, double u, double) const { return left(rho, u) ? cl : cr; }
+    __device__ EosPt at(double rho, double u) const { return EosPt{left(rho, u) ? pl : pr, 0., 0.}; }
+    __device__ double cs2(double rho, double u, const EosPt &) const { return left(rho, u) ? cl : cr; }
 };
 
 // fluxcalc (step_ch.c:331-504) with the face pressures k_face_eos formed:
@@ -1447,11 +1447,15 @@ __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(CEOS_W
 #pragma unroll
         for (int k = 0; k < NPR; k++) pbz[k] = pb[k * nz + z];
         State q;
-        source(pbz, geom, g.conn, g.ncol, col, eos, dU, q, fatal);
+        EosPt e = eos.at(pbz[RHO], pbz[UU]);
+        source(pbz, geom, g.conn, g.ncol, col, e.p, dU, q, fatal);
 #pragma unroll
         for (int k = 0; k < NPR; k++) piz[k] = pi_is_pb ? pbz[k] : pi[k * nz + z];
-        if (!pi_is_pb) get_state(piz, geom, q, fatal);
-        primtoflux(piz, q, 0, geom, eos, U);
+        if (!pi_is_pb) {
+            get_state(piz, geom, q, fatal);
+            e = eos.at(piz[RHO], piz[UU]);
+        }
+        primtoflux_P(piz, q, 0, geom, e.p, U);
 #pragma unroll
         for (int k = 0; k < NPR; k++) U[k] += Dt * (S[k * na + idx] + dU[k]);
         double pr[NPR];
@@ -1459,7 +1463,7 @@ __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(CEOS_W
         for (int k = 0; k < NPR; k++) pr[k] = piz[k];
         int niter = 0;
         const Eos5CacheT<V> e5{eos, g.gam};
-        const int ret = utoprim_5d(U, geom, e5, pr, niter);
+        const int ret = utoprim_5d(U, geom, e5, e, pr, niter);
         lastT[z] = zs.T;
         nsolve = zs.nsolve;
         c_call = 1;
@@ -2172,7 +2176,7 @@ __global__ void __launch_bounds__(TPB) k_diag(DGrid g, const double *__restrict_
         State q;
         get_state(pr, geom, q, fatal);
         if (TAB)
-            primtoflux(pr, q, 0, geom, EosTable{g.tab, g.ref_derivs}, U);
+            primtoflux_P(pr, q, 0, geom, EosTable{g.tab, g.ref_derivs}.at(pr[RHO], pr[UU]).p, U);
         else
             primtoflux(pr, q, 0, geom, g.gam, U);
         acc[0] = U[RHO] * dV;
@@ -2676,10 +2680,12 @@ __global__ void __launch_bounds__(TPB) k_dump_cols(DGrid g, const double *__rest
     }
     double vmax, vmin;
     for (int dir = 1; dir <= 2; dir++) {
-        if (TAB)
-            vchar(pr, q, geom, dir, EosTable{g.tab, g.ref_derivs}, &vmax, &vmin);
-        else
+        if (TAB) {
+            const EosTable eos{g.tab, g.ref_derivs};
+            vchar(pr, q, geom, dir, eos, eos.at(pr[RHO], pr[UU]), &vmax, &vmin);
+        } else {
             vchar(pr, q, geom, dir, g.gam, &vmax, &vmin);
+        }
         o[36 + 2 * (dir - 1)] = vmin;
         o[37 + 2 * (dir - 1)] = vmax;
     }
@@ -2972,7 +2978,7 @@ __global__ void __launch_bounds__(TPB) k_c2p5_batch(const double *__restrict__ U
     eos.tab = tab.nr > 0 ? &tab : nullptr;
     eos.gam = gam;
     int niter = 0;
-    const int r = utoprim_5d(Uz, geom, eos, pr, niter);
+    const int r = utoprim_5d(Uz, geom, eos, eos.at(pr[RHO], pr[UU]), pr, niter);
 #pragma unroll
     for (int k = 0; k < NPR; k++) prim[(size_t)k * n + z] = pr[k];
     ret[z] = (int8_t)r;

@@ -79,11 +79,6 @@ __device__ inline int eos_table_p(const EosTab &t, double rho, double u, double 
     return 1;
 }
 
-// The pressure at one iterate and, where the EOS forms them with it, its derivatives.
-struct Eos5Pt {
-    double p, dpdrho, dpdu;
-};
-
 // The 5D solver's view of the EOS: tab == nullptr is the Gamma-law pressure.  at() is
 // called once per iterate: its pressure serves the residual, the Jacobian and the
 // step's W, where each searched the table again (three times an iterate).
@@ -91,13 +86,13 @@ struct Eos5 {
     const EosTab *tab;
     double gam;
     __device__ bool tabulated() const { return tab != nullptr; }
-    __device__ Eos5Pt at(double rho, double u) const
+    __device__ EosPt at(double rho, double u) const
     {
-        Eos5Pt e{(gam - 1.) * u, 0., 0.};
+        EosPt e{(gam - 1.) * u, 0., 0.};
         if (tab) eos_table_p(*tab, rho, u, e.p, e.dpdrho, e.dpdu);
         return e;
     }
-    __device__ void derivs(double, double, Eos5Pt &) const {}
+    __device__ void derivs(double, double, EosPt &) const {}
 };
 
 // ---- utoprim_5d.c, restated for one zone -----------------------------------
@@ -240,7 +235,7 @@ __device__ inline void lu5_solve(double (&A)[N5][N5], double (&B)[N5])
 // start from 0 and carry terms with the zero components, which change no value.
 template <class E5>
 __device__ inline void func_5d(const E5 &eos, const double *U_target, const Geom &g, const Zone5 &z, const double *x,
-                               const double *Bf, Eos5Pt e, double (&dx)[N5], double &f, double &df)
+                               const double *Bf, EosPt e, double (&dx)[N5], double &f, double &df)
 {
     double ucon[4], ucov[4], bcon[4], bcov[4], Bcov[4], resid[N5], Am[N5][N5];
     {
@@ -411,8 +406,9 @@ __device__ inline void func_5d(const E5 &eos, const double *U_target, const Geom
 
 // Utoprim_5d (utoprim_5d.c:179-239) with general_newton_raphson
 // (utoprim_5d.c:890-983) and calc_errx_5d (utoprim_5d.c:378-400).
+// e: the EOS at prim's density and energy.
 template <class E5>
-__device__ inline int utoprim_5d(const double *U, const Geom &g, const E5 &eos, double *prim, int &n_iter_out)
+__device__ inline int utoprim_5d(const double *U, const Geom &g, const E5 &eos, EosPt e, double *prim, int &n_iter_out)
 {
 #pragma unroll
     for (int k = B1; k <= B3; k++) prim[k] = U[k] / g.g;
@@ -420,7 +416,6 @@ __device__ inline int utoprim_5d(const double *U, const Geom &g, const E5 &eos, 
 #pragma unroll
     for (int k = 0; k < N5; k++) x[k] = prim[k];
     const Zone5 z5 = zone5(g);
-    Eos5Pt e = eos.at(x[RHO], x[UU]);
     double f = 1., df = 1., errx = 1., W = 0.;
     int n_iter = 0, i_extra = 0, doing_extra = 0;
     bool keep = true;
@@ -483,16 +478,16 @@ struct EosTable {
     static constexpr bool TAB = true;
     EosTab t;
     int ref_derivs;
-    __device__ double pres(double rho, double u) const
+    __device__ EosPt at(double rho, double u) const
     {
-        double p, a, b;
-        eos_table_p(t, rho, u, p, a, b);
-        return p;
+        EosPt e;
+        eos_table_p(t, rho, u, e.p, e.dpdrho, e.dpdu);
+        return e;
     }
-    __device__ double cs2(double rho, double u, double p) const
+    __device__ double cs2(double rho, double u, const EosPt &pt) const
     {
-        double pp, dpdrho, dpdu;
-        eos_table_p(t, rho, u, pp, dpdrho, dpdu);
+        const double p = pt.p;
+        double dpdrho = pt.dpdrho, dpdu = pt.dpdu;
         if (ref_derivs) {
             dpdrho = 0.;
             dpdu = 0.;

@@ -318,12 +318,19 @@ HD void get_state(const double *pr, const Geom &geom, State &q, int &fatal)
     lower(q.bcon, geom, q.bcov);
 }
 
+// An EOS at one (rho, u): the pressure and, where the EOS forms them with it, its
+// derivatives.  A state's EOS is evaluated once and handed on, as a tabulated one
+// searches its table for it.
+struct EosPt {
+    double p, dpdrho, dpdu;
+};
+
 // The Gamma-law EOS policy of the physics templates below (p = (gam - 1) u,
 // phys.c:150); the tabulated policy lives with the table (harm_eos5d.hpp).
 struct EosGamma {
     static constexpr bool TAB = false;
     double gam;
-    HD double pres(double, double u) const { return (gam - 1.) * u; }
+    HD EosPt at(double, double u) const { return EosPt{(gam - 1.) * u, 0., 0.}; }
 };
 
 // phys.c:122-161: one row of the MHD stress tensor for a given pressure P.
@@ -363,11 +370,6 @@ HD void primtoflux_P(const double *pr, const State &q, int dir, const Geom &geom
 }
 
 // phys.c:59-96
-template <class E>
-HD void primtoflux(const double *pr, const State &q, int dir, const Geom &geom, const E &eos, double *flux)
-{
-    primtoflux_P(pr, q, dir, geom, eos.pres(pr[RHO], pr[UU]), flux);
-}
 HD void primtoflux(const double *pr, const State &q, int dir, const Geom &geom, double gam, double *flux)
 {
     primtoflux_P(pr, q, dir, geom, (gam - 1.) * pr[UU], flux);
@@ -376,20 +378,20 @@ HD void primtoflux(const double *pr, const State &q, int dir, const Geom &geom, 
 // phys.c:337-476; returns how often the reference would fail().  Gamma-law:
 // cs2 = gam (gam - 1) u / (rho + gam u) and fail() outside [0, 1].  Tabulated
 // (phys.c:359-378, 398-406): cs2 from the EOS derivatives (E::cs2), clipped
-// to [SMALL, 1] without fail().
+// to [SMALL, 1] without fail().  pt: the EOS at the state.
 template <class E>
-HD int vchar(const double *pr, const State &q, const Geom &geom, int js, const E &eos, double *vmax, double *vmin)
+HD int vchar(const double *pr, const State &q, const Geom &geom, int js, const E &eos, const EosPt &pt, double *vmax,
+             double *vmin)
 {
     int nfail = 0;
     double bsq = dot4(q.bcon, q.bcov);
     double rho = pr[RHO], u = pr[UU];
     double cms2;
     if constexpr (E::TAB) {
-        const double p = eos.pres(rho, u);
-        double EF = rho + u + p;
+        double EF = rho + u + pt.p;
         double EE = bsq + EF;
         double va2 = bsq / EE;
-        double cs2 = eos.cs2(rho, u, p);
+        double cs2 = eos.cs2(rho, u, pt);
         cms2 = cs2 + va2 - cs2 * va2;
         if (cms2 < SMALL) cms2 = SMALL;
         if (cms2 > 1.) cms2 = 1.;
@@ -440,7 +442,7 @@ HD int vchar(const double *pr, const State &q, const Geom &geom, int js, const E
 }
 HD int vchar(const double *pr, const State &q, const Geom &geom, int js, double gam, double *vmax, double *vmin)
 {
-    return vchar(pr, q, geom, js, EosGamma{gam}, vmax, vmin);
+    return vchar(pr, q, geom, js, EosGamma{gam}, EosPt{}, vmax, vmin);
 }
 
 // interp.c:49-93
@@ -510,18 +512,18 @@ HD void face_flux(const double *p_l, const double *p_r, const Geom &geom, int di
         // the left state is finished before the right one is formed
         State sl;
         get_state(p_l, geom, sl, fatal);
-        const double P_l = eos.pres(p_l[RHO], p_l[UU]);
-        primtoflux_P(p_l, sl, dir, geom, P_l, F_l);
-        primtoflux_P(p_l, sl, 0, geom, P_l, U_l);
-        fatal += vchar(p_l, sl, geom, dir, eos, &cmax_l, &cmin_l);
+        const EosPt e_l = eos.at(p_l[RHO], p_l[UU]);
+        primtoflux_P(p_l, sl, dir, geom, e_l.p, F_l);
+        primtoflux_P(p_l, sl, 0, geom, e_l.p, U_l);
+        fatal += vchar(p_l, sl, geom, dir, eos, e_l, &cmax_l, &cmin_l);
     }
     {
         State sr;
         get_state(p_r, geom, sr, fatal);
-        const double P_r = eos.pres(p_r[RHO], p_r[UU]);
-        primtoflux_P(p_r, sr, dir, geom, P_r, F_r);
-        primtoflux_P(p_r, sr, 0, geom, P_r, U_r);
-        fatal += vchar(p_r, sr, geom, dir, eos, &cmax_r, &cmin_r);
+        const EosPt e_r = eos.at(p_r[RHO], p_r[UU]);
+        primtoflux_P(p_r, sr, dir, geom, e_r.p, F_r);
+        primtoflux_P(p_r, sr, 0, geom, e_r.p, U_r);
+        fatal += vchar(p_r, sr, geom, dir, eos, e_r, &cmax_r, &cmin_r);
     }
     double cmax = fabs(dmax(dmax(0., cmax_l), cmax_r));
     double cmin = fabs(dmax(dmax(0., -cmin_l), -cmin_r));
@@ -545,12 +547,11 @@ HD void face_flux(const double *p_l, const double *p_r, const Geom &geom, int di
 // conn[((k*4+mu)*4+j)*cstride + col] = Gamma^k_{mu j}: cstride = ncol for the
 // variable-major table, 1 (with col = 0 and conn at the column block) for the
 // column-major one.
-template <class E>
-HD void source(const double *ph, const Geom &geom, const double *__restrict__ conn, size_t ncol, size_t col,
-               const E &eos, double *dU, State &q, int &fatal)
+// P: the pressure at ph.
+HD void source(const double *ph, const Geom &geom, const double *__restrict__ conn, size_t ncol, size_t col, double P,
+               double *dU, State &q, int &fatal)
 {
     get_state(ph, geom, q, fatal);
-    const double P = eos.pres(ph[RHO], ph[UU]);
 #pragma unroll
     for (int k = 0; k < NPR; k++) dU[k] = 0.;
     // mhd_calc_P's row j with u^j, b^j picked by selects (an index into the
@@ -577,12 +578,6 @@ HD void source(const double *ph, const Geom &geom, const double *__restrict__ co
 #pragma unroll
     for (int k = 0; k < NPR; k++) dU[k] *= geom.g;
 }
-HD void source(const double *ph, const Geom &geom, const double *__restrict__ conn, size_t ncol, size_t col,
-               double gam, double *dU, State &q, int &fatal)
-{
-    source(ph, geom, conn, ncol, col, EosGamma{gam}, dU, q, fatal);
-}
-
 // ---------------------------------------------------------------------------
 // Conserved -> primitive inversion (utoprim_2d.c, utoprim_1dvsq2fix1.c,
 // utoprim_1dfix1.c, u2p_util.c).  The reference's file-scope solver globals are
