@@ -109,17 +109,17 @@ HD double dot4(const double *a, const double *b) { return a[0] * b[0] + a[1] * b
 struct dd {
     double hi, lo;
 };
-HD dd dd_two_sum(double a, double b)
+__host__ __device__ inline dd dd_two_sum(double a, double b)
 {
     double s = a + b, bb = s - a;
     return {s, (a - (s - bb)) + (b - bb)};
 }
-HD dd dd_fast(double a, double b)
+__host__ __device__ inline dd dd_fast(double a, double b)
 {
     double s = a + b;
     return {s, b - (s - a)};
 }
-HD dd dd_add(dd a, dd b)
+__host__ __device__ inline dd dd_add(dd a, dd b)
 {
     dd s = dd_two_sum(a.hi, b.hi);
     dd t = dd_two_sum(a.lo, b.lo);
@@ -128,21 +128,21 @@ HD dd dd_add(dd a, dd b)
     s.lo += t.lo;
     return dd_fast(s.hi, s.lo);
 }
-HD dd dd_mul(dd a, dd b)
+__host__ __device__ inline dd dd_mul(dd a, dd b)
 {
     double p = a.hi * b.hi;
     double e = fma(a.hi, b.hi, -p);
     e += a.hi * b.lo + a.lo * b.hi;
     return dd_fast(p, e);
 }
-HD dd dd_mul_d(dd a, double b)
+__host__ __device__ inline dd dd_mul_d(dd a, double b)
 {
     double p = a.hi * b;
     double e = fma(a.hi, b, -p);
     e += a.lo * b;
     return dd_fast(p, e);
 }
-HD dd dd_div(dd a, dd b)
+__host__ __device__ inline dd dd_div(dd a, dd b)
 {
     double q1 = a.hi / b.hi;
     dd r = dd_add(a, dd_mul_d(b, -q1));
@@ -152,13 +152,13 @@ HD dd dd_div(dd a, dd b)
     dd q = dd_fast(q1, q2);
     return dd_add(q, dd{q3, 0.});
 }
-HD dd dd_recip_int(int n)  // 1/n to ~2^-106
+__host__ __device__ inline dd dd_recip_int(int n)  // 1/n to ~2^-106
 {
     double h = 1.0 / n;
     double r = fma(-h, (double)n, 1.0);
     return dd_fast(h, r / n);
 }
-HD dd dd_log(double x)  // x > 0, finite
+__host__ __device__ inline dd dd_log(double x)  // x > 0, finite
 {
     int e;
     double m = frexp(x, &e);  // m in [0.5, 1)
@@ -176,7 +176,7 @@ HD dd dd_log(double x)  // x > 0, finite
     const dd ln2 = {6.93147180559945286227e-01, 2.31904681384629955842e-17};
     return dd_add(dd_mul_d(ln2, (double)e), lm);
 }
-HD double dd_exp_round(dd x)  // exp(x) rounded to double; |x.hi| < 700
+__host__ __device__ inline double dd_exp_round(dd x)  // exp(x) rounded to double; |x.hi| < 700
 {
     const dd ln2 = {6.93147180559945286227e-01, 2.31904681384629955842e-17};
     double k = rint(x.hi / ln2.hi);
@@ -188,12 +188,80 @@ HD double dd_exp_round(dd x)  // exp(x) rounded to double; |x.hi| < 700
     for (int q = 0; q < 5; q++) t = dd_mul(t, t);
     return ldexp(t.hi + t.lo, (int)k);
 }
-HD double cr_pow(double x, double y)
+// The method above at full length; out of line, as cr_pow hardly ever needs it.
+__host__ __device__ __noinline__ inline double cr_pow_full(double x, double y)
 {
-    if (!(x > 0.) || !isfinite(x) || !isfinite(y) || y == 0.) return pow(x, y);
     dd l = dd_mul_d(dd_log(x), y);
     if (!(fabs(l.hi) < 700.)) return pow(x, y);
     return dd_exp_round(l);
+}
+
+// c + p for |c| > |p|, c's low part given (1/3 and so on have one)
+__host__ __device__ inline dd dd_step(double chi, double clo, dd p)
+{
+    const double s = chi + p.hi;
+    return {s, ((chi - s) + p.hi) + (clo + p.lo)};
+}
+
+// x^y by the same two series with their small terms in plain FP64: log's from s^12 on
+// (below 2^-34 of the sum, so their rounding is below 2^-87 of it) and exp's from r^5 on
+// (2^-39 and 2^-92), and Horner steps with constant 1/n.  The error stays below 2^-76
+// of the result (|y log x| < 700), so where the sum moved by 2^-75 either way rounds to
+// one value that is the correctly rounded one, and the full method's too; otherwise
+// (one argument in 2^20) false.  A Font-fix zone waits for a chain of these, one after
+// another: a quarter of the full method's length (24 + 13 steps with 74 divisions).
+__host__ __device__ inline bool cr_pow_quick(double x, double y, double &r)
+{
+    int e;
+    double m = frexp(x, &e);
+    if (m < 0.70710678118654752) {
+        m *= 2.;
+        e -= 1;
+    }
+    const double f = m - 1.;  // exact
+    const dd den = dd_two_sum(m, 1.);
+    const double rd = 1. / den.hi, q1 = f * rd;
+    const dd s = dd_fast(q1, (fma(-q1, den.hi, f) - q1 * den.lo) * rd);
+    const dd z = dd_mul(s, s);
+    double T = 1. / 35.;
+#pragma unroll
+    for (int k = 16; k >= 6; k--) T = fma(T, z.hi, 1. / (2 * k + 1));
+    constexpr double third = 1. / 3., fifth = 1. / 5., seventh = 1. / 7., ninth = 1. / 9., eleventh = 1. / 11.;
+    dd t = dd_step(eleventh, -2.523234146875356e-18, dd_mul_d(z, T));
+    t = dd_step(ninth, 6.1679056923619804e-18, dd_mul(z, t));
+    t = dd_step(seventh, 7.93016446160826e-18, dd_mul(z, t));
+    t = dd_step(fifth, -1.1102230246251566e-17, dd_mul(z, t));
+    t = dd_step(third, 1.850371707708594e-17, dd_mul(z, t));
+    t = dd_step(1., 0., dd_mul(z, t));
+    t = dd_mul(s, t);
+    const dd ln2 = {6.93147180559945286227e-01, 2.31904681384629955842e-17};
+    const dd l = dd_mul_d(dd_add(dd_mul_d(ln2, (double)e), dd{2. * t.hi, 2. * t.lo}), y);
+    if (!(fabs(l.hi) < 700.)) return false;
+    const double k = rint(l.hi * 1.4426950408889634);
+    dd d = dd_add(l, dd_mul_d(ln2, -k));
+    d.hi *= 0.03125;
+    d.lo *= 0.03125;
+    double P = 1. / 362880.;
+    P = fma(P, d.hi, 1. / 40320.);
+    P = fma(P, d.hi, 1. / 5040.);
+    P = fma(P, d.hi, 1. / 720.);
+    P = fma(P, d.hi, 1. / 120.);
+    t = dd_step(1. / 24., 2.3129646346357427e-18, dd_mul_d(d, P));
+    t = dd_step(1. / 6., 9.25185853854297e-18, dd_mul(d, t));
+    t = dd_step(0.5, 0., dd_mul(d, t));
+    t = dd_step(1., 0., dd_mul(d, t));
+    t = dd_step(1., 0., dd_mul(d, t));
+#pragma unroll
+    for (int q = 0; q < 5; q++) t = dd_mul(t, t);
+    const double w = t.hi * 0x1p-75, a = t.hi + (t.lo - w), b = t.hi + (t.lo + w);
+    r = ldexp(a, (int)k);
+    return a == b;
+}
+HD double cr_pow(double x, double y)
+{
+    if (!(x > 0.) || !isfinite(x) || !isfinite(y) || y == 0.) return pow(x, y);
+    double r;
+    return cr_pow_quick(x, y, r) ? r : cr_pow_full(x, y);
 }
 HD double dmax(double a, double b) { return (a > b) ? a : b; }
 HD double dmin(double a, double b) { return (a < b) ? a : b; }
@@ -1026,16 +1094,17 @@ HD double W_of_vsq_iso(const U2P &s, double vsq, double &p, double &rho, double 
 }
 
 // utoprim_1dvsq2fix1.c:398-519 with func_1d_gnr (:538-566) and validate_x (:372-384)
-HD int gnr_1dvsq(const U2P &s, double &x)
+// p, rho, u and the returned code's W are those of the last x.
+HD int gnr_1dvsq(const U2P &s, double &x, double &W, double &p, double &rho, double &u)
 {
     const double GAMMA = s.gam, G_ATM = s.gam;
-    double f = 1., df = 1., errx = 1., W = 0., W_old;
+    double f = 1., df = 1., errx = 1., W_old;
     int n_iter = 0, i_extra = 0, doing_extra = 0;
     bool keep = true;
+    W = 0.;
+    double Wv = W_of_vsq_iso(s, x, p, rho, u);
     while (keep) {
-        double p, rho, u;
         double vsq = x;
-        double Wv = W_of_vsq_iso(s, vsq, p, rho, u);
         double Wsq = Wv * Wv;
         double W3 = Wv * Wsq;
         double dWdvsq = ((GAMMA * (2. - G_ATM) * p + (GAMMA - 1.) * rho) / (2. * (GAMMA - 1.) * (1. - vsq) * (1. - vsq)));
@@ -1051,7 +1120,7 @@ HD int gnr_1dvsq(const U2P &s, double &x)
         x = (x < -1.e-10) ? (0.5 * x_old) : x;
         x = fabs(x);
         W_old = W;
-        W = W_of_vsq_iso(s, x, p, rho, u);
+        Wv = W = W_of_vsq_iso(s, x, p, rho, u);  // the next iterate's too
         errx = (W == 0.) ? fabs(W - W_old) : fabs((W - W_old) / W);
         errx += (x == 0.) ? fabs(x - x_old) : fabs((x - x_old) / x);
         if ((fabs(errx) <= NEWT_TOL) && (doing_extra == 0)) doing_extra = 1;
@@ -1084,12 +1153,11 @@ HD int utoprim_1dvsq2fix1(const double *U, const Geom &geom, double gam, double 
     if (utsq < 0. || utsq > UTSQ_TOO_BIG) return 2;
     double gammasq = 1. + utsq;
     double x = 1. - 1. / gammasq;
-    int retval = gnr_1dvsq(s, x);
+    double p, rho0, u, W;
+    int retval = gnr_1dvsq(s, x, W, p, rho0, u);
     if (retval != 0) return retval * 100 + 1;
     double vsq = x;
     if ((vsq >= 1.) || (vsq < 0.)) return 4;
-    double p, rho0, u;
-    double W = W_of_vsq_iso(s, vsq, p, rho0, u);
     double gtmp = sqrt(1. - vsq);
     double gamma = 1. / gtmp;
     if ((rho0 <= 0.) || (u <= 0.)) return 5;
