@@ -104,10 +104,8 @@ __device__ __forceinline__ double &at32(double *base, unsigned zz)
 // mapping each XCD walks one contiguous range of logical blocks, so the stencil
 // neighbours that adjacent logical blocks read come from the same L2.  Grids
 // using it are launched with a multiple of 8 workgroups.
-__device__ __forceinline__ unsigned xcd_block()
-{
-    return (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-}
+__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb) { return (b & 7u) * (nb >> 3) + (b >> 3); }
+__device__ __forceinline__ unsigned xcd_block() { return xcd_block(blockIdx.x, gridDim.x); }
 
 // Zone (i, j, h) of logical index idx over an ni x nj x N3 box at (i0, j0).
 // I_FAST orders the columns with i fastest (for stencils along X1), else j.
@@ -192,10 +190,10 @@ __device__ __forceinline__ void block_counts(const int (&v)[N], unsigned long lo
     }
 }
 
-// Per-block minimum of v stored at out[blockIdx.x]; every thread of the NT-thread
+// Per-block minimum of v stored at out[slot]; every thread of the NT-thread
 // block must call it.
 template <int NT = TPB>
-__device__ __forceinline__ void block_min(double v, double *__restrict__ out)
+__device__ __forceinline__ void block_min(double v, double *__restrict__ out, unsigned slot)
 {
     __shared__ double red[NT / 64];
     const double m = wave_min_dbl(v);
@@ -205,7 +203,7 @@ __device__ __forceinline__ void block_min(double v, double *__restrict__ out)
         double t = red[0];
 #pragma unroll
         for (int q = 1; q < NT / 64; q++) t = (red[q] < t) ? red[q] : t;
-        out[blockIdx.x] = t;
+        out[slot] = t;
     }
 }
 
@@ -214,39 +212,61 @@ struct CntMap {
     int idx[8];
 };
 
-// cnt[map.idx[k]] += sum over blocks b of part[b*map.n + k].  Grid
-// (RED_BLOCKS, map.n): block (x, k) folds every RED_BLOCKS-th partial of
-// counter k and adds its total with one atomic.
-constexpr int RED_BLOCKS = 64;
-__global__ void __launch_bounds__(256) k_sum_partials(const unsigned long long *__restrict__ part, size_t nb,
-                                                      CntMap map, unsigned long long *__restrict__ cnt,
-                                                      const double *__restrict__ halt)
+// The folds of the blocks' partials ride at the end of a launch that comes later anyway
+// (a launch of their own costs about 4.5 us, as much as 30% of a small grid's step).
+
+// cnt[map.idx[k]] += sum over blocks b of part[b*map.n + k], by fold_blocks(nb) blocks
+// of 256 threads per counter: block x folds every so-many-th partial of counter k and
+// adds its total with one atomic.  nb = 0: nothing.
+struct SumArgs {
+    const unsigned long long *part;
+    unsigned nb;
+    CntMap map;
+};
+// The CFL minima of the three directions' flux launches, part[d * stride + block].
+struct MinArgs {
+    const double *part;
+    size_t stride;
+    unsigned nb[3];
+};
+constexpr unsigned RED_BLOCKS = 64;
+__host__ __device__ inline unsigned fold_blocks(unsigned nb)
 {
-    if (halted(halt)) return;
+    const unsigned n = (nb + 255) / 256;
+    return n < RED_BLOCKS ? n : RED_BLOCKS;
+}
+
+__device__ __forceinline__ void fold_counts(const SumArgs &a, unsigned blk, unsigned long long *__restrict__ cnt)
+{
     __shared__ unsigned long long red[256];
-    const int k = blockIdx.y;
+    const unsigned nf = fold_blocks(a.nb), x = blk % nf, k = blk / nf;
     unsigned long long s = 0;
-    for (size_t b = (size_t)blockIdx.x * 256 + threadIdx.x; b < nb; b += (size_t)RED_BLOCKS * 256)
-        s += part[b * map.n + k];
+    for (size_t b = (size_t)x * 256 + threadIdx.x; b < a.nb; b += (size_t)nf * 256) s += a.part[b * a.map.n + k];
     red[threadIdx.x] = s;
     __syncthreads();
     for (int o = 128; o > 0; o >>= 1) {
         if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0 && red[0]) atomicAdd(&cnt[map.idx[k]], red[0]);
+    if (threadIdx.x == 0 && red[0]) atomicAdd(&cnt[a.map.idx[k]], red[0]);
 }
-
-// slot = min(slot, min over blocks of part[b]) where that minimum is < 1e9
-// (the CFL limit of a direction, step_ch.c:477-484); grid RED_BLOCKS.
-__global__ void __launch_bounds__(256) k_min_partials(const double *__restrict__ part, size_t nb,
-                                                      unsigned long long *__restrict__ slot,
+__global__ void __launch_bounds__(256) k_sum_partials(SumArgs a, unsigned long long *__restrict__ cnt,
                                                       const double *__restrict__ halt)
 {
     if (halted(halt)) return;
+    fold_counts(a, blockIdx.x, cnt);
+}
+
+// slot[d] = min(slot[d], min over blocks of direction d's partials) where that minimum
+// is < 1e9 (the CFL limit of a direction, step_ch.c:477-484), by RED_BLOCKS blocks of
+// 256 threads a direction.
+__device__ __forceinline__ void fold_min(const MinArgs &a, unsigned blk, unsigned long long *__restrict__ slot)
+{
     __shared__ double red[256];
+    const unsigned d = blk / RED_BLOCKS, x = blk % RED_BLOCKS;
+    const double *part = a.part + d * a.stride;
     double m = 1.e300;
-    for (size_t b = (size_t)blockIdx.x * 256 + threadIdx.x; b < nb; b += (size_t)RED_BLOCKS * 256)
+    for (size_t b = (size_t)x * 256 + threadIdx.x; b < a.nb[d]; b += (size_t)RED_BLOCKS * 256)
         m = (part[b] < m) ? part[b] : m;
     red[threadIdx.x] = m;
     __syncthreads();
@@ -254,7 +274,13 @@ __global__ void __launch_bounds__(256) k_min_partials(const double *__restrict__
         if (threadIdx.x < o && red[threadIdx.x + o] < red[threadIdx.x]) red[threadIdx.x] = red[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0 && red[0] < 1.e9) atomicMin(slot, (unsigned long long)__double_as_longlong(red[0]));
+    if (threadIdx.x == 0 && red[0] < 1.e9) atomicMin(slot + d, (unsigned long long)__double_as_longlong(red[0]));
+}
+__global__ void __launch_bounds__(256) k_min_partials(MinArgs a, unsigned long long *__restrict__ slot,
+                                                      const double *__restrict__ halt)
+{
+    if (halted(halt)) return;
+    fold_min(a, blockIdx.x, slot);
 }
 
 // ---------------------------------------------------------------------------
@@ -270,18 +296,17 @@ __global__ void __launch_bounds__(256) k_min_partials(const double *__restrict__
 // it from the grid.  ROWS (DIR 3 with N3 dividing TPB): the block holds whole
 // phi rows, so each thread loads only its own zone and forms only its own
 // zone's slopes; the neighbour's values come through LDS.
-template <int DIR, bool UNI, bool TAB, int LIM, bool ROWS = false>
-__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(4, 8)))
-k_flux(DGrid g, const double *__restrict__ pb, double *__restrict__ F, double *__restrict__ dtpart, int fullstep,
-       unsigned long long *__restrict__ cnt)
+template <int DIR, bool UNI, bool TAB, int LIM, bool ROWS>
+__device__ __forceinline__ void flux_faces(const DGrid &g, unsigned blk, unsigned nblk, const double *__restrict__ pb,
+                                           double *__restrict__ F, double *__restrict__ dtpart, int fullstep,
+                                           unsigned long long *__restrict__ cnt)
 {
     static_assert(!ROWS || DIR == 3, "row-local reconstruction is along phi only");
-    if (halted(g)) return;
     const int i0 = (DIR == 1) ? g.is : g.is - 1;
     const int j0 = (DIR == 2) ? g.js : g.js - 1;
     const int ni = g.ie + 1 - i0 + 1;
     const int nj = g.je + 1 - j0 + 1;
-    const unsigned idx = xcd_block() * TPB + threadIdx.x;
+    const unsigned idx = xcd_block(blk, nblk) * TPB + threadIdx.x;
     const unsigned total = (unsigned)ni * nj * g.N3;
     const bool act = idx < total;
     const int lim = (LIM >= 0) ? LIM : g.lim;
@@ -466,8 +491,40 @@ k_flux(DGrid g, const double *__restrict__ pb, double *__restrict__ F, double *_
             if (d < 1.e9) dtij = d;
         }
     }
-    if (fullstep) block_min(dtij, dtpart);
+    if (fullstep) block_min(dtij, dtpart, blk);
     add_counter(cnt, HARM_FATAL, fatal);
+}
+
+// One direction of a wave-uniform grid.
+template <int DIR, bool TAB, int LIM, bool ROWS = false>
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(4, 8)))
+k_flux(DGrid g, const double *__restrict__ pb, double *__restrict__ F, double *__restrict__ dtpart, int fullstep,
+       unsigned long long *__restrict__ cnt)
+{
+    if (halted(g)) return;
+    flux_faces<DIR, true, TAB, LIM, ROWS>(g, blockIdx.x, gridDim.x, pb, F, dtpart, fullstep, cnt);
+}
+
+// Every direction of the other grids in one launch, blocks [nb1 + nb2, ..) the third
+// (none in 2D): most of these grids are too small for one direction to fill the CUs.
+// Three wavefronts a SIMD, as the per-lane metric spills at four.  With the EMFs formed in
+// the update and the folds riding on other launches, a 128x128 step went from 26 launches
+// to 16 and from 225 to 168 us.
+template <bool TAB, int LIM>
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(3, 8)))
+k_flux_all(DGrid g, const double *__restrict__ pb, double *__restrict__ F1, double *__restrict__ F2,
+           double *__restrict__ F3, double *__restrict__ dtpart, size_t dtstride, unsigned nb1, unsigned nb2,
+           int fullstep, unsigned long long *__restrict__ cnt)
+{
+    if (halted(g)) return;
+    const unsigned b = blockIdx.x;
+    if (b < nb1)
+        flux_faces<1, false, TAB, LIM, false>(g, b, nb1, pb, F1, dtpart, fullstep, cnt);
+    else if (b < nb1 + nb2)
+        flux_faces<2, false, TAB, LIM, false>(g, b - nb1, nb2, pb, F2, dtpart + dtstride, fullstep, cnt);
+    else
+        flux_faces<3, false, TAB, LIM, false>(g, b - nb1 - nb2, gridDim.x - nb1 - nb2, pb, F3, dtpart + 2 * dtstride,
+                                              fullstep, cnt);
 }
 
 // The X1 / X2 fluxes of the wave-uniform path with the reconstruction shared
@@ -613,7 +670,7 @@ k_flux_strip(DGrid g, const double *__restrict__ pb, double *__restrict__ F, dou
         for (int k = 0; k < NPR; k++) p_r[k] = B[w + 4][k][lane];
         strip_face<DIR, TAB>(g, F, p_l, p_r, f0 + w, o, h, fullstep, dtij, fatal);
     }
-    if (fullstep) block_min<STRIP_TPB>(dtij, dtpart);
+    if (fullstep) block_min<STRIP_TPB>(dtij, dtpart, blockIdx.x);
     add_counter(cnt, HARM_FATAL, fatal);
 }
 
@@ -723,7 +780,7 @@ k_flux_strip_ppm(DGrid g, const double *__restrict__ pb, double *__restrict__ F,
     double dtij = 1.e300;
     int fatal = 0;
     if (blk_act && f0 + w <= fe) strip_face<DIR, TAB>(g, F, p_l, p_r, f0 + w, o, h, fullstep, dtij, fatal);
-    if (fullstep) block_min<STRIP_TPB>(dtij, dtpart);
+    if (fullstep) block_min<STRIP_TPB>(dtij, dtpart, blockIdx.x);
     add_counter(cnt, HARM_FATAL, fatal);
 }
 
@@ -846,6 +903,7 @@ __device__ __forceinline__ void flux_div(const DGrid &g, const DivArgs &a, int i
 // operations in the same order.  The twelve corner EMFs it needs are formed
 // here from the face B-fluxes with k_emf's expressions (step_ch.c:773-781), so
 // the fused update needs no EMF pass.
+template <bool UNI>
 __device__ __forceinline__ void flux_div32(const DGrid &g, const DivArgs &a, int i, int j, int h, double *d)
 {
     const unsigned sI = (unsigned)g.SN2 * (unsigned)g.N3, sJ = (unsigned)g.N3;
@@ -854,6 +912,33 @@ __device__ __forceinline__ void flux_div32(const DGrid &g, const DivArgs &a, int
     const unsigned zhm = z - (unsigned)h + (unsigned)((h + g.N3 - 1) % g.N3);
     const unsigned zi1 = z + sI, zj1 = z + sJ, zi1h1 = zh1 + sI, zj1h1 = zh1 + sJ, zi1j1 = zi1 + sJ;
     const size_t nz = g.nz;
+    if (!UNI && g.N3 <= 2) {
+        // flux_ct of two dimensions (step_ch.c:514-554): one EMF, B3's fluxes as they are
+        const double *F1B2 = a.F1 + B2 * nz, *F2B1 = a.F2 + B1 * nz;
+        auto e3 = [&](unsigned q) {
+            return 0.25 * (at32(F1B2, q) + at32(F1B2, q - sJ) - at32(F2B1, q) - at32(F2B1, q - sI));
+        };
+        const double e3z = e3(z), e3j = e3(zj1), e3i = e3(zi1), e3ij = e3(zi1j1);
+#pragma unroll
+        for (int k = 0; k < NPR; k++) {
+            double a1 = 0., b1 = 0., a2 = 0., b2 = 0.;
+            if (k == B1) {
+                a2 = -0.5 * (e3z + e3i);
+                b2 = -0.5 * (e3j + e3ij);
+            } else if (k == B2) {
+                a1 = 0.5 * (e3z + e3j);
+                b1 = 0.5 * (e3i + e3ij);
+            } else {
+                const double *F1 = a.F1 + k * nz, *F2 = a.F2 + k * nz;
+                a1 = at32(F1, z);
+                b1 = at32(F1, zi1);
+                a2 = at32(F2, z);
+                b2 = at32(F2, zj1);
+            }
+            d[k] = -div_r(b1 - a1, g.dx1, g.rdx1) - div_r(b2 - a2, g.dx2, g.rdx2);
+        }
+        return;
+    }
     const double *F1B2 = a.F1 + B2 * nz, *F1B3 = a.F1 + B3 * nz, *F2B1 = a.F2 + B1 * nz, *F2B3 = a.F2 + B3 * nz,
                  *F3B1 = a.F3 + B1 * nz, *F3B2 = a.F3 + B2 * nz;
     // e1 = ((F2[B3] + F2[B3](h-1)) - (F3[B2] + F3[B2](j-1))) / 4 at (j, h), (j, h+1), (j+1, h), (j+1, h+1)
@@ -1032,7 +1117,7 @@ __device__ __forceinline__ unsigned upd_tiled_row(unsigned b, unsigned G, unsign
 // (its seed-list store would otherwise take it past 128 VGPRs); every other
 // instance keeps the compiler's choice.
 template <bool UNI, int MODE, bool TAB, bool FUSED>
-__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu((UNI && MODE == UPD_GATED) ? 4 : 1, 8)))
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu((UNI && MODE == UPD_GATED) ? 4 : MODE == UPD_LEARNED ? 3 : 1, 8)))
 k_update(DGrid g, const double *__restrict__ pi, const double *__restrict__ pb, double *__restrict__ pf,
          int8_t *__restrict__ pflag, const double *__restrict__ S, DivArgs dv, const double *__restrict__ tstate,
          double dtfac, int pi_is_pb, FontList fl, unsigned long long *__restrict__ cpart, UpdateExtra ex)
@@ -1041,7 +1126,7 @@ k_update(DGrid g, const double *__restrict__ pi, const double *__restrict__ pb, 
     const int ni = g.ie - g.is + 1, nj = g.je - g.js + 1;
     const size_t na = (size_t)ni * nj * g.N3;
     size_t idx = (size_t)blockIdx.x * TPB + threadIdx.x;
-    if constexpr (FUSED) {
+    if constexpr (FUSED && UNI) {
         // One block is one phi row (N3 == TPB): the rows go to the XCDs as
         // contiguous ranges of UPD_TI x UPD_TJ (i, j) tiles, j fastest, so the
         // rows that share face fluxes run on one XCD at about the same time
@@ -1102,7 +1187,7 @@ k_update(DGrid g, const double *__restrict__ pi, const double *__restrict__ pb, 
         }
         if constexpr (FUSED) {
             double d[NPR];
-            flux_div32(g, dv, i, j, h, d);
+            flux_div32<UNI>(g, dv, i, j, h, d);
 #pragma unroll
             for (int k = 0; k < NPR; k++) U[k] += Dt * (d[k] + dU[k]);
         } else {
@@ -1144,7 +1229,8 @@ k_update(DGrid g, const double *__restrict__ pi, const double *__restrict__ pb, 
 #pragma unroll
             for (int k = 0; k < MLP_NIN; k++) x[k] = 0.f;
         float y0, y1;
-        mlp_forward_wave(ex.mlp, x, y0, y1);
+        __shared__ MlpLds lds;
+        mlp_forward_wave<true>(mlp_stage(ex.mlp, lds), x, y0, y1);
         if (active) {
             double W0 = 0., vsq0 = 0.;
             if (ok) mlp_unstandardize(ex.mlp, y0, y1, mlp_wref(f), W0, vsq0);
@@ -1409,7 +1495,7 @@ __global__ void __launch_bounds__(TPB) k_flux_ceos(DGrid g, const double *__rest
             if (d < 1.e9 && d < dtij) dtij = d;
         }
     });
-    if (fullstep) block_min(dtij, dtpart);
+    if (fullstep) block_min(dtij, dtpart, blockIdx.x);
     add_counter(cnt, HARM_FATAL, fatal);
 }
 
@@ -1711,9 +1797,14 @@ __device__ __forceinline__ size_t bound_nthreads(const DGrid &g)
 
 __global__ void __launch_bounds__(TPB) k_bound(DGrid g, double *__restrict__ p, int8_t *__restrict__ pflag,
                                                int *__restrict__ font_count, int *__restrict__ seed_count,
-                                               unsigned long long *__restrict__ cnt)
+                                               unsigned nbound, SumArgs sum, unsigned long long *__restrict__ cnt)
 {
+    static_assert(TPB == 256, "fold_counts takes blocks of 256 threads");
     if (halted(g)) return;
+    if (blockIdx.x >= nbound) {  // the zone update's counters
+        fold_counts(sum, blockIdx.x - nbound, cnt);
+        return;
+    }
     const size_t idx = (size_t)blockIdx.x * TPB + threadIdx.x;
     if (idx == 0 && font_count) *font_count = 0;
     if (idx == 0 && seed_count) *seed_count = 0;
@@ -1834,6 +1925,7 @@ __device__ __forceinline__ void repair_zone(const DGrid &g, double *p, int8_t *p
 // of a plane reads and writes that plane only (fixup_utoprim's stencil is
 // i+-1, j+-1 at fixed h), so the planes are repaired independently and each in
 // the reference's (i, j) order with no list, sort or capacity.
+constexpr int SCAN_ZONES = 32;
 __global__ void __launch_bounds__(TPB) k_fixutoprim_scan(DGrid g, double *__restrict__ p,
                                                          const int8_t *__restrict__ fin, int8_t *__restrict__ fout,
                                                          unsigned long long *__restrict__ bits,
@@ -1841,39 +1933,50 @@ __global__ void __launch_bounds__(TPB) k_fixutoprim_scan(DGrid g, double *__rest
                                                          unsigned long long *__restrict__ cnt)
 {
     if (halted(g)) return;
-    // 8 zones per thread: the common all-good octet is one 8-byte load and store.
-    const size_t z0 = ((size_t)blockIdx.x * TPB + threadIdx.x) * 8;
+    // 32 zones per thread: the common all-good octet is an 8-byte load and store, and a
+    // wavefront whose lanes met no bad zone leaves the counters alone (8 zones a thread
+    // with every counter's wave sum: 30 us on 288x256x256, now 10 us).
+    const size_t t0 = ((size_t)blockIdx.x * TPB + threadIdx.x) * SCAN_ZONES;
     int c_rep = 0, c_nost = 0, c_flr = 0, c_cap = 0, c_gam = 0, fatal = 0;
-    if (z0 < g.nz) {
-        const bool full = z0 + 8 <= g.nz;
-        const unsigned long long f8 = full ? *reinterpret_cast<const unsigned long long *>(fin + z0) : 1ull;
-        if (full && f8 == 0ull) {
+    bool bad = false;
+    unsigned long long f8[SCAN_ZONES / 8];
+#pragma unroll
+    for (int o = 0; o < SCAN_ZONES / 8; o++) {
+        const size_t z0 = t0 + 8 * o;
+        f8[o] = z0 + 8 <= g.nz ? *reinterpret_cast<const unsigned long long *>(fin + z0) : 1ull;
+    }
+    for (int o = 0; o < SCAN_ZONES / 8; o++) {
+        const size_t z0 = t0 + 8 * o;
+        if (z0 >= g.nz) break;
+        if (f8[o] == 0ull) {
             *reinterpret_cast<unsigned long long *>(fout + z0) = 0x0101010101010101ull;
-        } else {
-            for (int q = 0; q < 8; q++) {
-                const size_t idx = z0 + q;
-                if (idx >= g.nz) break;
-                const unsigned col = (unsigned)idx / (unsigned)g.N3;
-                const int h = (int)((unsigned)idx - col * (unsigned)g.N3);
-                const unsigned ci = col / (unsigned)g.SN2;
-                const int j = (int)(col - ci * (unsigned)g.SN2), i = (int)ci;
-                const int8_t f = fin[idx];
-                fout[idx] = (int8_t)(!f);
-                if (f != 0 && i >= g.is && i <= g.ie && j >= g.js && j <= g.je) {
-                    bool isolated = true;
-                    for (int di = -1; di <= 1; di++)
-                        for (int dj = -1; dj <= 1; dj++)
-                            if ((di || dj) && fin[zidx(g, i + di, j + dj, h)] != 0) isolated = false;
-                    if (isolated) {
-                        repair_zone(g, p, fout, i, j, h, false, fin, c_rep, c_nost, c_flr, c_cap, c_gam, fatal);
-                    } else {
-                        atomicOr(&bits[(size_t)h * nwords + (col >> 6)], 1ull << (col & 63u));
-                        atomicAdd(&pcount[h], 1);
-                    }
+            continue;
+        }
+        bad = true;
+        for (int q = 0; q < 8; q++) {
+            const size_t idx = z0 + q;
+            if (idx >= g.nz) break;
+            const unsigned col = (unsigned)idx / (unsigned)g.N3;
+            const int h = (int)((unsigned)idx - col * (unsigned)g.N3);
+            const unsigned ci = col / (unsigned)g.SN2;
+            const int j = (int)(col - ci * (unsigned)g.SN2), i = (int)ci;
+            const int8_t f = fin[idx];
+            fout[idx] = (int8_t)(!f);
+            if (f != 0 && i >= g.is && i <= g.ie && j >= g.js && j <= g.je) {
+                bool isolated = true;
+                for (int di = -1; di <= 1; di++)
+                    for (int dj = -1; dj <= 1; dj++)
+                        if ((di || dj) && fin[zidx(g, i + di, j + dj, h)] != 0) isolated = false;
+                if (isolated) {
+                    repair_zone(g, p, fout, i, j, h, false, fin, c_rep, c_nost, c_flr, c_cap, c_gam, fatal);
+                } else {
+                    atomicOr(&bits[(size_t)h * nwords + (col >> 6)], 1ull << (col & 63u));
+                    atomicAdd(&pcount[h], 1);
                 }
             }
         }
     }
+    if (!__any(bad)) return;
     add_counter(cnt, HARM_FIXUP_REPAIRS, c_rep);
     add_counter(cnt, HARM_FIXUP_NOSTENCIL, c_nost);
     add_counter(cnt, HARM_FLOOR_ZONES, c_flr);
@@ -1936,11 +2039,10 @@ __global__ void __launch_bounds__(64) k_fixutoprim_serial(DGrid g, double *__res
 // diag_mass (diag.c:477-580, MDOTTYPE=NEU_AGA_GHOST1) partial sums of the mass
 // flux through the first ghost columns, one block per phi plane.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(TPB) k_mdot_partials(DGrid g, const double *__restrict__ p, double *__restrict__ part)
+__device__ __forceinline__ void mdot_plane(const DGrid &g, int h, const double *__restrict__ p,
+                                           double *__restrict__ part)
 {
-    if (halted(g)) return;
     __shared__ double s_in[TPB], s_out[TPB];
-    const int h = blockIdx.x;
     double a_in = 0., a_out = 0.;
     int fatal = 0;
     for (int j = g.js + threadIdx.x; j <= g.je; j += TPB) {
@@ -1972,6 +2074,11 @@ __global__ void __launch_bounds__(TPB) k_mdot_partials(DGrid g, const double *__
         part[2 * h + 1] = s_out[0];
     }
 }
+__global__ void __launch_bounds__(TPB) k_mdot_partials(DGrid g, const double *__restrict__ p, double *__restrict__ part)
+{
+    if (halted(g)) return;
+    mdot_plane(g, blockIdx.x, p, part);
+}
 
 // Start of a harm_step batch: tstate[5] = the fail() event count so far, so
 // that k_stepend sees the events of its own step.  One thread.
@@ -1988,28 +2095,22 @@ __global__ void k_step_begin(double *tstate, const unsigned long long *cnt)
 // step in which such an event happened completes, t is not advanced, and the
 // batch stops.  A dt below 1e-9 exits after diag_mass and before t += dt
 // (step_ch.c:119-129), which is where this kernel stops too.
-__global__ void k_stepend(DGrid g, double *tstate, unsigned long long *ndt_slot, const double *part, int nparts,
-                          const unsigned long long *cnt)
+__device__ __forceinline__ void step_end(const DGrid &g, double *tstate, unsigned long long *ndt_slot,
+                                         double mdot_in, double mdot_out, const unsigned long long *cnt)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    if (halted(g)) return;
     const double nfatal = (double)cnt[HARM_FATAL];
     if (nfatal != tstate[5]) {
         tstate[5] = nfatal;
         tstate[4] = 14.;
         return;
     }
-    double mdot_in = 0., mdot_out = 0.;
-    for (int q = 0; q < nparts; q++) {
-        mdot_in += part[2 * q];
-        mdot_out += part[2 * q + 1];
-    }
     const double dt = tstate[1];
     tstate[2] += mdot_in * dt;
     tstate[3] += mdot_out * dt;
-    const double ndt1 = __longlong_as_double((long long)ndt_slot[0]);
-    const double ndt2 = __longlong_as_double((long long)ndt_slot[1]);
-    const double ndt3 = __longlong_as_double((long long)ndt_slot[2]);
+    auto ndt_of = [&](int d) {
+        return __longlong_as_double((long long)__hip_atomic_load(ndt_slot + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    };
+    const double ndt1 = ndt_of(0), ndt2 = ndt_of(1), ndt3 = ndt_of(2);
     double ndt;
     if (g.N3 > 2)
         ndt = g.defcon * 1. / (1. / ndt1 + 1. / ndt2 + 1. / ndt3);
@@ -2029,6 +2130,50 @@ __global__ void k_stepend(DGrid g, double *tstate, unsigned long long *ndt_slot,
     ndt_slot[0] = big;
     ndt_slot[1] = big;
     ndt_slot[2] = big;
+}
+
+// The end of a step: blocks [0, N3) the mass fluxes of a phi plane each, the others the
+// CFL minima; the last block to finish adds the planes in order and closes the step.
+// done: the count of finished blocks, 0 between launches.
+__global__ void __launch_bounds__(TPB) k_stepend(DGrid g, const double *__restrict__ p, double *part, MinArgs mins,
+                                                 unsigned *done, double *tstate, unsigned long long *ndt_slot,
+                                                 const unsigned long long *cnt)
+{
+    if (halted(g)) return;
+    if (blockIdx.x < (unsigned)g.N3)
+        mdot_plane(g, blockIdx.x, p, part);
+    else
+        fold_min(mins, blockIdx.x - g.N3, ndt_slot);
+    // thread 0 wrote this block's results: its release makes them visible to the block
+    // whose acquire finds every other one done
+    __shared__ bool last;
+    if (threadIdx.x == 0)
+        last = __hip_atomic_fetch_add(done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    __syncthreads();
+    if (!last) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    __shared__ double in[TPB], out[TPB];
+    double mdot_in = 0., mdot_out = 0.;
+    for (int q0 = 0; q0 < g.N3; q0 += TPB) {
+        const int q = q0 + (int)threadIdx.x;
+        if (q < g.N3) {
+            in[threadIdx.x] = part[2 * q];
+            out[threadIdx.x] = part[2 * q + 1];
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const int n = min(TPB, g.N3 - q0);
+#pragma unroll 16
+            for (int r = 0; r < n; r++) {
+                mdot_in += in[r];
+                mdot_out += out[r];
+            }
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x != 0) return;
+    *done = 0;
+    step_end(g, tstate, ndt_slot, mdot_in, mdot_out, cnt);
 }
 
 // ---------------------------------------------------------------------------
@@ -2706,19 +2851,25 @@ __global__ void __launch_bounds__(TPB) k_dump_cols(DGrid g, const double *__rest
 }
 
 // Batched Noble 2D inversion over SoA arrays (utoprim_2d.c:126, plus the Font fix).
-// Batched inversion; LEARNED seeds Newton from the network (all lanes take
-// part in the wave-level forward pass, so there is no early exit).
-template <bool LEARNED>
-__global__ void __launch_bounds__(TPB) k_c2p_batch(const double *__restrict__ U, const double *__restrict__ gcov,
+// GUESS 1 seeds Newton from the network, 2 gates that by the plain start's first step
+// (all lanes take part in the wave-level forward pass, so there is no early exit).
+// FONT: the Font fix where the inversion fails; its solvers would double the
+// registers of the others (2 and 1 wavefronts a SIMD), so they have kernels without it.
+template <int GUESS, bool FONT>
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(FONT ? 1 : GUESS ? 3 : 4, 8))) k_c2p_batch(const double *__restrict__ U, const double *__restrict__ gcov,
                                                    const double *__restrict__ gcon, const double *__restrict__ gdet,
                                                    double *__restrict__ prim, int8_t *__restrict__ ret,
                                                    uint8_t *__restrict__ iters, uint8_t *__restrict__ kconv, size_t n,
-                                                   double gam, int font_fix, double K, int *__restrict__ ret_full,
-                                                   MlpDev mlp, double gate_tau)
+                                                   double gam, double K, int *__restrict__ ret_full, MlpDev mlp,
+                                                   double gate_tau)
 {
     const size_t z = (size_t)blockIdx.x * TPB + threadIdx.x;
     const bool act = z < n;
-    if (!LEARNED && !act) return;
+    if (!GUESS && !act) return;
+    if constexpr (GUESS != 0) {
+        __shared__ MlpLds lds;
+        mlp = mlp_stage(mlp, lds);
+    }
     Geom geom;
     double Uz[NPR], pr[NPR];
     if (act) {
@@ -2736,7 +2887,7 @@ __global__ void __launch_bounds__(TPB) k_c2p_batch(const double *__restrict__ U,
         }
     }
     int niter = 0, kc = 0, r = 0;
-    if (LEARNED && gate_tau > 0.) {
+    if constexpr (GUESS == 2) {
         // gated: the network only for the waves with a zone whose plain start is poor
         Gnr2 st;
         bool need = false;
@@ -2753,13 +2904,13 @@ __global__ void __launch_bounds__(TPB) k_c2p_batch(const double *__restrict__ U,
 #pragma unroll
                 for (int k = 0; k < MLP_NIN; k++) x[k] = 0.f;
             float y0, y1;
-            mlp_forward_wave(mlp, x, y0, y1);
+            mlp_forward_wave<true>(mlp, x, y0, y1);
             if (ok) mlp_unstandardize(mlp, y0, y1, mlp_wref(f), W0, vsq0);
         }
         if (!act) return;
         int seeded;
         r = u2p_gate_finish(Uz, geom, gam, pr, ph1, st, need, W0, vsq0, mlp.vsq_from_W, niter, kc, seeded);
-    } else if constexpr (LEARNED) {
+    } else if constexpr (GUESS == 1) {
         double f[MLP_NIN];
         const bool ok = act && mlp_features_U(Uz, geom, f);
         float x[MLP_NIN];
@@ -2769,7 +2920,7 @@ __global__ void __launch_bounds__(TPB) k_c2p_batch(const double *__restrict__ U,
 #pragma unroll
             for (int k = 0; k < MLP_NIN; k++) x[k] = 0.f;
         float y0, y1;
-        mlp_forward_wave(mlp, x, y0, y1);
+        mlp_forward_wave<true>(mlp, x, y0, y1);
         if (!act) return;
         double W0 = 0., vsq0 = 0.;
         if (ok) mlp_unstandardize(mlp, y0, y1, mlp_wref(f), W0, vsq0);
@@ -2779,9 +2930,11 @@ __global__ void __launch_bounds__(TPB) k_c2p_batch(const double *__restrict__ U,
         r = utoprim_2d(Uz, geom, gam, pr, niter, kc);
     }
     int8_t flag = (int8_t)r;
-    if (flag && font_fix) {
-        flag = (int8_t)utoprim_1dvsq2fix1(Uz, geom, gam, K, pr);
-        if (flag) flag = (int8_t)utoprim_1dfix1(Uz, geom, gam, K, pr);
+    if constexpr (FONT) {
+        if (flag) {
+            flag = (int8_t)utoprim_1dvsq2fix1(Uz, geom, gam, K, pr);
+            if (flag) flag = (int8_t)utoprim_1dfix1(Uz, geom, gam, K, pr);
+        }
     }
 #pragma unroll
     for (int k = 0; k < NPR; k++) prim[(size_t)k * n + z] = pr[k];
@@ -3082,7 +3235,11 @@ struct harm_ctx {
     double *d_geom[5], *d_conn, *d_floors, *d_katm, *d_cblk, *d_fblk;
     double *tstate;                   // t, dt, mass_in, mass_out, err
     unsigned long long *ndt_slot;     // 3
-    double *dtpart;                   // per-block CFL minima of one flux launch
+    double *dtpart;                   // per-block CFL minima of the flux launches, dtstride a direction
+    size_t dtstride;
+    unsigned dt_nb[3];                // blocks of the last full-step flux launch of each direction
+    unsigned sum_nb;                  // blocks of the last zone update whose counters are not folded yet
+    unsigned *step_done;              // k_stepend's finished blocks
     unsigned long long *cpart;        // per-block counter totals of one update launch
     unsigned long long *cnt;          // HARM_NCOUNTERS
     double *part;                     // reduction partials
@@ -3186,11 +3343,11 @@ int ev_collect(harm_ctx *c)
         if (rc_) return rc_;                                   \
     } while (0)
 
-template <int DIR, bool UNI, bool TAB, int LIM = -1, bool ROWS = false>
+template <int DIR, bool TAB, int LIM = -1, bool ROWS = false>
 void flux_kernel(harm_ctx *c, dim3 grid, const double *pb, double *F, int fullstep)
 {
-    hipLaunchKernelGGL((k_flux<DIR, UNI, TAB, LIM, ROWS>), grid, dim3(TPB), 0, c->stream, c->g, pb, F, c->dtpart,
-                       fullstep, c->cnt);
+    hipLaunchKernelGGL((k_flux<DIR, TAB, LIM, ROWS>), grid, dim3(TPB), 0, c->stream, c->g, pb, F,
+                       c->dtpart + (DIR - 1) * c->dtstride, fullstep, c->cnt);
 }
 
 template <int DIR>
@@ -3201,7 +3358,7 @@ void flux_kernel_any(harm_ctx *c, dim3 &grid, const double *pb, double *F, int f
         // wave-uniform grids share the zones' slopes and parabolas through LDS
         // (strips along X1 / X2, whole rows along phi where they divide the
         // block); otherwise six zones per face, one face per thread
-        if (c->uniform && DIR != 3) {
+        if (DIR != 3) {
             const DGrid &g = c->g;
             const size_t nf = (DIR == 1) ? (size_t)(g.ie + 2 - g.is) : (size_t)(g.je + 2 - g.js);
             const size_t no = (DIR == 1) ? (size_t)(g.je + 3 - g.js) : (size_t)(g.ie + 3 - g.is);
@@ -3210,27 +3367,22 @@ void flux_kernel_any(harm_ctx *c, dim3 &grid, const double *pb, double *F, int f
             constexpr int D = (DIR == 3) ? 1 : DIR;
             if (tab)
                 hipLaunchKernelGGL((k_flux_strip_ppm<D, true>), grid, dim3(STRIP_TPB), 0, c->stream, c->g, pb, F,
-                                   c->dtpart, fullstep, c->cnt);
+                                   c->dtpart + (DIR - 1) * c->dtstride, fullstep, c->cnt);
             else
                 hipLaunchKernelGGL((k_flux_strip_ppm<D, false>), grid, dim3(STRIP_TPB), 0, c->stream, c->g, pb, F,
-                                   c->dtpart, fullstep, c->cnt);
-        } else if (c->uniform && DIR == 3 && TPB % c->g.N3 == 0) {
+                                   c->dtpart + (DIR - 1) * c->dtstride, fullstep, c->cnt);
+        } else if (TPB % c->g.N3 == 0) {
             if (tab)
-                flux_kernel<DIR, true, true, LIM_PPM, DIR == 3>(c, grid, pb, F, fullstep);
+                flux_kernel<DIR, true, LIM_PPM, DIR == 3>(c, grid, pb, F, fullstep);
             else
-                flux_kernel<DIR, true, false, LIM_PPM, DIR == 3>(c, grid, pb, F, fullstep);
-        } else if (c->uniform) {
-            if (tab)
-                flux_kernel<DIR, true, true, LIM_PPM>(c, grid, pb, F, fullstep);
-            else
-                flux_kernel<DIR, true, false, LIM_PPM>(c, grid, pb, F, fullstep);
+                flux_kernel<DIR, false, LIM_PPM, DIR == 3>(c, grid, pb, F, fullstep);
         } else {
             if (tab)
-                flux_kernel<DIR, false, true, LIM_PPM>(c, grid, pb, F, fullstep);
+                flux_kernel<DIR, true, LIM_PPM>(c, grid, pb, F, fullstep);
             else
-                flux_kernel<DIR, false, false, LIM_PPM>(c, grid, pb, F, fullstep);
+                flux_kernel<DIR, false, LIM_PPM>(c, grid, pb, F, fullstep);
         }
-    } else if (c->uniform && DIR != 3) {
+    } else if (DIR != 3) {
         // strips of STRIP faces along DIR x one other index x 64 phi zones
         const DGrid &g = c->g;
         const size_t nf = (DIR == 1) ? (size_t)(g.ie + 2 - g.is) : (size_t)(g.je + 2 - g.js);
@@ -3238,36 +3390,55 @@ void flux_kernel_any(harm_ctx *c, dim3 &grid, const double *pb, double *F, int f
         const size_t nb = (nf + STRIP - 1) / STRIP * no * (size_t)(g.N3 / 64);
         grid = dim3((unsigned)((nb + 7) / 8 * 8));
         constexpr int D = (DIR == 3) ? 1 : DIR;
-        if (tab)
+        if (tab && mc)
+            hipLaunchKernelGGL((k_flux_strip<D, true, LIM_MC>), grid, dim3(STRIP_TPB), 0, c->stream, c->g, pb, F,
+                               c->dtpart + (DIR - 1) * c->dtstride, fullstep, c->cnt);
+        else if (tab)
             hipLaunchKernelGGL((k_flux_strip<D, true, -1>), grid, dim3(STRIP_TPB), 0, c->stream, c->g, pb, F,
-                               c->dtpart, fullstep, c->cnt);
+                               c->dtpart + (DIR - 1) * c->dtstride, fullstep, c->cnt);
         else if (mc)
             hipLaunchKernelGGL((k_flux_strip<D, false, 0>), grid, dim3(STRIP_TPB), 0, c->stream, c->g, pb, F,
-                               c->dtpart, fullstep, c->cnt);
+                               c->dtpart + (DIR - 1) * c->dtstride, fullstep, c->cnt);
         else
             hipLaunchKernelGGL((k_flux_strip<D, false, -1>), grid, dim3(STRIP_TPB), 0, c->stream, c->g, pb, F,
-                               c->dtpart, fullstep, c->cnt);
-    } else if (c->uniform && TPB % c->g.N3 == 0) {
+                               c->dtpart + (DIR - 1) * c->dtstride, fullstep, c->cnt);
+    } else if (TPB % c->g.N3 == 0) {
         // DIR 3, whole phi rows per block
-        if (tab)
-            flux_kernel<DIR, true, true, -1, DIR == 3>(c, grid, pb, F, fullstep);
+        if (tab && mc)
+            flux_kernel<DIR, true, LIM_MC, DIR == 3>(c, grid, pb, F, fullstep);
+        else if (tab)
+            flux_kernel<DIR, true, -1, DIR == 3>(c, grid, pb, F, fullstep);
         else if (mc)
-            flux_kernel<DIR, true, false, 0, DIR == 3>(c, grid, pb, F, fullstep);
+            flux_kernel<DIR, false, 0, DIR == 3>(c, grid, pb, F, fullstep);
         else
-            flux_kernel<DIR, true, false, -1, DIR == 3>(c, grid, pb, F, fullstep);
-    } else if (c->uniform) {
-        if (tab)
-            flux_kernel<DIR, true, true>(c, grid, pb, F, fullstep);
-        else if (mc)
-            flux_kernel<DIR, true, false, 0>(c, grid, pb, F, fullstep);
-        else
-            flux_kernel<DIR, true, false>(c, grid, pb, F, fullstep);
+            flux_kernel<DIR, false, -1, DIR == 3>(c, grid, pb, F, fullstep);
     } else {
         if (tab)
-            flux_kernel<DIR, false, true>(c, grid, pb, F, fullstep);
+            flux_kernel<DIR, true>(c, grid, pb, F, fullstep);
+        else if (mc)
+            flux_kernel<DIR, false, 0>(c, grid, pb, F, fullstep);
         else
-            flux_kernel<DIR, false, false>(c, grid, pb, F, fullstep);
+            flux_kernel<DIR, false>(c, grid, pb, F, fullstep);
     }
+}
+
+// Every direction of a grid that is not wave-uniform (k_flux_all).
+int flux_launch_all(harm_ctx *c, const double *pb, int fullstep)
+{
+    const DGrid &g = c->g;
+    unsigned nb[3] = {0, 0, 0};
+    for (int d = 0; d < (g.N3 > 2 ? 3 : 2); d++) {
+        const size_t ni = (size_t)(g.ie + 2 - (d == 0 ? g.is : g.is - 1)), nj = (size_t)(g.je + 2 - (d == 1 ? g.js : g.js - 1));
+        nb[d] = nblocks8(ni * nj * g.N3);
+        if (fullstep) c->dt_nb[d] = nb[d];
+    }
+    const bool tab = c->eos_kind == 1, ppm = g.lim == LIM_PPM;
+    const bool mc = g.lim == LIM_MC;
+    auto *k = tab ? (ppm ? k_flux_all<true, LIM_PPM> : mc ? k_flux_all<true, LIM_MC> : k_flux_all<true, -1>)
+                  : (ppm ? k_flux_all<false, LIM_PPM> : mc ? k_flux_all<false, LIM_MC> : k_flux_all<false, -1>);
+    LAUNCH(HARM_K_FLUX1, hipLaunchKernelGGL(k, dim3(nb[0] + nb[1] + nb[2]), dim3(TPB), 0, c->stream, g, pb, c->F1, c->F2,
+                                            c->F3, c->dtpart, c->dtstride, nb[0], nb[1], fullstep, c->cnt));
+    return 0;
 }
 
 int flux_launch(harm_ctx *c, int dir, const double *pb, double *F, int fullstep)
@@ -3289,8 +3460,8 @@ int flux_launch(harm_ctx *c, int dir, const double *pb, double *F, int fullstep)
                                                       c->lastT, pb, c->ceos_fe, chain, c->ceos_solves);            \
                else hipLaunchKernelGGL((k_face_eos<D_, false>), ge, dim3(TPB), 0, c->stream, g, c->ceos, c->lastT, pb, \
                                        c->ceos_fe, chain, c->ceos_solves);                                         \
-           hipLaunchKernelGGL(k_flux_ceos<D_>, grid, dim3(TPB), 0, c->stream, g, c->ceos_fe, pb, F, c->dtpart,     \
-                              fullstep, c->cnt))
+           hipLaunchKernelGGL(k_flux_ceos<D_>, grid, dim3(TPB), 0, c->stream, g, c->ceos_fe, pb, F,                \
+                              c->dtpart + (D_ - 1) * c->dtstride, fullstep, c->cnt))
         if (dir == 1)
             CEOS_FLUX(1, HARM_K_FLUX1);
         else if (dir == 2)
@@ -3305,11 +3476,30 @@ int flux_launch(harm_ctx *c, int dir, const double *pb, double *F, int fullstep)
         LAUNCH(HARM_K_FLUX2, flux_kernel_any<2>(c, grid, pb, F, fullstep));
     else
         LAUNCH(HARM_K_FLUX3, flux_kernel_any<3>(c, grid, pb, F, fullstep));
-    if (fullstep) {
-        hipLaunchKernelGGL(k_min_partials, dim3(RED_BLOCKS), dim3(256), 0, c->stream, c->dtpart, (size_t)grid.x,
-                           c->ndt_slot + (dir - 1), c->g.halt);
-        HIPCHK(hipGetLastError());
+    if (fullstep) c->dt_nb[dir - 1] = grid.x;
+    return 0;
+}
+
+MinArgs min_args(const harm_ctx *c) { return MinArgs{c->dtpart, c->dtstride, {c->dt_nb[0], c->dt_nb[1], c->dt_nb[2]}}; }
+SumArgs sum_args(const harm_ctx *c)
+{
+    return SumArgs{c->cpart, c->sum_nb,
+                   {8, {HARM_C2P_CALLS, HARM_NEWTON_ITERS, HARM_NEWTON_KCONV, HARM_FAIL_2D, HARM_FIXUP_GAMMA,
+                        HARM_FLOOR_ZONES, HARM_GAMMA_CAP, HARM_FATAL}}};
+}
+
+// What bound() and k_stepend fold in a step, for the entries that run one stage of it.
+int fold_now(harm_ctx *c, bool mins)
+{
+    if (c->sum_nb) {
+        hipLaunchKernelGGL(k_sum_partials, dim3(8 * fold_blocks(c->sum_nb)), dim3(256), 0, c->stream, sum_args(c), c->cnt,
+                           c->g.halt);
+        c->sum_nb = 0;
     }
+    if (mins)
+        hipLaunchKernelGGL(k_min_partials, dim3((c->g.N3 > 2 ? 3 : 2) * RED_BLOCKS), dim3(256), 0, c->stream, min_args(c),
+                           c->ndt_slot, c->g.halt);
+    HIPCHK(hipGetLastError());
     return 0;
 }
 
@@ -3318,9 +3508,13 @@ int fluxes_and_emf(harm_ctx *c, const double *pb, int fullstep, bool emf = true)
 {
     const DGrid &g = c->g;
     int rc;
-    if ((rc = flux_launch(c, 1, pb, c->F1, fullstep))) return rc;
-    if ((rc = flux_launch(c, 2, pb, c->F2, fullstep))) return rc;
-    if (g.N3 > 2 && (rc = flux_launch(c, 3, pb, c->F3, fullstep))) return rc;
+    if (!c->uniform && c->eos_kind != 2) {
+        if ((rc = flux_launch_all(c, pb, fullstep))) return rc;
+    } else {
+        if ((rc = flux_launch(c, 1, pb, c->F1, fullstep))) return rc;
+        if ((rc = flux_launch(c, 2, pb, c->F2, fullstep))) return rc;
+        if (g.N3 > 2 && (rc = flux_launch(c, 3, pb, c->F3, fullstep))) return rc;
+    }
     if (!emf) return 0;
     const size_t ne = (size_t)(g.ie + 2 - g.is) * (g.je + 2 - g.js) * g.N3;
     LAUNCH(HARM_K_EMF, hipLaunchKernelGGL(k_emf, dim3(nblocks8(ne)), dim3(TPB), 0, c->stream, g, c->F1, c->F2, c->F3,
@@ -3332,8 +3526,10 @@ int bound(harm_ctx *c, double *p)
 {
     const DGrid &g = c->g;
     const size_t nb = ((size_t)4 * g.SN2 + (size_t)g.N1 * (4 + 2 * g.polefix)) * g.N3;
-    LAUNCH(HARM_K_BOUND, hipLaunchKernelGGL(k_bound, dim3(nblocks(nb)), dim3(TPB), 0, c->stream, g, p, c->pflag,
-                                            c->font.count, c->seeds.count, c->cnt));
+    const unsigned nbl = nblocks(nb);
+    LAUNCH(HARM_K_BOUND, hipLaunchKernelGGL(k_bound, dim3(nbl + 8 * fold_blocks(c->sum_nb)), dim3(TPB), 0, c->stream, g,
+                                            p, c->pflag, c->font.count, c->seeds.count, nbl, sum_args(c), c->cnt));
+    c->sum_nb = 0;
     return 0;
 }
 
@@ -3341,7 +3537,7 @@ int fixup_utoprim(harm_ctx *c, double *p)
 {
     const DGrid &g = c->g;
     LAUNCH(HARM_K_FIXUTOPRIM,
-           hipLaunchKernelGGL(k_fixutoprim_scan, dim3(nblocks((g.nz + 7) / 8)), dim3(TPB), 0, c->stream, g, p, c->pflag,
+           hipLaunchKernelGGL(k_fixutoprim_scan, dim3(nblocks((g.nz + SCAN_ZONES - 1) / SCAN_ZONES)), dim3(TPB), 0, c->stream, g, p, c->pflag,
                               c->pflag2, c->fix_bits, c->fix_pcount, c->fix_nwords, c->cnt);
            hipLaunchKernelGGL(k_fixutoprim_serial, dim3(g.N3), dim3(64), 0, c->stream, g, p, c->pflag2, c->fix_bits,
                               c->fix_pcount, c->fix_nwords, c->cnt));
@@ -3371,11 +3567,7 @@ int advance_ceos(harm_ctx *c, double *pi, double *pb, double *pf, double dtfac, 
     else
         CEOS_UPD(false);
 #undef CEOS_UPD
-    CntMap map = {8, {HARM_C2P_CALLS, HARM_NEWTON_ITERS, HARM_NEWTON_KCONV, HARM_FAIL_2D, HARM_FIXUP_GAMMA,
-                      HARM_FLOOR_ZONES, HARM_GAMMA_CAP, HARM_FATAL}};
-    hipLaunchKernelGGL(k_sum_partials, dim3(RED_BLOCKS, 8), dim3(256), 0, c->stream, c->cpart, (size_t)nblocks(na), map,
-                       c->cnt, g.halt);
-    HIPCHK(hipGetLastError());
+    c->sum_nb = nblocks(na);
     return 0;
 }
 
@@ -3416,7 +3608,8 @@ int advance(harm_ctx *c, double *pi, double *pb, double *pf, double dtfac, int f
     const DivArgs dv = {c->F1, c->F2, c->F3, c->e1, c->e2, c->e3};
     // the plain wave-uniform update forms the EMFs and the divergence itself; the
     // others read S, which k_div forms from the EMF arrays
-    const bool fused = c->uniform && (mode != UPD_CAPTURE || c->eos_kind == 1) && c->nz < OFF32_MAX_ZONES;
+    const bool fused = c->nz < OFF32_MAX_ZONES &&
+                       (c->eos_kind == 1 || (c->uniform ? mode != UPD_CAPTURE : mode == UPD_PLAIN || mode == UPD_GATED));
     if ((rc = fluxes_and_emf(c, pb, fullstep, !fused))) return rc;
     if (!fused)
         LAUNCH(HARM_K_DIV, hipLaunchKernelGGL(k_div, dim3(nblocks8(na)), dim3(TPB), 0, c->stream, g, dv, c->S));
@@ -3426,7 +3619,9 @@ int advance(harm_ctx *c, double *pi, double *pb, double *pf, double dtfac, int f
                                              c->cpart, ex))
 #define GATED_LAUNCH(U_, F_) UPD_LAUNCH(U_, UPD_GATED, false, F_)
     if (c->eos_kind == 1) {
-        if (fused)
+        if (fused && !c->uniform)
+            UPD_LAUNCH(false, UPD_PLAIN, true, true);
+        else if (fused)
             UPD_LAUNCH(true, UPD_PLAIN, true, true);
         else if (c->uniform)
             UPD_LAUNCH(true, UPD_PLAIN, true, false);
@@ -3448,10 +3643,14 @@ int advance(harm_ctx *c, double *pi, double *pb, double *pf, double dtfac, int f
         else
             UPD_LAUNCH(true, UPD_LEARNED, false, false);
     } else {
-        if (mode == UPD_PLAIN)
+        if (mode == UPD_PLAIN && fused)
+            UPD_LAUNCH(false, UPD_PLAIN, false, true);
+        else if (mode == UPD_PLAIN)
             UPD_LAUNCH(false, UPD_PLAIN, false, false);
         else if (mode == UPD_CAPTURE)
             UPD_LAUNCH(false, UPD_CAPTURE, false, false);
+        else if (mode == UPD_GATED && fused)
+            GATED_LAUNCH(false, true);
         else if (mode == UPD_GATED)
             GATED_LAUNCH(false, false);
         else
@@ -3459,13 +3658,7 @@ int advance(harm_ctx *c, double *pi, double *pb, double *pf, double dtfac, int f
     }
 #undef UPD_LAUNCH
 #undef GATED_LAUNCH
-    {
-        CntMap map = {8, {HARM_C2P_CALLS, HARM_NEWTON_ITERS, HARM_NEWTON_KCONV, HARM_FAIL_2D, HARM_FIXUP_GAMMA,
-                          HARM_FLOOR_ZONES, HARM_GAMMA_CAP, HARM_FATAL}};
-        hipLaunchKernelGGL(k_sum_partials, dim3(RED_BLOCKS, 8), dim3(256), 0, c->stream, c->cpart, (size_t)nblocks(na), map,
-                           c->cnt, g.halt);
-        HIPCHK(hipGetLastError());
-    }
+    c->sum_nb = nblocks(na);
     if (mode == UPD_GATED)
         LAUNCH(HARM_K_MLP, hipLaunchKernelGGL(k_seedfix, dim3(SEEDFIX_BLOCKS), dim3(TPB), 0, c->stream, g, pi, pf,
                                               c->pflag, c->seeds, c->font, ex.mlp, c->cnt));
@@ -3504,9 +3697,8 @@ int one_step(harm_ctx *c)
                                                       c->tr.a, c->p, c->tstate, c->cnt));
     }
     LAUNCH(HARM_K_STEPEND,
-           hipLaunchKernelGGL(k_mdot_partials, dim3(g.N3), dim3(TPB), 0, c->stream, g, c->p, c->part);
-           hipLaunchKernelGGL(k_stepend, dim3(1), dim3(1), 0, c->stream, g, c->tstate, c->ndt_slot, c->part, g.N3,
-                              c->cnt));
+           hipLaunchKernelGGL(k_stepend, dim3(g.N3 + (g.N3 > 2 ? 3 : 2) * RED_BLOCKS), dim3(TPB), 0, c->stream, g, c->p,
+                              c->part, min_args(c), c->step_done, c->tstate, c->ndt_slot, c->cnt));
     return 0;
 }
 
@@ -3624,7 +3816,9 @@ int ctx_alloc(harm_ctx *c)
     }
     if ((rc = dalloc(&c->tstate, 8))) return rc;
     if ((rc = dalloc(&c->ndt_slot, 3))) return rc;
-    if ((rc = dalloc(&c->dtpart, (size_t)nblocks8(c->nz)))) return rc;
+    c->dtstride = nblocks8(c->nz);
+    if ((rc = dalloc(&c->dtpart, 3 * c->dtstride))) return rc;
+    if ((rc = dalloc(&c->step_done, 1))) return rc;
     if ((rc = dalloc(&c->cpart, 8 * (size_t)nblocks(c->nz)))) return rc;
     if ((rc = dalloc(&c->cnt, HARM_NCOUNTERS))) return rc;
     c->npart = std::max<size_t>(DIAG_NPART * nblocks(c->nz) + 16, 2 * (size_t)hg.N3 + 16);
@@ -3687,7 +3881,7 @@ void ctx_free(harm_ctx *c)
 {
     for (void *q : {(void *)c->p, (void *)c->ph, (void *)c->F1, (void *)c->F2, (void *)c->F3, (void *)c->e1,
                     (void *)c->e2, (void *)c->e3, (void *)c->S, (void *)c->pflag, (void *)c->pflag2, (void *)c->d_conn,
-                    (void *)c->d_floors, (void *)c->d_katm, (void *)c->tstate, (void *)c->ndt_slot, (void *)c->dtpart, (void *)c->cpart, (void *)c->cnt,
+                    (void *)c->d_floors, (void *)c->d_katm, (void *)c->tstate, (void *)c->ndt_slot, (void *)c->dtpart, (void *)c->step_done, (void *)c->cpart, (void *)c->cnt,
                     (void *)c->part, (void *)c->fix_bits, (void *)c->fix_pcount, (void *)c->fix_err, (void *)c->font.count, (void *)c->font.zone, (void *)c->font.U,
                     (void *)c->d_cblk, (void *)c->d_fblk, (void *)c->seeds.count, (void *)c->seeds.zone,
                     (void *)c->seeds.U, (void *)c->lastT, (void *)c->ceos_vals, (void *)c->ceos_solves,
@@ -4128,7 +4322,7 @@ int harm_debug_fluxes(harm_ctx *c, int fullstep, double *F1, double *F2, double 
     int rc;
     const DGrid &g = c->g;
     c->flux_valid = false;
-    if ((rc = fluxes_and_emf(c, c->p, fullstep))) return rc;
+    if ((rc = fluxes_and_emf(c, c->p, fullstep)) || (rc = fold_now(c, fullstep != 0))) return rc;
     // materialize the flux_ct rewrite on the host from the EMFs (step_ch.c:541-554, 783-797)
     const size_t n = 8 * c->nz;
     std::vector<double> e1, e2, e3(c->nz);
@@ -4202,9 +4396,9 @@ int harm_debug_advance(harm_ctx *c, int fullstep, double *ph)
     c->flux_valid = false;
     if (fullstep) {
         HIPCHK(hipMemcpyAsync(c->ph, ph, bytes, hipMemcpyHostToDevice, c->stream));
-        if ((rc = advance(c, c->p, c->ph, c->p, 1.0, 1))) return rc;
+        if ((rc = advance(c, c->p, c->ph, c->p, 1.0, 1)) || (rc = fold_now(c, true))) return rc;
     } else {
-        if ((rc = advance(c, c->p, c->p, c->ph, 0.5, 0))) return rc;
+        if ((rc = advance(c, c->p, c->p, c->ph, 0.5, 0)) || (rc = fold_now(c, false))) return rc;
         HIPCHK(hipMemcpyAsync(ph, c->ph, bytes, hipMemcpyDeviceToHost, c->stream));
     }
     // the step's next bound() would empty the Font-fix and seed lists
@@ -4643,14 +4837,17 @@ int harm_utoprim2d_batch(const double *U, const double *gcov, const double *gcon
         if (opts->guess_mode == 2 && !(opts->gate_tau > 0.)) return set_err("guess_mode 2 needs gate_tau > 0", 4);
         if (opts->guess_mode == 2) gate = opts->gate_tau;
         mv = harm_mlp_view((const harm_mlp *)opts->mlp);
-        hipLaunchKernelGGL((k_c2p_batch<true>), dim3(nblocks(n)), dim3(TPB), 0, (hipStream_t)stream, U, gcov, gcon,
-                           gdet, prim, ret, iters, kconv, n, opts->gam, opts->font_fix, opts->K, (int *)nullptr, mv, gate);
-    } else if (opts->guess_mode == 0) {
-        hipLaunchKernelGGL((k_c2p_batch<false>), dim3(nblocks(n)), dim3(TPB), 0, (hipStream_t)stream, U, gcov, gcon,
-                           gdet, prim, ret, iters, kconv, n, opts->gam, opts->font_fix, opts->K, (int *)nullptr, mv, gate);
-    } else {
+    } else if (opts->guess_mode != 0) {
         return set_err("unknown guess_mode", 4);
     }
+    auto *k = opts->font_fix ? (opts->guess_mode == 0   ? k_c2p_batch<0, true>
+                                : opts->guess_mode == 1 ? k_c2p_batch<1, true>
+                                                        : k_c2p_batch<2, true>)
+                             : (opts->guess_mode == 0   ? k_c2p_batch<0, false>
+                                : opts->guess_mode == 1 ? k_c2p_batch<1, false>
+                                                        : k_c2p_batch<2, false>);
+    hipLaunchKernelGGL(k, dim3(nblocks(n)), dim3(TPB), 0, (hipStream_t)stream, U, gcov, gcon, gdet, prim, ret, iters,
+                       kconv, n, opts->gam, opts->K, (int *)nullptr, mv, gate);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -4834,9 +5031,9 @@ int Utoprim_2d(double U[8], double gcov[4][4], double gcon[4][4], double gdet, d
     if (rc) return rc;
     MlpDev mv;
     std::memset(&mv, 0, sizeof(mv));
-    hipLaunchKernelGGL((k_c2p_batch<false>), dim3(1), dim3(TPB), 0, 0, s.buf, s.buf + 8, s.buf + 24, s.buf + 40,
-                       s.buf + 41, s.ret8, (uint8_t *)nullptr, (uint8_t *)nullptr, (size_t)1, g_gamma, 0, 0., s.ret,
-                       mv, 0.);
+    hipLaunchKernelGGL((k_c2p_batch<0, false>), dim3(1), dim3(TPB), 0, 0, s.buf, s.buf + 8, s.buf + 24, s.buf + 40,
+                       s.buf + 41, s.ret8, (uint8_t *)nullptr, (uint8_t *)nullptr, (size_t)1, g_gamma, 0., s.ret, mv,
+                       0.);
     HIPCHK(hipGetLastError());
     int r = 0;
     if ((rc = u2p_unstage(s, prim, r))) return rc;

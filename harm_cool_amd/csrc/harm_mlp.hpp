@@ -103,7 +103,7 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float mlp_tanh(float x)
 {
     // tanh(x) = 1 - 2 / (exp(2x) + 1); saturates correctly at both ends.
-    const float e = __expf(2.f * x);
+    const float e = __builtin_amdgcn_exp2f(2.88539008f * x);  // 2 log2(e)
     return 1.f - 2.f * __builtin_amdgcn_rcpf(e + 1.f);
 }
 
@@ -143,15 +143,38 @@ __device__ __forceinline__ void mlp_hidden(const MlpDev &m, int chunk0, int boff
         }
 }
 
+// The packed operands and biases in a block's LDS (22.5 KB), for kernels whose zones'
+// state leaves no room for the 88 registers that hold them over a forward pass: m with
+// its pointers moved there.  Every thread of the block must call it.
+struct MlpLds {
+    uint4 w[MLP_CHUNKS * 64];
+    float4 b[MLP_BIAS_LEN / 4];
+};
+__device__ __forceinline__ MlpDev mlp_stage(const MlpDev &m, MlpLds &lds)
+{
+    for (int k = threadIdx.x; k < MLP_CHUNKS * 64; k += blockDim.x) lds.w[k] = m.wpack[k];
+    for (int k = threadIdx.x; k < MLP_BIAS_LEN / 4; k += blockDim.x)
+        lds.b[k] = reinterpret_cast<const float4 *>(m.bias)[k];
+    __syncthreads();
+    MlpDev r = m;
+    r.wpack = lds.w;
+    r.bias = reinterpret_cast<const float *>(lds.b);
+    return r;
+}
+
 // Forward pass for the 64 zones of this wavefront.  x = standardized inputs
 // of this lane's zone; returns the standardized outputs of this lane's zone.
 // Every lane of the wavefront must call it (MFMA reads all 64 lanes).
+// STAGED: m points to LDS (mlp_stage); each tile then reads the operands where it uses
+// them instead of keeping them over the tiles.
+template <bool STAGED = false>
 __device__ __forceinline__ void mlp_forward_wave(const MlpDev &m, const float (&x)[MLP_NIN], float &y0, float &y1)
 {
     const int lane = threadIdx.x & 63, gq = lane >> 4, n = lane & 15;
     float o0 = 0.f, o1 = 0.f;
 #pragma unroll 1
     for (int t = 0; t < 4; t++) {
+        if (STAGED) asm volatile("" ::: "memory");
         const int src = 16 * t + n;
         bf16x8_t b;
 #pragma unroll
