@@ -189,8 +189,9 @@ __device__ inline int ceos_solve_Tp(const CacheView &c, const CeosHint &hx, cons
 
 // pressure_rho0_u_CoolEOS with the zone's last temperature T (cooleos.c:314-444;
 // MAXLOS 1: one solve, no random restart): the pressure and the new last T.
-// One out-of-line copy serves every call site of a kernel.
-__device__ __noinline__ CeosOut ceos_solve(const CeosParams *P, int r, double T, double rho0, double u)
+// Inlined where a kernel has one or two call sites: the call's stack frame and the
+// registers it saves there cost the zone update more traffic than its arrays.
+__device__ __forceinline__ CeosOut ceos_solve(const CeosParams *P, int r, double T, double rho0, double u)
 {
     // every parameter read at once, ahead of the first branch
     const double rho_unit = P->rho_unit, u_unit = P->u_unit, p_unit = P->p_unit, gam = P->gam;
@@ -223,6 +224,12 @@ __device__ __noinline__ CeosOut ceos_solve(const CeosParams *P, int r, double T,
     return o;
 }
 
+// One out-of-line copy for kernels whose finite-difference derivatives solve too.
+__device__ __noinline__ CeosOut ceos_solve_call(const CeosParams *P, int r, double T, double rho0, double u)
+{
+    return ceos_solve(P, r, T, rho0, u);
+}
+
 // The tabulated EOS policy of the step's physics templates (face_flux, vchar,
 // source, primtoflux) and, through Eos5Cache, of the 5D inversion.
 // V: the finite-difference steps rho0 hh / RHO_UNIT and u hh / U_UNIT are below
@@ -241,7 +248,7 @@ struct EosCacheT {
         const unsigned long long kr = (unsigned long long)__double_as_longlong(rho0);
         const unsigned long long ku = (unsigned long long)__double_as_longlong(u);
         if (z->has && kr == z->kr && ku == z->ku) return z->p;
-        const CeosOut o = ceos_solve(P, r, z->T, rho0, u);
+        const CeosOut o = V ? ceos_solve(P, r, z->T, rho0, u) : ceos_solve_call(P, r, z->T, rho0, u);
         z->T = o.T;
         z->nsolve += o.solved;
         z->has = true;
@@ -303,7 +310,17 @@ template <bool V>
 struct Eos5CacheT {
     EosCacheT<V> e;
     double gam;
+    const double *tab;  // the zone's metric (load_geom)
+    size_t ncol, col;
     __device__ static constexpr bool tabulated() { return true; }
+    // The lanes of a wavefront share one or two columns, so the metric's 40 numbers are a
+    // few cache lines, where spilled they are 320 bytes a zone.
+    __device__ void refresh(Geom &g) const
+    {
+        const double *p = tab;
+        asm volatile("" : "+s"(p));  // a new value to the compiler, which would keep the old loads'
+        load_geom(p, ncol, col, g);
+    }
     __device__ EosPt at(double rho, double u) const { return e.at(rho, u); }
     __device__ void derivs(double rho, double u, EosPt &pt) const
     {

@@ -1338,6 +1338,15 @@ __global__ void __launch_bounds__(TPB) k_ceos_table(CacheView v, const double *c
     cache_tab_fill(c, 0, comp, ix, left, tab[blockIdx.y] + comp * cache_tab_plane(v.X, v.Y));
 }
 
+// The solves of a block, into one of SOLVE_SLOTS counts on lines of their own (every
+// wavefront of these kernels has some; one count for all of them is one address that
+// every XCD waits for).
+constexpr int SOLVE_SLOTS = 64, SOLVE_LINE = 16;
+__device__ __forceinline__ void add_solves(unsigned long long *__restrict__ solves, int v)
+{
+    add_counter(solves, (int)(blockIdx.x % SOLVE_SLOTS) * SOLVE_LINE, v);
+}
+
 // The stencil of a face along DIR: zones m-2, m-1 (left of the face), m, m+1.
 template <int DIR>
 __device__ __forceinline__ void ceos_stencil(const DGrid &g, size_t z, int h, size_t &zm2, size_t &zm1, size_t &zp1)
@@ -1416,18 +1425,17 @@ k_face_eos(DGrid g, CeosParams ce, double *__restrict__ lastT, const double *__r
         zs.T = lastT[z];
         if (chain && zs.T == 0.0 && j > g.js) zs.T = lastT[z - g.N3];
         const EosCacheT<V> eos{&ce, ceos_radius(ce, i), &zs};
-        const EosPt el = eos.at(rl, ul);
-        const double cl = eos.cs2(rl, ul, el);
-        const EosPt er = eos.at(rr, ur);
-        const double cr = eos.cs2(rr, ur, er);
+#pragma unroll 1
+        for (int s = 0; s < 2; s++) {  // one copy of the solve for both states
+            const double r = s ? rr : rl, u = s ? ur : ul;
+            const EosPt e = eos.at(r, u);
+            fe[(2 * s) * nz + z] = e.p;
+            fe[(2 * s + 1) * nz + z] = eos.cs2(r, u, e);
+        }
         lastT[z] = zs.T;
         nsolve += zs.nsolve;
-        fe[0 * nz + z] = el.p;
-        fe[1 * nz + z] = cl;
-        fe[2 * nz + z] = er.p;
-        fe[3 * nz + z] = cr;
     });
-    add_counter(solves, 0, nsolve);
+    add_solves(solves, nsolve);
 }
 
 // The EOS policy of a face whose two states' pressures and sound speeds
@@ -1499,17 +1507,77 @@ __global__ void __launch_bounds__(TPB) k_flux_ceos(DGrid g, const double *__rest
     add_counter(cnt, HARM_FATAL, fatal);
 }
 
-// advance()'s zone loop with COOL_EOS (step_ch.c:237-306): InitCache_CoolEOS,
-// the source at pb, primtoU at pi, the update with the flux divergence S,
-// Utoprim_5d seeded with pi (no Font fix), then fixup1zone (fixup.c:51-60).
+// advance()'s zone loop with COOL_EOS (step_ch.c:237-306) in two kernels, as one holds
+// more than its registers (256 and 131 spilled: 1.5 KB a zone of scratch traffic).
+//
+// InitCache_CoolEOS, the source at pb, primtoU at pi and the flux divergence (formed
+// here with the EMFs, or S from k_div on grids beyond 32-bit offsets): the conserved
+// vector of active zone idx into S and the pressure at pi into fe.
+template <bool V, bool FUSED>
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(CEOS_WPE, 8)))
+k_cons_ceos(DGrid g, CeosParams ce, DivArgs dv, double *__restrict__ lastT, const double *__restrict__ pi,
+            const double *__restrict__ pb, double *__restrict__ S, double *__restrict__ fe,
+            const double *__restrict__ tstate, double dtfac, int pi_is_pb, unsigned long long *__restrict__ solves,
+            unsigned long long *__restrict__ cnt)
+{
+    if (halted(g)) return;
+    const int ni = g.ie - g.is + 1, nj = g.je - g.js + 1;
+    const size_t na = (size_t)ni * nj * g.N3;
+    const size_t idx = (size_t)xcd_block() * TPB + threadIdx.x;
+    int fatal = 0, nsolve = 0;
+    if (idx < na) {
+        const unsigned rest = (unsigned)idx / (unsigned)g.N3;
+        const int h = (int)((unsigned)idx - rest * (unsigned)g.N3);
+        const unsigned ri = rest / (unsigned)nj;
+        const int j = g.js + (int)(rest - ri * (unsigned)nj);
+        const int i = g.is + (int)ri;
+        const size_t z = zidx(g, i, j, h), nz = g.nz, col = (size_t)i * g.SN2 + j;
+        const double Dt = dtfac * tstate[1];
+        double pbz[NPR], piz[NPR], dU[NPR], U[NPR];
+#pragma unroll
+        for (int k = 0; k < NPR; k++) pbz[k] = pb[k * nz + z];
+#pragma unroll
+        for (int k = 0; k < NPR; k++) piz[k] = pi_is_pb ? pbz[k] : pi[k * nz + z];
+        CeosZone zs;
+        zs.T = lastT[z];
+        const EosCacheT<V> eos{&ce, ceos_radius(ce, i), &zs};
+        double P = 0., Ppb = 0.;
+#pragma unroll 1
+        for (int s = 0; s <= (pi_is_pb ? 0 : 1); s++) {  // one copy of the solve for both states
+            P = eos.at(s ? piz[RHO] : pbz[RHO], s ? piz[UU] : pbz[UU]).p;
+            if (s == 0) Ppb = P;
+        }
+        lastT[z] = zs.T;
+        nsolve = zs.nsolve;
+        fe[z] = P;
+        Geom geom;
+        load_geom(g.geom[CENT], g.ncol, col, geom);
+        State q;
+        source(pbz, geom, g.conn, g.ncol, col, Ppb, dU, q, fatal);
+        if (!pi_is_pb) get_state(piz, geom, q, fatal);
+        primtoflux_P(piz, q, 0, geom, P, U);
+        double d[NPR];
+        if constexpr (FUSED) {
+            flux_div32<false>(g, dv, i, j, h, d);
+        } else {
+#pragma unroll
+            for (int k = 0; k < NPR; k++) d[k] = S[k * na + idx];
+        }
+#pragma unroll
+        for (int k = 0; k < NPR; k++) S[k * na + idx] = U[k] + Dt * (d[k] + dU[k]);
+    }
+    add_counter(cnt, HARM_FATAL, fatal);
+    add_solves(solves, nsolve);
+}
+
+// Utoprim_5d of those vectors seeded with pi (no Font fix), then fixup1zone
+// (fixup.c:51-60).
 template <bool V>
-__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(CEOS_WPE, 8))) k_update_ceos(DGrid g, CeosParams ce, double *__restrict__ lastT,
-                                                     const double *__restrict__ pi, const double *__restrict__ pb,
-                                                     double *__restrict__ pf, int8_t *__restrict__ pflag,
-                                                     const double *__restrict__ S,
-                                                     const double *__restrict__ tstate, double dtfac, int pi_is_pb,
-                                                     unsigned long long *__restrict__ cpart,
-                                                     unsigned long long *__restrict__ solves)
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(CEOS_WPE, 8)))
+k_update_ceos(DGrid g, CeosParams ce, double *__restrict__ lastT, const double *__restrict__ pi,
+              double *__restrict__ pf, int8_t *__restrict__ pflag, const double *__restrict__ S,
+              const double *__restrict__ fe, unsigned long long *__restrict__ cpart,
+              unsigned long long *__restrict__ solves)
 {
     if (halted(g)) return;
     const int ni = g.ie - g.is + 1, nj = g.je - g.js + 1;
@@ -1523,33 +1591,24 @@ __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(CEOS_W
         const int j = g.js + (int)(rest - ri * (unsigned)nj);
         const int i = g.is + (int)ri;
         const size_t z = zidx(g, i, j, h), nz = g.nz, col = (size_t)i * g.SN2 + j;
-        const double Dt = dtfac * tstate[1];
         Geom geom;
         load_geom(g.geom[CENT], g.ncol, col, geom);
         CeosZone zs;
         zs.T = lastT[z];
         const EosCacheT<V> eos{&ce, ceos_radius(ce, i), &zs};
-        double pbz[NPR], piz[NPR], dU[NPR], U[NPR];
+        double pr[NPR], U[NPR];
 #pragma unroll
-        for (int k = 0; k < NPR; k++) pbz[k] = pb[k * nz + z];
-        State q;
-        EosPt e = eos.at(pbz[RHO], pbz[UU]);
-        source(pbz, geom, g.conn, g.ncol, col, e.p, dU, q, fatal);
+        for (int k = 0; k < NPR; k++) pr[k] = pi[k * nz + z];
 #pragma unroll
-        for (int k = 0; k < NPR; k++) piz[k] = pi_is_pb ? pbz[k] : pi[k * nz + z];
-        if (!pi_is_pb) {
-            get_state(piz, geom, q, fatal);
-            e = eos.at(piz[RHO], piz[UU]);
-        }
-        primtoflux_P(piz, q, 0, geom, e.p, U);
-#pragma unroll
-        for (int k = 0; k < NPR; k++) U[k] += Dt * (S[k * na + idx] + dU[k]);
-        double pr[NPR];
-#pragma unroll
-        for (int k = 0; k < NPR; k++) pr[k] = piz[k];
+        for (int k = 0; k < NPR; k++) U[k] = S[k * na + idx];
+        // the pressure call at pi was k_cons_ceos's last: a call there repeats it
+        zs.has = true;
+        zs.kr = (unsigned long long)__double_as_longlong(pr[RHO]);
+        zs.ku = (unsigned long long)__double_as_longlong(pr[UU]);
+        zs.p = fe[z];
         int niter = 0;
-        const Eos5CacheT<V> e5{eos, g.gam};
-        const int ret = utoprim_5d(U, geom, e5, e, pr, niter);
+        const Eos5CacheT<V> e5{eos, g.gam, g.geom[CENT], (size_t)g.ncol, col};
+        const int ret = utoprim_5d(U, geom, e5, EosPt{zs.p, 0., 0.}, pr, niter);
         lastT[z] = zs.T;
         nsolve = zs.nsolve;
         c_call = 1;
@@ -1570,7 +1629,7 @@ __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(CEOS_W
     }
     const int v[8] = {c_call, c_iter, c_kconv, c_f2d, c_gam, c_flr, c_cap, fatal};
     block_counts<8>(v, cpart);
-    add_counter(solves, 0, nsolve);
+    add_solves(solves, nsolve);
 }
 
 // The zones the gated update put on the seed list: the network's seed for
@@ -1935,7 +1994,7 @@ __global__ void __launch_bounds__(TPB) k_fixutoprim_scan(DGrid g, double *__rest
     if (halted(g)) return;
     // 32 zones per thread: the common all-good octet is an 8-byte load and store, and a
     // wavefront whose lanes met no bad zone leaves the counters alone (8 zones a thread
-    // with every counter's wave sum: 30 us on 288x256x256, now 10 us).
+    // with every counter's wave sum: 30 us on 288x256x256, now 14 us).
     const size_t t0 = ((size_t)blockIdx.x * TPB + threadIdx.x) * SCAN_ZONES;
     int c_rep = 0, c_nost = 0, c_flr = 0, c_cap = 0, c_gam = 0, fatal = 0;
     bool bad = false;
@@ -3548,20 +3607,25 @@ int fixup_utoprim(harm_ctx *c, double *p)
 // advance() (step_ch.c:153-318) with fixup() folded into the update and the
 // Font-fix pass (step_ch.c:101-103, 112-114).  The Font-fix and seed lists it
 // fills are emptied by the next bound().
-// advance() with the cache EOS: the fluxes, their divergence, then the zone
-// update (k_update_ceos) with its fixup.
+// advance() with the cache EOS: the fluxes, the conserved vectors (k_cons_ceos), then
+// the zone update (k_update_ceos) with its fixup.
 int advance_ceos(harm_ctx *c, double *pi, double *pb, double *pf, double dtfac, int fullstep)
 {
     const DGrid &g = c->g;
     int rc;
     const size_t na = (size_t)(g.ie - g.is + 1) * (g.je - g.js + 1) * g.N3;
     const DivArgs dv = {c->F1, c->F2, c->F3, c->e1, c->e2, c->e3};
-    if ((rc = fluxes_and_emf(c, pb, fullstep, true))) return rc;
-    LAUNCH(HARM_K_DIV, hipLaunchKernelGGL(k_div, dim3(nblocks8(na)), dim3(TPB), 0, c->stream, g, dv, c->S));
-#define CEOS_UPD(V_)                                                                                             \
-    LAUNCH(HARM_K_UPDATE, hipLaunchKernelGGL(k_update_ceos<V_>, dim3(nblocks(na)), dim3(TPB), 0, c->stream, g,     \
-                                             c->ceos, c->lastT, pi, pb, pf, c->pflag, c->S, c->tstate, dtfac,      \
-                                             (pi == pb) ? 1 : 0, c->cpart, c->ceos_solves))
+    const bool fused = c->nz < OFF32_MAX_ZONES;
+    if ((rc = fluxes_and_emf(c, pb, fullstep, !fused))) return rc;
+    if (!fused)
+        LAUNCH(HARM_K_DIV, hipLaunchKernelGGL(k_div, dim3(nblocks8(na)), dim3(TPB), 0, c->stream, g, dv, c->S));
+#define CEOS_UPD(V_)                                                                                                \
+    LAUNCH(HARM_K_UPDATE,                                                                                           \
+           auto *cons = fused ? k_cons_ceos<V_, true> : k_cons_ceos<V_, false>;                                     \
+           hipLaunchKernelGGL(cons, dim3(nblocks8(na)), dim3(TPB), 0, c->stream, g, c->ceos, dv, c->lastT, pi, pb,  \
+                              c->S, c->ceos_fe, c->tstate, dtfac, (pi == pb) ? 1 : 0, c->ceos_solves, c->cnt);      \
+           hipLaunchKernelGGL(k_update_ceos<V_>, dim3(nblocks(na)), dim3(TPB), 0, c->stream, g, c->ceos, c->lastT,  \
+                              pi, pf, c->pflag, c->S, c->ceos_fe, c->cpart, c->ceos_solves))
     if (c->ceos_vanish)
         CEOS_UPD(true);
     else
@@ -4545,9 +4609,9 @@ int harm_set_eos_cache(harm_ctx *c, const harm_cache *const *caches, int n, cons
     HIPCHK(hipStreamSynchronize(c->stream));
     if (!c->lastT && (rc = dalloc(&c->lastT, c->nz))) return rc;
     if (!c->ceos_fe && (rc = dalloc(&c->ceos_fe, 4 * c->nz))) return rc;
-    if (!c->ceos_solves && (rc = dalloc(&c->ceos_solves, 1))) return rc;
+    if (!c->ceos_solves && (rc = dalloc(&c->ceos_solves, SOLVE_SLOTS * SOLVE_LINE))) return rc;
     HIPCHK(hipMemset(c->lastT, 0, c->nz * sizeof(double)));  // calloc'ed by SetupCache_CoolEOS, cooleos.c:834
-    HIPCHK(hipMemset(c->ceos_solves, 0, sizeof(unsigned long long)));
+    HIPCHK(hipMemset(c->ceos_solves, 0, SOLVE_SLOTS * SOLVE_LINE * sizeof(unsigned long long)));
     HIPCHK(hipDeviceSynchronize());
     c->ceos = P;
     c->ceos_vanish = ceos_vanishing_steps(P.rho_unit, P.u_unit);
@@ -4579,12 +4643,13 @@ int harm_set_last_T(harm_ctx *c, const double *T)
 int harm_get_eos_solves(harm_ctx *c, int64_t *n)
 {
     if (!c || !n) return set_err("null argument");
-    unsigned long long v = 0;
+    unsigned long long v[SOLVE_SLOTS * SOLVE_LINE] = {0}, sum = 0;
     if (c->ceos_solves) {
-        HIPCHK(hipMemcpyAsync(&v, c->ceos_solves, sizeof(v), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipMemcpyAsync(v, c->ceos_solves, sizeof(v), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
     }
-    *n = (int64_t)v;
+    for (unsigned long long k : v) sum += k;
+    *n = (int64_t)sum;
     return 0;
 }
 

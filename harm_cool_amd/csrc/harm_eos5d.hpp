@@ -93,6 +93,7 @@ struct Eos5 {
         return e;
     }
     __device__ void derivs(double, double, EosPt &) const {}
+    __device__ void refresh(Geom &) const {}
 };
 
 // ---- utoprim_5d.c, restated for one zone -----------------------------------
@@ -406,9 +407,10 @@ __device__ inline void func_5d(const E5 &eos, const double *U_target, const Geom
 
 // Utoprim_5d (utoprim_5d.c:179-239) with general_newton_raphson
 // (utoprim_5d.c:890-983) and calc_errx_5d (utoprim_5d.c:378-400).
-// e: the EOS at prim's density and energy.
+// e: the EOS at prim's density and energy.  E5::refresh may read the metric again, where
+// at() needs the registers that would hold it.
 template <class E5>
-__device__ inline int utoprim_5d(const double *U, const Geom &g, const E5 &eos, EosPt e, double *prim, int &n_iter_out)
+__device__ inline int utoprim_5d(const double *U, Geom &g, const E5 &eos, EosPt e, double *prim, int &n_iter_out)
 {
 #pragma unroll
     for (int k = B1; k <= B3; k++) prim[k] = U[k] / g.g;
@@ -421,6 +423,7 @@ __device__ inline int utoprim_5d(const double *U, const Geom &g, const E5 &eos, 
     bool keep = true;
     while (keep) {
         double dx[N5];
+        eos.refresh(g);
         func_5d(eos, U, g, z5, x, prim + B1, e, dx, f, df);
 #pragma unroll
         for (int id = 0; id < N5; id++) x[id] += dx[id];
@@ -445,6 +448,7 @@ __device__ inline int utoprim_5d(const double *U, const Geom &g, const E5 &eos, 
         n_iter++;
     }
     n_iter_out = n_iter;
+    eos.refresh(g);
     int ret = 0;
     if (!isfinite(f) || !isfinite(df))
         ret = 2;
