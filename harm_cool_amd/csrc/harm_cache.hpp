@@ -557,24 +557,37 @@ HC_HD void cache_spline_tab(int X, int Y, const double *tab, const CacheXWin &w,
 {
     const size_t is = (size_t)X * Y * 4;
     const double *p = tab + ((size_t)u.left * X + w.x0) * 4;
+    const int r3 = w.w4 ? 12 : 8;  // (a row that the axis does not have is not read)
     double q[4], d[4];
 #pragma unroll
     for (int b = 0; b < 4; b++) {
-        const double *r = p + 4 * (b == 3 && !w.w4 ? 2 : b);  // (a row that the axis does not have is not read)
-        const CacheD2 lo = cache_ld2(r + u.i * is), hi = cache_ld2(r + u.i * is + 2);
+        const double *r = p + u.i * is + (b == 3 ? r3 : 4 * b);
+        const CacheD2 lo = cache_ld2(r), hi = cache_ld2(r + 2);
         q[b] = lo.a + lo.b * u.t + hi.a * u.t * u.t + hi.b * u.t * u.t * u.t;
         if (DER) {
-            CacheD2 l = lo, g = hi;
-            if (u.im != u.i) l = cache_ld2(r + u.im * is), g = cache_ld2(r + u.im * is + 2);
-            const double om = l.a + l.b * u.tm + g.a * u.tm * u.tm + g.b * u.tm * u.tm * u.tm;
-            l = lo, g = hi;
-            if (u.ip != u.i) l = cache_ld2(r + u.ip * is), g = cache_ld2(r + u.ip * is + 2);
-            const double op = l.a + l.b * u.tp + g.a * u.tp * u.tp + g.b * u.tp * u.tp * u.tp;
+            const double om = lo.a + lo.b * u.tm + hi.a * u.tm * u.tm + hi.b * u.tm * u.tm * u.tm;
+            const double op = lo.a + lo.b * u.tp + hi.a * u.tp * u.tp + hi.b * u.tp * u.tp * u.tp;
+            d[b] = (op - om) / u.h2;
+        }
+    }
+    if (DER && u.im != u.ip) {  // y - h or y + h lies in the interval beside
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            const double *r = p + (b == 3 ? r3 : 4 * b);
+            CacheD2 lo = cache_ld2(r + u.im * is), hi = cache_ld2(r + u.im * is + 2);
+            const double om = lo.a + lo.b * u.tm + hi.a * u.tm * u.tm + hi.b * u.tm * u.tm * u.tm;
+            lo = cache_ld2(r + u.ip * is), hi = cache_ld2(r + u.ip * is + 2);
+            const double op = lo.a + lo.b * u.tp + hi.a * u.tp * u.tp + hi.b * u.tp * u.tp * u.tp;
             d[b] = (op - om) / u.h2;
         }
     }
     v = cache_xspline(w, q[0], q[1], q[2], q[3]);
-    if (DER) dv = cache_xspline(w, d[0], d[1], d[2], d[3]);
+    if (DER) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        __builtin_amdgcn_sched_barrier(0);  // the two side by side take half as many registers again
+#endif
+        dv = cache_xspline(w, d[0], d[1], d[2], d[3]);
+    }
 }
 
 // cache_lookup's status of (x, y) in z plane zindex, or for the plane -1 of a cache

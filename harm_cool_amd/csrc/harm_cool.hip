@@ -1315,12 +1315,9 @@ k_update(DGrid g, const double *__restrict__ pi, const double *__restrict__ pb, 
 // calls (harm_ceos.hpp).  lastT is zone-indexed like the primitives.
 // ---------------------------------------------------------------------------
 
-#ifndef CEOS_WPE
-#define CEOS_WPE 2
-#endif
-#ifndef CEOS_EOS_WPE
-#define CEOS_EOS_WPE 2
-#endif
+// Wavefronts a SIMD of the cache-EOS kernels: two for the inversion's 256 registers,
+// three for the solves of faces and zones (165).
+constexpr int CEOS_WPE = 2, CEOS_EOS_WPE = 3;
 
 // The tables of the splines along T of e and p of cache blockIdx.y (cache_tab_fill): one
 // (component, x row, bracket) per thread.
@@ -1507,53 +1504,77 @@ __global__ void __launch_bounds__(TPB) k_flux_ceos(DGrid g, const double *__rest
     add_counter(cnt, HARM_FATAL, fatal);
 }
 
-// advance()'s zone loop with COOL_EOS (step_ch.c:237-306) in two kernels, as one holds
-// more than its registers (256 and 131 spilled: 1.5 KB a zone of scratch traffic).
-//
-// InitCache_CoolEOS, the source at pb, primtoU at pi and the flux divergence (formed
-// here with the EMFs, or S from k_div on grids beyond 32-bit offsets): the conserved
-// vector of active zone idx into S and the pressure at pi into fe.
-template <bool V, bool FUSED>
-__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(CEOS_WPE, 8)))
-k_cons_ceos(DGrid g, CeosParams ce, DivArgs dv, double *__restrict__ lastT, const double *__restrict__ pi,
-            const double *__restrict__ pb, double *__restrict__ S, double *__restrict__ fe,
-            const double *__restrict__ tstate, double dtfac, int pi_is_pb, unsigned long long *__restrict__ solves,
-            unsigned long long *__restrict__ cnt)
+// advance()'s zone loop with COOL_EOS (step_ch.c:237-306) in three kernels: the solves,
+// which wait for a chain of reads each, want wavefronts, the rest registers (one kernel
+// for all held 256 and spilled 131, 1.5 KB of scratch traffic a zone; 96^3 zones: 870 us,
+// now 615).
+
+// Active zone idx of a grid-order launch.
+__device__ __forceinline__ void active_zone(const DGrid &g, size_t idx, int &i, int &j, int &h)
+{
+    const unsigned nj = (unsigned)(g.je - g.js + 1);
+    const unsigned rest = (unsigned)idx / (unsigned)g.N3;
+    h = (int)((unsigned)idx - rest * (unsigned)g.N3);
+    const unsigned ri = rest / nj;
+    j = g.js + (int)(rest - ri * nj);
+    i = g.is + (int)ri;
+}
+
+// InitCache_CoolEOS and the pressures at pb (into fe[0]) and at pi (fe[1]).
+template <bool V>
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(CEOS_EOS_WPE, 8)))
+k_zone_eos(DGrid g, CeosParams ce, double *__restrict__ lastT, const double *__restrict__ pi,
+           const double *__restrict__ pb, double *__restrict__ fe, int pi_is_pb, unsigned long long *__restrict__ solves)
 {
     if (halted(g)) return;
-    const int ni = g.ie - g.is + 1, nj = g.je - g.js + 1;
-    const size_t na = (size_t)ni * nj * g.N3;
-    const size_t idx = (size_t)xcd_block() * TPB + threadIdx.x;
-    int fatal = 0, nsolve = 0;
+    const size_t na = (size_t)(g.ie - g.is + 1) * (g.je - g.js + 1) * g.N3;
+    const size_t idx = (size_t)blockIdx.x * TPB + threadIdx.x;
+    int nsolve = 0;
     if (idx < na) {
-        const unsigned rest = (unsigned)idx / (unsigned)g.N3;
-        const int h = (int)((unsigned)idx - rest * (unsigned)g.N3);
-        const unsigned ri = rest / (unsigned)nj;
-        const int j = g.js + (int)(rest - ri * (unsigned)nj);
-        const int i = g.is + (int)ri;
+        int i, j, h;
+        active_zone(g, idx, i, j, h);
+        const size_t z = zidx(g, i, j, h), nz = g.nz;
+        const double r[2] = {pb[RHO * nz + z], pi[RHO * nz + z]}, u[2] = {pb[UU * nz + z], pi[UU * nz + z]};
+        CeosZone zs;
+        zs.T = lastT[z];
+        const EosCacheT<V> eos{&ce, ceos_radius(ce, i), &zs};
+        const int ns = pi_is_pb ? 1 : 2;
+#pragma unroll 1
+        for (int s = 0; s < ns; s++)  // one copy of the solve for both states
+            fe[s * nz + z] = eos.at(s ? r[1] : r[0], s ? u[1] : u[0]).p;
+        lastT[z] = zs.T;
+        nsolve = zs.nsolve;
+    }
+    add_solves(solves, nsolve);
+}
+
+// The source at pb, primtoU at pi and the flux divergence (formed here with the EMFs, or
+// S from k_div on grids beyond 32-bit offsets): the conserved vector into S.
+template <bool FUSED>
+__global__ void __launch_bounds__(TPB) k_cons_ceos(DGrid g, DivArgs dv, const double *__restrict__ pi,
+                                                   const double *__restrict__ pb, double *__restrict__ S,
+                                                   const double *__restrict__ fe, const double *__restrict__ tstate,
+                                                   double dtfac, int pi_is_pb, unsigned long long *__restrict__ cnt)
+{
+    if (halted(g)) return;
+    const size_t na = (size_t)(g.ie - g.is + 1) * (g.je - g.js + 1) * g.N3;
+    const size_t idx = (size_t)xcd_block() * TPB + threadIdx.x;
+    int fatal = 0;
+    if (idx < na) {
+        int i, j, h;
+        active_zone(g, idx, i, j, h);
         const size_t z = zidx(g, i, j, h), nz = g.nz, col = (size_t)i * g.SN2 + j;
         const double Dt = dtfac * tstate[1];
         double pbz[NPR], piz[NPR], dU[NPR], U[NPR];
 #pragma unroll
         for (int k = 0; k < NPR; k++) pbz[k] = pb[k * nz + z];
-#pragma unroll
-        for (int k = 0; k < NPR; k++) piz[k] = pi_is_pb ? pbz[k] : pi[k * nz + z];
-        CeosZone zs;
-        zs.T = lastT[z];
-        const EosCacheT<V> eos{&ce, ceos_radius(ce, i), &zs};
-        double P = 0., Ppb = 0.;
-#pragma unroll 1
-        for (int s = 0; s <= (pi_is_pb ? 0 : 1); s++) {  // one copy of the solve for both states
-            P = eos.at(s ? piz[RHO] : pbz[RHO], s ? piz[UU] : pbz[UU]).p;
-            if (s == 0) Ppb = P;
-        }
-        lastT[z] = zs.T;
-        nsolve = zs.nsolve;
-        fe[z] = P;
+        const double Ppb = fe[z], P = pi_is_pb ? Ppb : fe[nz + z];
         Geom geom;
         load_geom(g.geom[CENT], g.ncol, col, geom);
         State q;
         source(pbz, geom, g.conn, g.ncol, col, Ppb, dU, q, fatal);
+#pragma unroll
+        for (int k = 0; k < NPR; k++) piz[k] = pi_is_pb ? pbz[k] : pi[k * nz + z];
         if (!pi_is_pb) get_state(piz, geom, q, fatal);
         primtoflux_P(piz, q, 0, geom, P, U);
         double d[NPR];
@@ -1567,7 +1588,6 @@ k_cons_ceos(DGrid g, CeosParams ce, DivArgs dv, double *__restrict__ lastT, cons
         for (int k = 0; k < NPR; k++) S[k * na + idx] = U[k] + Dt * (d[k] + dU[k]);
     }
     add_counter(cnt, HARM_FATAL, fatal);
-    add_solves(solves, nsolve);
 }
 
 // Utoprim_5d of those vectors seeded with pi (no Font fix), then fixup1zone
@@ -1576,20 +1596,16 @@ template <bool V>
 __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(CEOS_WPE, 8)))
 k_update_ceos(DGrid g, CeosParams ce, double *__restrict__ lastT, const double *__restrict__ pi,
               double *__restrict__ pf, int8_t *__restrict__ pflag, const double *__restrict__ S,
-              const double *__restrict__ fe, unsigned long long *__restrict__ cpart,
+              const double *__restrict__ pe, unsigned long long *__restrict__ cpart,
               unsigned long long *__restrict__ solves)
 {
     if (halted(g)) return;
-    const int ni = g.ie - g.is + 1, nj = g.je - g.js + 1;
-    const size_t na = (size_t)ni * nj * g.N3;
+    const size_t na = (size_t)(g.ie - g.is + 1) * (g.je - g.js + 1) * g.N3;
     const size_t idx = (size_t)blockIdx.x * TPB + threadIdx.x;
     int c_call = 0, c_iter = 0, c_kconv = 0, c_f2d = 0, c_gam = 0, c_flr = 0, c_cap = 0, fatal = 0, nsolve = 0;
     if (idx < na) {
-        const unsigned rest = (unsigned)idx / (unsigned)g.N3;
-        const int h = (int)((unsigned)idx - rest * (unsigned)g.N3);
-        const unsigned ri = rest / (unsigned)nj;
-        const int j = g.js + (int)(rest - ri * (unsigned)nj);
-        const int i = g.is + (int)ri;
+        int i, j, h;
+        active_zone(g, idx, i, j, h);
         const size_t z = zidx(g, i, j, h), nz = g.nz, col = (size_t)i * g.SN2 + j;
         Geom geom;
         load_geom(g.geom[CENT], g.ncol, col, geom);
@@ -1601,11 +1617,11 @@ k_update_ceos(DGrid g, CeosParams ce, double *__restrict__ lastT, const double *
         for (int k = 0; k < NPR; k++) pr[k] = pi[k * nz + z];
 #pragma unroll
         for (int k = 0; k < NPR; k++) U[k] = S[k * na + idx];
-        // the pressure call at pi was k_cons_ceos's last: a call there repeats it
+        // the pressure call at pi was k_zone_eos's last: a call there repeats it
         zs.has = true;
         zs.kr = (unsigned long long)__double_as_longlong(pr[RHO]);
         zs.ku = (unsigned long long)__double_as_longlong(pr[UU]);
-        zs.p = fe[z];
+        zs.p = pe[z];
         int niter = 0;
         const Eos5CacheT<V> e5{eos, g.gam, g.geom[CENT], (size_t)g.ncol, col};
         const int ret = utoprim_5d(U, geom, e5, EosPt{zs.p, 0., 0.}, pr, niter);
@@ -3607,8 +3623,8 @@ int fixup_utoprim(harm_ctx *c, double *p)
 // advance() (step_ch.c:153-318) with fixup() folded into the update and the
 // Font-fix pass (step_ch.c:101-103, 112-114).  The Font-fix and seed lists it
 // fills are emptied by the next bound().
-// advance() with the cache EOS: the fluxes, the conserved vectors (k_cons_ceos), then
-// the zone update (k_update_ceos) with its fixup.
+// advance() with the cache EOS: the fluxes, the zones' pressures (k_zone_eos) and
+// conserved vectors (k_cons_ceos), then their inversion (k_update_ceos) with its fixup.
 int advance_ceos(harm_ctx *c, double *pi, double *pb, double *pf, double dtfac, int fullstep)
 {
     const DGrid &g = c->g;
@@ -3619,13 +3635,16 @@ int advance_ceos(harm_ctx *c, double *pi, double *pb, double *pf, double dtfac, 
     if ((rc = fluxes_and_emf(c, pb, fullstep, !fused))) return rc;
     if (!fused)
         LAUNCH(HARM_K_DIV, hipLaunchKernelGGL(k_div, dim3(nblocks8(na)), dim3(TPB), 0, c->stream, g, dv, c->S));
+    auto *cons = fused ? k_cons_ceos<true> : k_cons_ceos<false>;
+    const int same = (pi == pb) ? 1 : 0;
 #define CEOS_UPD(V_)                                                                                                \
     LAUNCH(HARM_K_UPDATE,                                                                                           \
-           auto *cons = fused ? k_cons_ceos<V_, true> : k_cons_ceos<V_, false>;                                     \
-           hipLaunchKernelGGL(cons, dim3(nblocks8(na)), dim3(TPB), 0, c->stream, g, c->ceos, dv, c->lastT, pi, pb,  \
-                              c->S, c->ceos_fe, c->tstate, dtfac, (pi == pb) ? 1 : 0, c->ceos_solves, c->cnt);      \
+           hipLaunchKernelGGL(k_zone_eos<V_>, dim3(nblocks(na)), dim3(TPB), 0, c->stream, g, c->ceos, c->lastT, pi, \
+                              pb, c->ceos_fe, same, c->ceos_solves);                                                \
+           hipLaunchKernelGGL(cons, dim3(nblocks8(na)), dim3(TPB), 0, c->stream, g, dv, pi, pb, c->S, c->ceos_fe,   \
+                              c->tstate, dtfac, same, c->cnt);                                                      \
            hipLaunchKernelGGL(k_update_ceos<V_>, dim3(nblocks(na)), dim3(TPB), 0, c->stream, g, c->ceos, c->lastT,  \
-                              pi, pf, c->pflag, c->S, c->ceos_fe, c->cpart, c->ceos_solves))
+                              pi, pf, c->pflag, c->S, c->ceos_fe + (same ? 0 : c->nz), c->cpart, c->ceos_solves))
     if (c->ceos_vanish)
         CEOS_UPD(true);
     else
