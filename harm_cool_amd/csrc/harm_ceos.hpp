@@ -306,11 +306,21 @@ struct EosCacheT {
 
 // The 5D inversion's view of the cache EOS (utoprim_5d.c:388-389, 454-481):
 // the pressure, then dp/drho and dp/du, each by its calls above.
-template <bool V>
+// ROWS: every lane of the wavefront is in one column, whose block tab is (load_geom_block).
+template <bool ROWS>
+__device__ __forceinline__ void ceos_metric(const double *tab, size_t ncol, size_t col, Geom &g)
+{
+    if (ROWS)
+        load_geom_block<CENT_DERIVED>(tab, g);
+    else
+        load_geom(tab, ncol, col, g);
+}
+
+template <bool V, bool ROWS>
 struct Eos5CacheT {
     EosCacheT<V> e;
     double gam;
-    const double *tab;  // the zone's metric (load_geom)
+    const double *tab;  // the zone's metric (ceos_metric)
     size_t ncol, col;
     __device__ static constexpr bool tabulated() { return true; }
     // The lanes of a wavefront share one or two columns, so the metric's 40 numbers are a
@@ -319,7 +329,7 @@ struct Eos5CacheT {
     {
         const double *p = tab;
         asm volatile("" : "+s"(p));  // a new value to the compiler, which would keep the old loads'
-        load_geom(p, ncol, col, g);
+        ceos_metric<ROWS>(p, ncol, col, g);
     }
     __device__ EosPt at(double rho, double u) const { return e.at(rho, u); }
     __device__ void derivs(double rho, double u, EosPt &pt) const

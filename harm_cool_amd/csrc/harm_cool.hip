@@ -1366,19 +1366,33 @@ __device__ __forceinline__ void ceos_stencil(const DGrid &g, size_t z, int h, si
     }
 }
 
+// Phi rows of a launch that takes the metric as wave-uniform (ROWS): padded to whole
+// wavefronts, so that every wavefront's lanes share one (i, j) column and read it through
+// the scalar unit.  k_cons_ceos, which waits for the metric's and the connection's 104
+// numbers, gains by that with idle lanes too (96 of 128 lanes: 184 -> 108 us at 96^3) and
+// takes it where at least 60% of the lanes are zones (ceos_rows); the fluxes (64 -> 70 us)
+// and the inversion (374 -> 435 us) only lose the lanes and take it on grids without any.
+__host__ __device__ inline unsigned ceos_row(int n3, bool rows)
+{
+    return rows ? ((unsigned)n3 + 63u) & ~63u : (unsigned)n3;
+}
+inline bool ceos_rows(int n3) { return (size_t)n3 * 5 >= (size_t)ceos_row(n3, true) * 3; }
+
 // The face range of a sweep along DIR (k_flux's) and, with chain, one (h, i)
 // column per thread walked in j order; calls f(i, j, h) per face.
-template <int DIR, class Fn>
+template <int DIR, bool ROWS = false, class Fn>
 __device__ __forceinline__ void ceos_faces(const DGrid &g, int chain, Fn &&f)
 {
     const int i0 = (DIR == 1) ? g.is : g.is - 1;
     const int j0 = (DIR == 2) ? g.js : g.js - 1;
     const int ni = g.ie + 1 - i0 + 1, nj = g.je + 1 - j0 + 1;
+    const size_t np = ceos_row(g.N3, ROWS);
     const size_t idx = (size_t)blockIdx.x * TPB + threadIdx.x;
-    const size_t n = chain ? (size_t)ni * g.N3 : (size_t)ni * nj * g.N3;
+    const size_t n = chain ? (size_t)ni * np : (size_t)ni * nj * np;
     if (idx >= n) return;
-    const int h = (int)(idx % (size_t)g.N3);
-    const size_t rest = idx / (size_t)g.N3;
+    const int h = (int)(idx % np);
+    if (ROWS && h >= g.N3) return;
+    const size_t rest = idx / np;
     const int i = chain ? i0 + (int)rest : i0 + (int)(rest / (size_t)nj);
     const int ja = chain ? j0 : j0 + (int)(rest % (size_t)nj), jb = chain ? g.je + 1 : ja;
     for (int j = ja; j <= jb; j++) f(i, j, h);
@@ -1451,8 +1465,8 @@ struct EosGiven {
 // fluxcalc (step_ch.c:331-504) with the face pressures k_face_eos formed:
 // slopes from four zones along DIR (MC / van Leer / minmod), fix_flux
 // (coord.c:264-324) and the CFL limit, as k_flux.  One face per thread.
-template <int DIR>
-__global__ void __launch_bounds__(TPB) k_flux_ceos(DGrid g, const double *__restrict__ fe,
+template <int DIR, bool ROWS>
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(ROWS ? 4 : 3, 8))) k_flux_ceos(DGrid g, const double *__restrict__ fe,
                                                    const double *__restrict__ pb, double *__restrict__ F,
                                                    double *__restrict__ dtpart, int fullstep,
                                                    unsigned long long *__restrict__ cnt)
@@ -1460,7 +1474,7 @@ __global__ void __launch_bounds__(TPB) k_flux_ceos(DGrid g, const double *__rest
     if (halted(g)) return;
     double dtij = 1.e300;
     int fatal = 0;
-    ceos_faces<DIR>(g, 0, [&](int i, int j, int h) {
+    ceos_faces<DIR, ROWS>(g, 0, [&](int i, int j, int h) {
         const size_t nz = g.nz, z = zidx(g, i, j, h);
         if (DIR == 2 && (j == g.js || j == g.je + 1)) {
 #pragma unroll
@@ -1478,7 +1492,10 @@ __global__ void __launch_bounds__(TPB) k_flux_ceos(DGrid g, const double *__rest
         }
         Geom geom;
         const int loc = (DIR == 1) ? FACE1 : (DIR == 2) ? FACE2 : FACE3;
-        load_geom(g.geom[loc], g.ncol, (size_t)i * g.SN2 + j, geom);
+        if (ROWS)
+            load_geom_block<FACE_DERIVED>(g.fblk[DIR - 1] + uni_col<true>((size_t)i * g.SN2 + j) * FACE_STRIDE, geom);
+        else
+            load_geom(g.geom[loc], g.ncol, (size_t)i * g.SN2 + j, geom);
         const EosGiven eos{p_l[RHO], p_l[UU], fe[0 * nz + z], fe[1 * nz + z], fe[2 * nz + z], fe[3 * nz + z]};
         double Fz[NPR], ctop;
         face_flux(p_l, p_r, geom, DIR, eos, g.hllf, g.laxf, Fz, ctop, fatal);
@@ -1507,17 +1524,20 @@ __global__ void __launch_bounds__(TPB) k_flux_ceos(DGrid g, const double *__rest
 // advance()'s zone loop with COOL_EOS (step_ch.c:237-306) in three kernels: the solves,
 // which wait for a chain of reads each, want wavefronts, the rest registers (one kernel
 // for all held 256 and spilled 131, 1.5 KB of scratch traffic a zone; 96^3 zones: 870 us,
-// now 615).
+// now 530).
 
-// Active zone idx of a grid-order launch.
-__device__ __forceinline__ void active_zone(const DGrid &g, size_t idx, int &i, int &j, int &h)
+// Thread idx's active zone and its index among them, false where it has none.
+template <bool ROWS>
+__device__ __forceinline__ bool active_zone(const DGrid &g, size_t idx, int &i, int &j, int &h, size_t &at)
 {
-    const unsigned nj = (unsigned)(g.je - g.js + 1);
-    const unsigned rest = (unsigned)idx / (unsigned)g.N3;
-    h = (int)((unsigned)idx - rest * (unsigned)g.N3);
+    const unsigned nj = (unsigned)(g.je - g.js + 1), np = ceos_row(g.N3, ROWS);
+    const unsigned rest = (unsigned)(idx / np);
+    h = (int)(idx - (size_t)rest * np);
     const unsigned ri = rest / nj;
     j = g.js + (int)(rest - ri * nj);
     i = g.is + (int)ri;
+    at = (size_t)rest * g.N3 + h;
+    return i <= g.ie && h < g.N3;
 }
 
 // InitCache_CoolEOS and the pressures at pb (into fe[0]) and at pi (fe[1]).
@@ -1527,12 +1547,10 @@ k_zone_eos(DGrid g, CeosParams ce, double *__restrict__ lastT, const double *__r
            const double *__restrict__ pb, double *__restrict__ fe, int pi_is_pb, unsigned long long *__restrict__ solves)
 {
     if (halted(g)) return;
-    const size_t na = (size_t)(g.ie - g.is + 1) * (g.je - g.js + 1) * g.N3;
     const size_t idx = (size_t)blockIdx.x * TPB + threadIdx.x;
-    int nsolve = 0;
-    if (idx < na) {
-        int i, j, h;
-        active_zone(g, idx, i, j, h);
+    int nsolve = 0, i, j, h;
+    size_t at;
+    if (active_zone<false>(g, idx, i, j, h, at)) {
         const size_t z = zidx(g, i, j, h), nz = g.nz;
         const double r[2] = {pb[RHO * nz + z], pi[RHO * nz + z]}, u[2] = {pb[UU * nz + z], pi[UU * nz + z]};
         CeosZone zs;
@@ -1550,7 +1568,7 @@ k_zone_eos(DGrid g, CeosParams ce, double *__restrict__ lastT, const double *__r
 
 // The source at pb, primtoU at pi and the flux divergence (formed here with the EMFs, or
 // S from k_div on grids beyond 32-bit offsets): the conserved vector into S.
-template <bool FUSED>
+template <bool FUSED, bool ROWS>
 __global__ void __launch_bounds__(TPB) k_cons_ceos(DGrid g, DivArgs dv, const double *__restrict__ pi,
                                                    const double *__restrict__ pb, double *__restrict__ S,
                                                    const double *__restrict__ fe, const double *__restrict__ tstate,
@@ -1559,10 +1577,9 @@ __global__ void __launch_bounds__(TPB) k_cons_ceos(DGrid g, DivArgs dv, const do
     if (halted(g)) return;
     const size_t na = (size_t)(g.ie - g.is + 1) * (g.je - g.js + 1) * g.N3;
     const size_t idx = (size_t)xcd_block() * TPB + threadIdx.x;
-    int fatal = 0;
-    if (idx < na) {
-        int i, j, h;
-        active_zone(g, idx, i, j, h);
+    int fatal = 0, i, j, h;
+    size_t at;
+    if (active_zone<ROWS>(g, idx, i, j, h, at)) {
         const size_t z = zidx(g, i, j, h), nz = g.nz, col = (size_t)i * g.SN2 + j;
         const double Dt = dtfac * tstate[1];
         double pbz[NPR], piz[NPR], dU[NPR], U[NPR];
@@ -1570,9 +1587,15 @@ __global__ void __launch_bounds__(TPB) k_cons_ceos(DGrid g, DivArgs dv, const do
         for (int k = 0; k < NPR; k++) pbz[k] = pb[k * nz + z];
         const double Ppb = fe[z], P = pi_is_pb ? Ppb : fe[nz + z];
         Geom geom;
-        load_geom(g.geom[CENT], g.ncol, col, geom);
         State q;
-        source(pbz, geom, g.conn, g.ncol, col, Ppb, dU, q, fatal);
+        if (ROWS) {
+            const double *blk = g.cblk + uni_col<true>(col) * CENT_STRIDE;
+            load_geom_block<CENT_DERIVED>(blk, geom);
+            source(pbz, geom, blk + CENT_CONN, 1, 0, Ppb, dU, q, fatal);
+        } else {
+            load_geom(g.geom[CENT], g.ncol, col, geom);
+            source(pbz, geom, g.conn, g.ncol, col, Ppb, dU, q, fatal);
+        }
 #pragma unroll
         for (int k = 0; k < NPR; k++) piz[k] = pi_is_pb ? pbz[k] : pi[k * nz + z];
         if (!pi_is_pb) get_state(piz, geom, q, fatal);
@@ -1582,17 +1605,17 @@ __global__ void __launch_bounds__(TPB) k_cons_ceos(DGrid g, DivArgs dv, const do
             flux_div32<false>(g, dv, i, j, h, d);
         } else {
 #pragma unroll
-            for (int k = 0; k < NPR; k++) d[k] = S[k * na + idx];
+            for (int k = 0; k < NPR; k++) d[k] = S[k * na + at];
         }
 #pragma unroll
-        for (int k = 0; k < NPR; k++) S[k * na + idx] = U[k] + Dt * (d[k] + dU[k]);
+        for (int k = 0; k < NPR; k++) S[k * na + at] = U[k] + Dt * (d[k] + dU[k]);
     }
     add_counter(cnt, HARM_FATAL, fatal);
 }
 
 // Utoprim_5d of those vectors seeded with pi (no Font fix), then fixup1zone
 // (fixup.c:51-60).
-template <bool V>
+template <bool V, bool ROWS>
 __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(CEOS_WPE, 8)))
 k_update_ceos(DGrid g, CeosParams ce, double *__restrict__ lastT, const double *__restrict__ pi,
               double *__restrict__ pf, int8_t *__restrict__ pflag, const double *__restrict__ S,
@@ -1603,12 +1626,13 @@ k_update_ceos(DGrid g, CeosParams ce, double *__restrict__ lastT, const double *
     const size_t na = (size_t)(g.ie - g.is + 1) * (g.je - g.js + 1) * g.N3;
     const size_t idx = (size_t)blockIdx.x * TPB + threadIdx.x;
     int c_call = 0, c_iter = 0, c_kconv = 0, c_f2d = 0, c_gam = 0, c_flr = 0, c_cap = 0, fatal = 0, nsolve = 0;
-    if (idx < na) {
-        int i, j, h;
-        active_zone(g, idx, i, j, h);
-        const size_t z = zidx(g, i, j, h), nz = g.nz, col = (size_t)i * g.SN2 + j;
+    int i, j, h;
+    size_t at;
+    if (active_zone<ROWS>(g, idx, i, j, h, at)) {
+        const size_t z = zidx(g, i, j, h), nz = g.nz, col = uni_col<ROWS>((size_t)i * g.SN2 + j);
+        const double *tab = ROWS ? g.cblk + col * CENT_STRIDE : g.geom[CENT];
         Geom geom;
-        load_geom(g.geom[CENT], g.ncol, col, geom);
+        ceos_metric<ROWS>(tab, g.ncol, col, geom);
         CeosZone zs;
         zs.T = lastT[z];
         const EosCacheT<V> eos{&ce, ceos_radius(ce, i), &zs};
@@ -1616,14 +1640,14 @@ k_update_ceos(DGrid g, CeosParams ce, double *__restrict__ lastT, const double *
 #pragma unroll
         for (int k = 0; k < NPR; k++) pr[k] = pi[k * nz + z];
 #pragma unroll
-        for (int k = 0; k < NPR; k++) U[k] = S[k * na + idx];
+        for (int k = 0; k < NPR; k++) U[k] = S[k * na + at];
         // the pressure call at pi was k_zone_eos's last: a call there repeats it
         zs.has = true;
         zs.kr = (unsigned long long)__double_as_longlong(pr[RHO]);
         zs.ku = (unsigned long long)__double_as_longlong(pr[UU]);
         zs.p = pe[z];
         int niter = 0;
-        const Eos5CacheT<V> e5{eos, g.gam, g.geom[CENT], (size_t)g.ncol, col};
+        const Eos5CacheT<V, ROWS> e5{eos, g.gam, tab, (size_t)g.ncol, col};
         const int ret = utoprim_5d(U, geom, e5, EosPt{zs.p, 0., 0.}, pr, niter);
         lastT[z] = zs.T;
         nsolve = zs.nsolve;
@@ -3529,13 +3553,15 @@ int flux_launch(harm_ctx *c, int dir, const double *pb, double *F, int fullstep)
         const int chain = c->ceos_chain[dir - 1] ? 1 : 0;
         const size_t nc = (size_t)(g.ie + 2 - i0) * g.N3;
         const dim3 ge(nblocks(chain ? nc : total));
+        const bool rows = c->uniform;
         grid = dim3(nblocks(total));
 #define CEOS_FLUX(D_, K_)                                                                                          \
     LAUNCH(K_, if (c->ceos_vanish) hipLaunchKernelGGL((k_face_eos<D_, true>), ge, dim3(TPB), 0, c->stream, g, c->ceos, \
                                                       c->lastT, pb, c->ceos_fe, chain, c->ceos_solves);            \
                else hipLaunchKernelGGL((k_face_eos<D_, false>), ge, dim3(TPB), 0, c->stream, g, c->ceos, c->lastT, pb, \
                                        c->ceos_fe, chain, c->ceos_solves);                                         \
-           hipLaunchKernelGGL(k_flux_ceos<D_>, grid, dim3(TPB), 0, c->stream, g, c->ceos_fe, pb, F,                \
+           auto *kf = rows ? k_flux_ceos<D_, true> : k_flux_ceos<D_, false>;                                        \
+           hipLaunchKernelGGL(kf, grid, dim3(TPB), 0, c->stream, g, c->ceos_fe, pb, F,                              \
                               c->dtpart + (D_ - 1) * c->dtstride, fullstep, c->cnt))
         if (dir == 1)
             CEOS_FLUX(1, HARM_K_FLUX1);
@@ -3635,15 +3661,19 @@ int advance_ceos(harm_ctx *c, double *pi, double *pb, double *pf, double dtfac, 
     if ((rc = fluxes_and_emf(c, pb, fullstep, !fused))) return rc;
     if (!fused)
         LAUNCH(HARM_K_DIV, hipLaunchKernelGGL(k_div, dim3(nblocks8(na)), dim3(TPB), 0, c->stream, g, dv, c->S));
-    auto *cons = fused ? k_cons_ceos<true> : k_cons_ceos<false>;
+    const bool rows = ceos_rows(g.N3);  // k_cons_ceos's
+    const size_t nt = na / (size_t)g.N3 * ceos_row(g.N3, rows);
+    auto *cons = fused ? (rows ? k_cons_ceos<true, true> : k_cons_ceos<true, false>)
+                       : (rows ? k_cons_ceos<false, true> : k_cons_ceos<false, false>);
     const int same = (pi == pb) ? 1 : 0;
 #define CEOS_UPD(V_)                                                                                                \
     LAUNCH(HARM_K_UPDATE,                                                                                           \
            hipLaunchKernelGGL(k_zone_eos<V_>, dim3(nblocks(na)), dim3(TPB), 0, c->stream, g, c->ceos, c->lastT, pi, \
                               pb, c->ceos_fe, same, c->ceos_solves);                                                \
-           hipLaunchKernelGGL(cons, dim3(nblocks8(na)), dim3(TPB), 0, c->stream, g, dv, pi, pb, c->S, c->ceos_fe,   \
+           hipLaunchKernelGGL(cons, dim3(nblocks8(nt)), dim3(TPB), 0, c->stream, g, dv, pi, pb, c->S, c->ceos_fe,   \
                               c->tstate, dtfac, same, c->cnt);                                                      \
-           hipLaunchKernelGGL(k_update_ceos<V_>, dim3(nblocks(na)), dim3(TPB), 0, c->stream, g, c->ceos, c->lastT,  \
+           auto *upd = c->uniform ? k_update_ceos<V_, true> : k_update_ceos<V_, false>;                             \
+           hipLaunchKernelGGL(upd, dim3(nblocks(na)), dim3(TPB), 0, c->stream, g, c->ceos, c->lastT,  \
                               pi, pf, c->pflag, c->S, c->ceos_fe + (same ? 0 : c->nz), c->cpart, c->ceos_solves))
     if (c->ceos_vanish)
         CEOS_UPD(true);
