@@ -2233,10 +2233,11 @@ __device__ __forceinline__ void step_end(const DGrid &g, double *tstate, unsigne
 
 // The end of a step: blocks [0, N3) the mass fluxes of a phi plane each, the others the
 // CFL minima; the last block to finish adds the planes in order and closes the step.
-// done: the count of finished blocks, 0 between launches.
+// done: the count of finished blocks, 0 between launches.  hstat: host memory that takes
+// the words harm_step looks at after a batch, which copied them (25 us of a small step).
 __global__ void __launch_bounds__(TPB) k_stepend(DGrid g, const double *__restrict__ p, double *part, MinArgs mins,
                                                  unsigned *done, double *tstate, unsigned long long *ndt_slot,
-                                                 const unsigned long long *cnt)
+                                                 const unsigned long long *cnt, const int *fix_err, double *hstat)
 {
     if (halted(g)) return;
     if (blockIdx.x < (unsigned)g.N3)
@@ -2273,6 +2274,8 @@ __global__ void __launch_bounds__(TPB) k_stepend(DGrid g, const double *__restri
     if (threadIdx.x != 0) return;
     *done = 0;
     step_end(g, tstate, ndt_slot, mdot_in, mdot_out, cnt);
+    hstat[0] = tstate[4];
+    hstat[1] = (double)*fix_err;
 }
 
 // ---------------------------------------------------------------------------
@@ -3339,6 +3342,7 @@ struct harm_ctx {
     unsigned dt_nb[3];                // blocks of the last full-step flux launch of each direction
     unsigned sum_nb;                  // blocks of the last zone update whose counters are not folded yet
     unsigned *step_done;              // k_stepend's finished blocks
+    double *hstat;                    // host memory: the halt code and fix_err after the last step
     unsigned long long *cpart;        // per-block counter totals of one update launch
     unsigned long long *cnt;          // HARM_NCOUNTERS
     double *part;                     // reduction partials
@@ -3811,7 +3815,7 @@ int one_step(harm_ctx *c)
     }
     LAUNCH(HARM_K_STEPEND,
            hipLaunchKernelGGL(k_stepend, dim3(g.N3 + (g.N3 > 2 ? 3 : 2) * RED_BLOCKS), dim3(TPB), 0, c->stream, g, c->p,
-                              c->part, min_args(c), c->step_done, c->tstate, c->ndt_slot, c->cnt));
+                              c->part, min_args(c), c->step_done, c->tstate, c->ndt_slot, c->cnt, c->fix_err, c->hstat));
     return 0;
 }
 
@@ -3822,6 +3826,16 @@ const char *halt_message(int code)
                         "stopped after that step";
 }
 
+int flags_error(harm_ctx *c, double halt, int fe)
+{
+    if (halt == 11. || halt == 14.) {
+        c->halted = (int)halt;
+        return set_err(halt_message(c->halted), c->halted);
+    }
+    if (fe & 1) return set_err("more failed inversions in one half-step than the Font-fix list holds", 13);
+    return 0;
+}
+
 int check_flags(harm_ctx *c)
 {
     double ts[5];
@@ -3829,12 +3843,7 @@ int check_flags(harm_ctx *c)
     HIPCHK(hipMemcpyAsync(ts, c->tstate, sizeof(ts), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipMemcpyAsync(&fe, c->fix_err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
-    if (ts[4] == 11. || ts[4] == 14.) {
-        c->halted = (int)ts[4];
-        return set_err(halt_message(c->halted), c->halted);
-    }
-    if (fe & 1) return set_err("more failed inversions in one half-step than the Font-fix list holds", 13);
-    return 0;
+    return flags_error(c, ts[4], fe);
 }
 
 // Clears a stopped batch's error (the caller resets the clock or the state).
@@ -3932,6 +3941,8 @@ int ctx_alloc(harm_ctx *c)
     c->dtstride = nblocks8(c->nz);
     if ((rc = dalloc(&c->dtpart, 3 * c->dtstride))) return rc;
     if ((rc = dalloc(&c->step_done, 1))) return rc;
+    HIPCHK(hipHostMalloc((void **)&c->hstat, 2 * sizeof(double), hipHostMallocMapped));
+    c->hstat[0] = c->hstat[1] = 0.;
     if ((rc = dalloc(&c->cpart, 8 * (size_t)nblocks(c->nz)))) return rc;
     if ((rc = dalloc(&c->cnt, HARM_NCOUNTERS))) return rc;
     c->npart = std::max<size_t>(DIAG_NPART * nblocks(c->nz) + 16, 2 * (size_t)hg.N3 + 16);
@@ -4000,6 +4011,7 @@ void ctx_free(harm_ctx *c)
                     (void *)c->seeds.U, (void *)c->lastT, (void *)c->ceos_vals, (void *)c->ceos_solves,
                     (void *)c->ceos_tab, (void *)c->ceos_fe, (void *)c->ceos_hint})
         if (q) (void)hipFree(q);
+    if (c->hstat) (void)hipHostFree(c->hstat);
     for (double *q : c->ceos_tabs) (void)hipFree(q);
     for (int l = 0; l < 5; l++)
         if (c->d_geom[l]) (void)hipFree(c->d_geom[l]);
@@ -4220,7 +4232,8 @@ int harm_step(harm_ctx *c, int nsteps)
     }
     int rc = ev_collect(c);
     if (rc) return rc;
-    return check_flags(c);
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return flags_error(c, c->hstat[0], (int)c->hstat[1]);  // written by every k_stepend up to one that halts
 }
 
 int harm_get_prims(harm_ctx *c, double *prim, int8_t *pflag) { return c ? copy_state(c, prim, pflag, true) : 1; }
