@@ -1896,10 +1896,15 @@ __device__ __forceinline__ size_t bound_nthreads(const DGrid &g)
 
 __global__ void __launch_bounds__(TPB) k_bound(DGrid g, double *__restrict__ p, int8_t *__restrict__ pflag,
                                                int *__restrict__ font_count, int *__restrict__ seed_count,
-                                               unsigned nbound, SumArgs sum, unsigned long long *__restrict__ cnt)
+                                               unsigned nbound, SumArgs sum, unsigned *redo, unsigned epoch, bool again,
+                                               unsigned long long *__restrict__ cnt)
 {
     static_assert(TPB == 256, "fold_counts takes blocks of 256 threads");
     if (halted(g)) return;
+    // The pass after fixup_utoprim() forms every value again from zones that it left alone
+    // where that found no flag and this half-step's first pass no failure (redo is not its
+    // epoch): the same bits, so nothing is done (27 us a pass on 288x256x256).
+    if (again && *redo != epoch) return;
     if (blockIdx.x >= nbound) {  // the zone update's counters
         fold_counts(sum, blockIdx.x - nbound, cnt);
         return;
@@ -1961,6 +1966,7 @@ __global__ void __launch_bounds__(TPB) k_bound(DGrid g, double *__restrict__ p, 
             pflag[z] = fl;
         }
     }
+    if (fatal) *redo = epoch;
     add_counter(cnt, HARM_FATAL, fatal);
 }
 
@@ -2028,8 +2034,8 @@ constexpr int SCAN_ZONES = 32;
 __global__ void __launch_bounds__(TPB) k_fixutoprim_scan(DGrid g, double *__restrict__ p,
                                                          const int8_t *__restrict__ fin, int8_t *__restrict__ fout,
                                                          unsigned long long *__restrict__ bits,
-                                                         int *__restrict__ pcount, unsigned nwords,
-                                                         unsigned long long *__restrict__ cnt)
+                                                         int *__restrict__ pcount, unsigned nwords, unsigned *redo,
+                                                         unsigned epoch, unsigned long long *__restrict__ cnt)
 {
     if (halted(g)) return;
     // 32 zones per thread: the common all-good octet is an 8-byte load and store, and a
@@ -2037,7 +2043,7 @@ __global__ void __launch_bounds__(TPB) k_fixutoprim_scan(DGrid g, double *__rest
     // with every counter's wave sum: 30 us on 288x256x256, now 14 us).
     const size_t t0 = ((size_t)blockIdx.x * TPB + threadIdx.x) * SCAN_ZONES;
     int c_rep = 0, c_nost = 0, c_flr = 0, c_cap = 0, c_gam = 0, fatal = 0;
-    bool bad = false;
+    bool bad = false;  // a flag is set
     unsigned long long f8[SCAN_ZONES / 8];
 #pragma unroll
     for (int o = 0; o < SCAN_ZONES / 8; o++) {
@@ -2051,7 +2057,6 @@ __global__ void __launch_bounds__(TPB) k_fixutoprim_scan(DGrid g, double *__rest
             *reinterpret_cast<unsigned long long *>(fout + z0) = 0x0101010101010101ull;
             continue;
         }
-        bad = true;
         for (int q = 0; q < 8; q++) {
             const size_t idx = z0 + q;
             if (idx >= g.nz) break;
@@ -2061,6 +2066,7 @@ __global__ void __launch_bounds__(TPB) k_fixutoprim_scan(DGrid g, double *__rest
             const int j = (int)(col - ci * (unsigned)g.SN2), i = (int)ci;
             const int8_t f = fin[idx];
             fout[idx] = (int8_t)(!f);
+            bad |= f != 0;
             if (f != 0 && i >= g.is && i <= g.ie && j >= g.js && j <= g.je) {
                 bool isolated = true;
                 for (int di = -1; di <= 1; di++)
@@ -2076,6 +2082,7 @@ __global__ void __launch_bounds__(TPB) k_fixutoprim_scan(DGrid g, double *__rest
         }
     }
     if (!__any(bad)) return;
+    if (bad) *redo = epoch;
     add_counter(cnt, HARM_FIXUP_REPAIRS, c_rep);
     add_counter(cnt, HARM_FIXUP_NOSTENCIL, c_nost);
     add_counter(cnt, HARM_FLOOR_ZONES, c_flr);
@@ -3342,6 +3349,7 @@ struct harm_ctx {
     unsigned dt_nb[3];                // blocks of the last full-step flux launch of each direction
     unsigned sum_nb;                  // blocks of the last zone update whose counters are not folded yet
     unsigned *step_done;              // k_stepend's finished blocks
+    unsigned *redo, epoch;            // the half-step that needs its second bound(), the present one
     double *hstat;                    // host memory: the halt code and fix_err after the last step
     unsigned long long *cpart;        // per-block counter totals of one update launch
     unsigned long long *cnt;          // HARM_NCOUNTERS
@@ -3627,13 +3635,15 @@ int fluxes_and_emf(harm_ctx *c, const double *pb, int fullstep, bool emf = true)
     return 0;
 }
 
-int bound(harm_ctx *c, double *p)
+// again: the pass after fixup_utoprim() of the same half-step (k_bound).
+int bound(harm_ctx *c, double *p, bool again = false)
 {
     const DGrid &g = c->g;
     const size_t nb = ((size_t)4 * g.SN2 + (size_t)g.N1 * (4 + 2 * g.polefix)) * g.N3;
     const unsigned nbl = nblocks(nb);
     LAUNCH(HARM_K_BOUND, hipLaunchKernelGGL(k_bound, dim3(nbl + 8 * fold_blocks(c->sum_nb)), dim3(TPB), 0, c->stream, g,
-                                            p, c->pflag, c->font.count, c->seeds.count, nbl, sum_args(c), c->cnt));
+                                            p, c->pflag, c->font.count, c->seeds.count, nbl, sum_args(c), c->redo, c->epoch, again,
+                                            c->cnt));
     c->sum_nb = 0;
     return 0;
 }
@@ -3643,7 +3653,7 @@ int fixup_utoprim(harm_ctx *c, double *p)
     const DGrid &g = c->g;
     LAUNCH(HARM_K_FIXUTOPRIM,
            hipLaunchKernelGGL(k_fixutoprim_scan, dim3(nblocks((g.nz + SCAN_ZONES - 1) / SCAN_ZONES)), dim3(TPB), 0, c->stream, g, p, c->pflag,
-                              c->pflag2, c->fix_bits, c->fix_pcount, c->fix_nwords, c->cnt);
+                              c->pflag2, c->fix_bits, c->fix_pcount, c->fix_nwords, c->redo, c->epoch, c->cnt);
            hipLaunchKernelGGL(k_fixutoprim_serial, dim3(g.N3), dim3(64), 0, c->stream, g, p, c->pflag2, c->fix_bits,
                               c->fix_pcount, c->fix_nwords, c->cnt));
     std::swap(c->pflag, c->pflag2);
@@ -3791,10 +3801,10 @@ int half_step(harm_ctx *c, double *pi, double *pb, double *pf, double dtfac, int
 {
     int rc;
     if ((rc = advance(c, pi, pb, pf, dtfac, fullstep))) return rc;
+    c->epoch++;
     if ((rc = bound(c, pf))) return rc;
     if ((rc = fixup_utoprim(c, pf))) return rc;
-    if ((rc = bound(c, pf))) return rc;
-    return 0;
+    return bound(c, pf, true);
 }
 
 int one_step(harm_ctx *c)
@@ -3940,7 +3950,7 @@ int ctx_alloc(harm_ctx *c)
     if ((rc = dalloc(&c->ndt_slot, 3))) return rc;
     c->dtstride = nblocks8(c->nz);
     if ((rc = dalloc(&c->dtpart, 3 * c->dtstride))) return rc;
-    if ((rc = dalloc(&c->step_done, 1))) return rc;
+    if ((rc = dalloc(&c->step_done, 1)) || (rc = dalloc(&c->redo, 1))) return rc;
     HIPCHK(hipHostMalloc((void **)&c->hstat, 2 * sizeof(double), hipHostMallocMapped));
     c->hstat[0] = c->hstat[1] = 0.;
     if ((rc = dalloc(&c->cpart, 8 * (size_t)nblocks(c->nz)))) return rc;
@@ -4005,7 +4015,7 @@ void ctx_free(harm_ctx *c)
 {
     for (void *q : {(void *)c->p, (void *)c->ph, (void *)c->F1, (void *)c->F2, (void *)c->F3, (void *)c->e1,
                     (void *)c->e2, (void *)c->e3, (void *)c->S, (void *)c->pflag, (void *)c->pflag2, (void *)c->d_conn,
-                    (void *)c->d_floors, (void *)c->d_katm, (void *)c->tstate, (void *)c->ndt_slot, (void *)c->dtpart, (void *)c->step_done, (void *)c->cpart, (void *)c->cnt,
+                    (void *)c->d_floors, (void *)c->d_katm, (void *)c->tstate, (void *)c->ndt_slot, (void *)c->dtpart, (void *)c->step_done, (void *)c->redo, (void *)c->cpart, (void *)c->cnt,
                     (void *)c->part, (void *)c->fix_bits, (void *)c->fix_pcount, (void *)c->fix_err, (void *)c->font.count, (void *)c->font.zone, (void *)c->font.U,
                     (void *)c->d_cblk, (void *)c->d_fblk, (void *)c->seeds.count, (void *)c->seeds.zone,
                     (void *)c->seeds.U, (void *)c->lastT, (void *)c->ceos_vals, (void *)c->ceos_solves,
