@@ -139,7 +139,7 @@ __device__ __forceinline__ int gamma_calc_g5(const double *pr, const Geom &g, do
         if (fabs(utsq) > 1.E-10) bad = 1;
         utsq = fabs(utsq);
     }
-    gamma = sqrt(1. + utsq);
+    gamma = fsqrt(1. + utsq);
     return bad;
 }
 
@@ -159,7 +159,7 @@ __device__ inline void lu5_solve(double (&A)[N5][N5], double (&B)[N5])
 #pragma unroll
         for (int j = 0; j < n; j++) absmax = fmax(absmax, fabs(A[i][j]));
         zero |= absmax == 0.;
-        row_norm[i] = 1. / absmax;
+        row_norm[i] = fdiv(1., absmax);
     }
     if (zero) {
         // the reference returns before factorizing and then substitutes with the
@@ -210,7 +210,7 @@ __device__ inline void lu5_solve(double (&A)[N5][N5], double (&B)[N5])
             }
             if (A[j][j] == 0.) A[j][j] = absmin;
             if (j != (n - 1)) {
-                const double inv = 1. / A[j][j];
+                const double inv = fdiv(1., A[j][j]);
 #pragma unroll
                 for (int i = j + 1; i < n; i++) A[i][j] *= inv;
             }
@@ -224,7 +224,7 @@ __device__ inline void lu5_solve(double (&A)[N5][N5], double (&B)[N5])
     for (int i = n - 1; i >= 0; i--) {
 #pragma unroll
         for (int j = i + 1; j < n; j++) B[i] -= A[i][j] * B[j];
-        B[i] /= A[i][i];
+        B[i] = fdiv(B[i], A[i][i]);
     }
 }
 
@@ -245,7 +245,7 @@ __device__ inline void func_5d(const E5 &eos, const double *U_target, const Geom
         for (int i = 1; i < 4; i++)
 #pragma unroll
             for (int j = 1; j < 4; j++) utsq += g.gcov[i][j] * x[UU + i] * x[UU + j];
-        const double gamma = sqrt(1. + fabs(utsq));
+        const double gamma = fsqrt(1. + fabs(utsq));
         const double lg = z.lapse * gamma;
         ucon[0] = 0. - lg * g.gcon[0][0];
 #pragma unroll
@@ -261,7 +261,7 @@ __device__ inline void func_5d(const E5 &eos, const double *U_target, const Geom
             Bn[i] = z.lapse * Bf[i - 1];
             u_dot_B += ucov[i] * Bn[i];
         }
-        const double rgb = 1. / gb;
+        const double rgb = fdiv(1., gb);
 #pragma unroll
         for (int i = 0; i < 4; i++) bcon[i] = div_r(Bn[i] + ucon[i] * u_dot_B, gb, rgb);
     }
@@ -285,13 +285,13 @@ __device__ inline void func_5d(const E5 &eos, const double *U_target, const Geom
             const double u = Uc[k] * g.g;
             resid[k] = u - U_target[k];
             double residnorm = 0.5 * (fabs(u) + fabs(U_target[k]));
-            residnorm = (residnorm == 0.) ? 1. : 1. / residnorm;
+            residnorm = (residnorm == 0.) ? 1. : fdiv(1., residnorm);
             df -= residnorm * resid[k] * resid[k];
         }
     }
     f = -0.5 * df;
 
-    const double ru = 1. / ucon[0], rut = 1. / ucov[0];
+    const double ru = fdiv(1., ucon[0]), rut = fdiv(1., ucov[0]);
     const double bu = div_r(bcon[0], ucon[0], ru);
     Bcov[0] = 0.;
 #pragma unroll
@@ -360,7 +360,7 @@ __device__ inline void func_5d(const E5 &eos, const double *U_target, const Geom
     {
         double gamma;
         gamma_calc_g5(x, g, gamma);
-        const double ig = 1.0 / gamma;
+        const double ig = fdiv(1.0, gamma);
 #pragma unroll
         for (int j = 1; j < 4; j++) {
             dg[j] = ig * g.gcov[j][1] * x[U1];
@@ -395,7 +395,7 @@ __device__ inline void func_5d(const E5 &eos, const double *U_target, const Geom
                 norm += fabs(Am[j][k]);
                 numnormterms++;
             }
-    norm = ((double)(numnormterms)) / (norm);
+    norm = fdiv((double)(numnormterms), norm);
 #pragma unroll
     for (int j = 0; j < N5; j++)
 #pragma unroll
@@ -439,7 +439,7 @@ __device__ inline int utoprim_5d(const double *U, Geom &g, const E5 &eos, EosPt 
             W = gsqtmp * (x[UU] + x[RHO] + e.p);
         else
             W = gsqtmp * (eos.gam * x[UU] + x[RHO]);
-        errx = (W == 0.) ? fabs(W - W_old) : fabs((W - W_old) / W);
+        errx = (W == 0.) ? fabs(W - W_old) : fabs(fdiv(W - W_old, W));
         if ((fabs(errx) <= NEWT_TOL) && (f <= 1.e-4) && (doing_extra == 0)) doing_extra = 1;
         if (doing_extra == 1) i_extra++;
         if (((fabs(errx) <= NEWT_TOL) && (doing_extra == 0)) || (i_extra > EXTRA_NEWT_ITER) ||

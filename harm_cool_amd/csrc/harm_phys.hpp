@@ -91,6 +91,34 @@ __host__ __device__ inline double div_r(double a, double b, double rb)
     return copysign(q2, q0);
 }
 
+// a / b and sqrt(x), correctly rounded, without the scaling that the compiler's sequences
+// carry for operands next to the ends of the exponent range: the reciprocal (square root)
+// estimate, two refinements and a corrected quotient (two corrected roots) by FMA residuals,
+// the very operations that the full sequences run where they do not scale.  Holds for |a|
+// = 0 or above 2^-960, |b| in 2^+-700 and a quotient in 2^+-700, for x = 0 or above 2^-767;
+// zeros, infinities and NaN come out as by IEEE division.  The kernels of the step are
+// bound by their FP64 instructions, of which divisions and roots were a third: 9
+// instructions for 11 and 12 for 17.
+HD double fdiv(double a, double b)
+{
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(fma(-b, r, 1.), r, r);
+    r = fma(fma(-b, r, 1.), r, r);
+    const double q = a * r;
+    return __builtin_amdgcn_div_fixup(fma(fma(-b, q, a), r, q), b, a);
+}
+HD double fsqrt(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
+    h = fma(h, r, h);
+    g = fma(g, r, g);
+    g = fma(fma(-g, g, x), h, g);
+    g = fma(fma(-g, g, x), h, g);
+    return (x == 0. || x == __builtin_inf()) ? x : g;
+}
+
 struct State {
     double ucon[4], ucov[4], bcon[4], bcov[4];
 };
@@ -352,7 +380,7 @@ HD int gamma_calc(const double *pr, const Geom &geom, double *gamma)
         }
         qsq = 1.E-10;
     }
-    *gamma = sqrt(1. + qsq);
+    *gamma = fsqrt(1. + qsq);
     return 0;
 }
 
@@ -372,7 +400,7 @@ HD void ucon_calc(const double *pr, const Geom &geom, double *ucon, int &fatal)
 HD void bcon_calc(const double *pr, const double *ucon, const double *ucov, double *bcon)
 {
     bcon[0] = pr[B1] * ucov[1] + pr[B2] * ucov[2] + pr[B3] * ucov[3];
-    const double r0 = 1. / ucon[0];
+    const double r0 = fdiv(1., ucon[0]);
 #pragma unroll
     for (int j = 1; j < 4; j++) bcon[j] = div_r(pr[B1 - 1 + j] + bcon[0] * ucon[j], ucon[0], r0);
 }
@@ -458,7 +486,7 @@ HD int vchar(const double *pr, const State &q, const Geom &geom, int js, const E
     if constexpr (E::TAB) {
         double EF = rho + u + pt.p;
         double EE = bsq + EF;
-        double va2 = bsq / EE;
+        double va2 = fdiv(bsq, EE);
         double cs2 = eos.cs2(rho, u, pt);
         cms2 = cs2 + va2 - cs2 * va2;
         if (cms2 < SMALL) cms2 = SMALL;
@@ -467,8 +495,8 @@ HD int vchar(const double *pr, const State &q, const Geom &geom, int js, const E
         const double gam = eos.gam;
         double EF = rho + gam * u;
         double EE = bsq + EF;
-        double va2 = bsq / EE;
-        double cs2 = gam * (gam - 1.) * u / EF;
+        double va2 = fdiv(bsq, EE);
+        double cs2 = fdiv(gam * (gam - 1.) * u, EF);
         cms2 = cs2 + va2 - cs2 * va2;
         if (cms2 < 0.) {
             nfail++;
@@ -496,9 +524,9 @@ HD int vchar(const double *pr, const State &q, const Geom &geom, int js, const E
         nfail++;
         discr = 0.;
     }
-    discr = sqrt(discr);
-    double vp = -(-B + discr) / (2. * A);
-    double vm = -(-B - discr) / (2. * A);
+    discr = fsqrt(discr);
+    double vp = fdiv(-(-B + discr), 2. * A);
+    double vm = fdiv(-(-B - discr), 2. * A);
     if (vp > vm) {
         *vmax = vp;
         *vmin = vm;
@@ -596,7 +624,7 @@ HD void face_flux(const double *p_l, const double *p_r, const Geom &geom, int di
     double cmax = fabs(dmax(dmax(0., cmax_l), cmax_r));
     double cmin = fabs(dmax(dmax(0., -cmin_l), -cmin_r));
     ctop = dmax(cmax, cmin);
-    const double den = cmax + cmin + SMALL, rden = 1. / den;
+    const double den = cmax + cmin + SMALL, rden = fdiv(1., den);
 #pragma unroll
     for (int k = 0; k < NPR; k++)
         F[k] = hllf * div_r(cmax * F_l[k] + cmin * F_r[k] - cmax * cmin * (U_r[k] - U_l[k]), den, rden) +
@@ -708,7 +736,7 @@ HD double vsq_calc(const U2P &s, double W)
 {
     double Wsq = W * W;
     double Xsq = (s.Bsq + W) * (s.Bsq + W);
-    return ((Wsq * s.Qtsq + s.QdotBsq * (s.Bsq + 2. * W)) / (Wsq * Xsq));
+    return fdiv(Wsq * s.Qtsq + s.QdotBsq * (s.Bsq + 2. * W), Wsq * Xsq);
 }
 
 // utoprim_2d.c:562-624 with the Gamma-law EOS of utoprim_2d.c:645-678
@@ -717,22 +745,22 @@ HD void func_vsq(const U2P &s, double W, double vsq, double &dx0, double &dx1, d
     const double GAMMA = s.gam;
     double Wsq = W * W;
     double gtmp = 1. - vsq;
-    double p_tmp = div_r((GAMMA - 1.) * (W * gtmp - s.D * sqrt(gtmp)), GAMMA, s.rgam);
+    double p_tmp = div_r((GAMMA - 1.) * (W * gtmp - s.D * fsqrt(gtmp)), GAMMA, s.rgam);
     double dPdW = div_r((GAMMA - 1.) * (1. - vsq), GAMMA, s.rgam);
-    double dPdvsq = div_r((GAMMA - 1.) * (0.5 * s.D / sqrt(1. - vsq) - W), GAMMA, s.rgam);
+    double dPdvsq = div_r((GAMMA - 1.) * (fdiv(0.5 * s.D, fsqrt(1. - vsq)) - W), GAMMA, s.rgam);
     double t2 = -0.5 * s.Bsq + dPdvsq;
     double t3 = s.Bsq + W;
     double t4 = t3 * t3;
-    double t9 = 1. / Wsq;
+    double t9 = fdiv(1., Wsq);
     double t11 = s.Qtsq - vsq * t4 + s.QdotBsq * (s.Bsq + 2.0 * W) * t9;
     double t16 = s.QdotBsq * t9;
     double t18 = -s.Qdotn - 0.5 * s.Bsq * (1.0 + vsq) + 0.5 * t16 - W + p_tmp;
-    double t21 = 1. / t3;
-    double t23 = 1. / W;
+    double t21 = fdiv(1., t3);
+    double t23 = fdiv(1., W);
     double t24 = t16 * t23;
     double t25 = -1.0 + dPdW - t24;
     double t35 = t25 * t3 + (s.Bsq - 2.0 * dPdvsq) * (s.QdotBsq + vsq * Wsq * W) * t9 * t23;
-    double t36 = 1. / t35;
+    double t36 = fdiv(1., t35);
     dx0 = -(t2 * t11 + t4 * t18) * t21 * t36;
     double t40 = (vsq + t24) * t3;
     dx1 = -(-t25 * t11 - 2.0 * t40 * t18) * t21 * t36;
@@ -770,8 +798,8 @@ HD void gnr_step(const U2P &s, Gnr2 &g)
     double xo0 = g.x0;
     g.x0 += dx0;
     g.x1 += dx1;
-    g.errx = (g.x0 == 0.) ? fabs(dx0) : fabs(dx0 / g.x0);
-    g.errx += (g.x1 == 0.) ? fabs(dx1) : fabs(dx1 / g.x1);
+    g.errx = (g.x0 == 0.) ? fabs(dx0) : fabs(fdiv(dx0, g.x0));
+    g.errx += (g.x1 == 0.) ? fabs(dx1) : fabs(fdiv(dx1, g.x1));
     g.x0 = fabs(g.x0);
     g.x0 = (g.x0 > W_TOO_BIG) ? xo0 : g.x0;
     g.x1 = (g.x1 < 0.) ? 0. : g.x1;
@@ -825,7 +853,7 @@ HD void u2p_recover_vel(const U2P &s, const double *Bcon, const double *Qcon, co
 #pragma unroll
     for (int i = 1; i < 4; i++) {
         double Qtcon = Qcon[i] + ncon[i] * s.Qdotn;
-        prim[U1 + i - 1] = gamma / (W + s.Bsq) * (Qtcon + QdotB * Bcon[i] / W);
+        prim[U1 + i - 1] = fdiv(gamma, W + s.Bsq) * (Qtcon + fdiv(QdotB * Bcon[i], W));
     }
 }
 
@@ -846,8 +874,8 @@ HD bool guess_W(const U2P &s, const Geom &geom, const double *prim, double &W_la
     if ((utsq < 0.) && (fabs(utsq) < 1.0e-13)) utsq = fabs(utsq);
     if (utsq < 0. || utsq > UTSQ_TOO_BIG) return false;
     double gammasq = 1. + utsq;
-    double gamma = sqrt(gammasq);
-    double rho0 = s.D / gamma;
+    double gamma = fsqrt(gammasq);
+    double rho0 = fdiv(s.D, gamma);
     double u = prim[UU];
     double p = (s.gam - 1.) * u;
     double w = rho0 + u + p;
@@ -877,8 +905,8 @@ HD int finish_2d(U2P &s, const double *Bcon, const double *Qcon, const double *n
     if ((retval != 0) || (W == FAIL_VAL)) return retval * 100 + 1;
     if (W <= 0. || W > W_TOO_BIG) return 3;
     if (vsq >= 1.) return 4;
-    double gtmp = sqrt(1. - vsq);
-    double gamma = 1. / gtmp;
+    double gtmp = fsqrt(1. - vsq);
+    double gamma = fdiv(1., gtmp);
     double rho0 = s.D * gtmp;
     double w = W * (1. - vsq);
     double p = div_r((s.gam - 1.) * (w - rho0), s.gam, s.rgam);
