@@ -2964,8 +2964,13 @@ __global__ void __launch_bounds__(TPB) k_dump_cols(DGrid g, const double *__rest
 // (all lanes take part in the wave-level forward pass, so there is no early exit).
 // FONT: the Font fix where the inversion fails; its solvers would double the
 // registers of the others (2 and 1 wavefronts a SIMD), so they have kernels without it.
-template <int GUESS, bool FONT>
-__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(FONT ? 1 : GUESS ? 3 : 4, 8))) k_c2p_batch(const double *__restrict__ U, const double *__restrict__ gcov,
+// WIDE: the network's operands in LDS and registers for 3 wavefronts a SIMD, for batches
+// of more than one (C2P_WIDE zones, a block on each of 256 CUs); a smaller one has no use
+// for them and keeps the operands where it reads them (20,000 gated zones 33 us, WIDE 41;
+// 200,000 from the seed on every zone 84 us, WIDE 65).
+constexpr size_t C2P_WIDE = 256 * TPB;
+template <int GUESS, bool FONT, bool WIDE>
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(FONT ? 1 : GUESS == 0 ? 4 : WIDE ? 3 : 1, 8))) k_c2p_batch(const double *__restrict__ U, const double *__restrict__ gcov,
                                                    const double *__restrict__ gcon, const double *__restrict__ gdet,
                                                    double *__restrict__ prim, int8_t *__restrict__ ret,
                                                    uint8_t *__restrict__ iters, uint8_t *__restrict__ kconv, size_t n,
@@ -2975,10 +2980,6 @@ __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(FONT ?
     const size_t z = (size_t)blockIdx.x * TPB + threadIdx.x;
     const bool act = z < n;
     if (!GUESS && !act) return;
-    if constexpr (GUESS != 0) {
-        __shared__ MlpLds lds;
-        mlp = mlp_stage(mlp, lds);
-    }
     Geom geom;
     double Uz[NPR], pr[NPR];
     if (act) {
@@ -2988,21 +2989,32 @@ __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(FONT ?
             geom.gcon[a / 4][a % 4] = gcon[(size_t)a * n + z];
         }
         geom.g = gdet[z];
-        geom_derive(geom);
 #pragma unroll
         for (int k = 0; k < NPR; k++) {
             Uz[k] = U[(size_t)k * n + z];
             pr[k] = prim[(size_t)k * n + z];
         }
     }
+    if constexpr (GUESS == 1 && WIDE) {  // after the zone's reads, which it need not wait for
+        __shared__ MlpLds lds;
+        mlp = mlp_stage(mlp, lds);
+    }
+    if (act) geom_derive(geom);
     int niter = 0, kc = 0, r = 0;
     if constexpr (GUESS == 2) {
-        // gated: the network only for the waves with a zone whose plain start is poor
+        // gated: the network only for the waves with a zone whose plain start is poor, its
+        // operands only for the blocks with such a wave
         Gnr2 st;
         bool need = false;
         int ph1 = 0;
         if (act) ph1 = u2p_gate_first(Uz, geom, gam, pr, gate_tau, st, need);
         double W0 = 0., vsq0 = 0.;
+        if constexpr (WIDE) {
+            if (__syncthreads_or(need)) {
+                __shared__ MlpLds lds;
+                mlp = mlp_stage(mlp, lds);
+            }
+        }
         if (__any(need)) {
             double f[MLP_NIN];
             const bool ok = need && mlp_features_U(Uz, geom, f);
@@ -3013,7 +3025,7 @@ __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(FONT ?
 #pragma unroll
                 for (int k = 0; k < MLP_NIN; k++) x[k] = 0.f;
             float y0, y1;
-            mlp_forward_wave<true>(mlp, x, y0, y1);
+            mlp_forward_wave<WIDE>(mlp, x, y0, y1);
             if (ok) mlp_unstandardize(mlp, y0, y1, mlp_wref(f), W0, vsq0);
         }
         if (!act) return;
@@ -3029,7 +3041,7 @@ __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(FONT ?
 #pragma unroll
             for (int k = 0; k < MLP_NIN; k++) x[k] = 0.f;
         float y0, y1;
-        mlp_forward_wave<true>(mlp, x, y0, y1);
+        mlp_forward_wave<WIDE>(mlp, x, y0, y1);
         if (!act) return;
         double W0 = 0., vsq0 = 0.;
         if (ok) mlp_unstandardize(mlp, y0, y1, mlp_wref(f), W0, vsq0);
@@ -4977,12 +4989,13 @@ int harm_utoprim2d_batch(const double *U, const double *gcov, const double *gcon
     } else if (opts->guess_mode != 0) {
         return set_err("unknown guess_mode", 4);
     }
-    auto *k = opts->font_fix ? (opts->guess_mode == 0   ? k_c2p_batch<0, true>
-                                : opts->guess_mode == 1 ? k_c2p_batch<1, true>
-                                                        : k_c2p_batch<2, true>)
-                             : (opts->guess_mode == 0   ? k_c2p_batch<0, false>
-                                : opts->guess_mode == 1 ? k_c2p_batch<1, false>
-                                                        : k_c2p_batch<2, false>);
+    const int gm = opts->guess_mode;
+    const bool wide = n > C2P_WIDE;
+    auto *k = opts->font_fix ? (gm == 0 ? k_c2p_batch<0, true, false> : gm == 1 ? k_c2p_batch<1, true, false>
+                                                                             : k_c2p_batch<2, true, false>)
+              : gm == 0      ? k_c2p_batch<0, false, false>
+              : gm == 1      ? (wide ? k_c2p_batch<1, false, true> : k_c2p_batch<1, false, false>)
+                             : (wide ? k_c2p_batch<2, false, true> : k_c2p_batch<2, false, false>);
     hipLaunchKernelGGL(k, dim3(nblocks(n)), dim3(TPB), 0, (hipStream_t)stream, U, gcov, gcon, gdet, prim, ret, iters,
                        kconv, n, opts->gam, opts->K, (int *)nullptr, mv, gate);
     HIPCHK(hipGetLastError());
@@ -5168,7 +5181,7 @@ int Utoprim_2d(double U[8], double gcov[4][4], double gcon[4][4], double gdet, d
     if (rc) return rc;
     MlpDev mv;
     std::memset(&mv, 0, sizeof(mv));
-    hipLaunchKernelGGL((k_c2p_batch<0, false>), dim3(1), dim3(TPB), 0, 0, s.buf, s.buf + 8, s.buf + 24, s.buf + 40,
+    hipLaunchKernelGGL((k_c2p_batch<0, false, false>), dim3(1), dim3(TPB), 0, 0, s.buf, s.buf + 8, s.buf + 24, s.buf + 40,
                        s.buf + 41, s.ret8, (uint8_t *)nullptr, (uint8_t *)nullptr, (size_t)1, g_gamma, 0., s.ret, mv,
                        0.);
     HIPCHK(hipGetLastError());
