@@ -215,7 +215,12 @@ __global__ void __launch_bounds__(64) k_abundance(const double *__restrict__ rho
 // table over rho 1e6-1e13, T 1e9-1e12 took 21.3 s and a 40x40 one over its
 // dense part (rho > 1e10, T 1e10-1e11) 125 ms; now 0.10 s and 3.1 ms.  A single
 // 4x4 patch at T < 3e9 K, whose outer solves cycle, went from 12 s to 4 ms.
+// out: rows of n (a call of more points than a launch takes passes the first of them).
 constexpr int TPB_P = 192;
+// A launch holds fewer than 2^32 threads: the runtime takes a larger one modulo that, with
+// no error.  Each of these launches runs for a second or more, so their number costs nothing.
+constexpr size_t POINTS_LAUNCH = (size_t)1 << 22;
+static_assert(POINTS_LAUNCH * TPB_P < (1ull << 32), "one launch");
 __global__ void __launch_bounds__(TPB_P) k_abundance_wave(const double *__restrict__ rho,
                                                           const double *__restrict__ T,
                                                           const double *__restrict__ hdfac,
@@ -277,9 +282,13 @@ int harm_eos_point_batch(const double *rho, const double *T, const double *hdfac
     hipStream_t s = (hipStream_t)stream;
     int rc = upload_rules();
     if (rc) return rc;
-    if (n > 0x7fffffffu) return harm_host::set_error("harm_eos_point_batch: too many points for one call", 3);
-    hipLaunchKernelGGL(k_abundance_wave, dim3((unsigned)n), dim3(TPB_P), 0, s, rho, T, hdfac, out, n);
-    FCHK(hipGetLastError());
+    if (n / 8 > 0x7fffffffu) return harm_host::set_error("harm_eos_point_batch: too many points for one call", 3);
+    for (size_t at = 0; at < n; at += POINTS_LAUNCH) {
+        const size_t m = std::min(n - at, POINTS_LAUNCH);
+        hipLaunchKernelGGL(k_abundance_wave, dim3((unsigned)m), dim3(TPB_P), 0, s, rho + at, T + at, hdfac + at, out + at,
+                           n);
+        FCHK(hipGetLastError());
+    }
     FCHK(hipStreamSynchronize(s));
     return 0;
 }

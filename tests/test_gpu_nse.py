@@ -67,3 +67,25 @@ def test_points_match_serial_chain():
     ref = np.array([p[1] for p in POINTS]).T
     got = _batch(hc.lib().harm_eos_point_batch, *ins)
     assert np.all(np.abs(got - ref) <= 1e-9 * np.abs(ref)), np.abs(got / ref - 1).max(axis=1)
+
+
+def test_more_points_than_one_launch_holds():
+    """2^32 threads and more: the points at the ends and at the launches' seams against
+    a call of those alone (1e11 g/cm^3, 1e13 K: the shortest chains, 0.3 us a point)."""
+    import torch
+
+    n, span = 2 ** 32 // 192 + 1, 1 << 22
+    at = torch.tensor([0, 1, 127, 128, span - 1, span, 3 * span - 1, 3 * span, n - 2, n - 1], device="cuda:0")
+    few = [torch.full((len(at),), v, dtype=torch.float64, device="cuda:0") for v in (1e11, 1e13, 6.28e-4)]
+    few[0] *= torch.linspace(0.5, 2.0, len(at), dtype=torch.float64, device="cuda:0")
+    many = [torch.full((n,), v, dtype=torch.float64, device="cuda:0") for v in (1e11, 1e13, 6.28e-4)]
+    many[0][at] = few[0]
+    got = []
+    for ins in (few, many):
+        out = torch.full((6, len(ins[0])), -1.0, dtype=torch.float64, device="cuda:0")
+        torch.cuda.synchronize()
+        assert hc.lib().harm_eos_point_batch(*(ctypes.c_void_p(t.data_ptr()) for t in ins),
+                                             ctypes.c_void_p(out.data_ptr()), len(ins[0]), None) == 0
+        got.append(out)
+    assert torch.equal(got[0], got[1][:, at])
+    assert bool((got[1] > 0).all())
