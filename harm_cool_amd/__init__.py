@@ -949,6 +949,18 @@ def device_pow(x: np.ndarray, y: np.ndarray) -> np.ndarray:
     return out
 
 
+def device_div_sqrt(a: np.ndarray, b: np.ndarray) -> "tuple[np.ndarray, np.ndarray]":
+    """The short division and root of the step's kernels, a / b and sqrt(a), evaluated on
+    the GPU (test entry)."""
+    L = lib()
+    L.harm_debug_div_sqrt.argtypes = [_dp, _dp, _dp, _dp, c_size_t]
+    a = np.ascontiguousarray(a, dtype=np.float64)
+    b = np.ascontiguousarray(b, dtype=np.float64)
+    q, r = np.empty_like(a), np.empty_like(a)
+    _check(L.harm_debug_div_sqrt(_ptr(a), _ptr(b), _ptr(q), _ptr(r), a.size), "harm_debug_div_sqrt")
+    return q, r
+
+
 def device_copy(nbytes: int, repeats: int = 10) -> float:
     """Time a plain device copy of nbytes; returns ms per copy (counter calibration)."""
     L = lib()

@@ -3273,6 +3273,15 @@ __global__ void __launch_bounds__(TPB) k_eos_eval(EosTab tab, const double *__re
     if (dpdu) dpdu[z] = b;
 }
 
+__global__ void __launch_bounds__(TPB) k_div_sqrt(const double *__restrict__ a, const double *__restrict__ b,
+                                                  double *__restrict__ q, double *__restrict__ r, size_t n)
+{
+    const size_t z = (size_t)blockIdx.x * TPB + threadIdx.x;
+    if (z >= n) return;
+    q[z] = fdiv(a[z], b[z]);
+    r[z] = fsqrt(a[z]);
+}
+
 __global__ void __launch_bounds__(TPB) k_pow(const double *__restrict__ x, const double *__restrict__ y,
                                              double *__restrict__ out, size_t n)
 {
@@ -5089,6 +5098,20 @@ int harm_debug_pow(const double *x, const double *y, double *out, size_t n)
     hipLaunchKernelGGL(k_pow, dim3(nblocks(n)), dim3(TPB), 0, 0, d, d + n, d + 2 * n, n);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpy(out, d + 2 * n, n * sizeof(double), hipMemcpyDeviceToHost));
+    HIPCHK(hipFree(d));
+    return 0;
+}
+
+int harm_debug_div_sqrt(const double *a, const double *b, double *q, double *r, size_t n)
+{
+    double *d = nullptr;
+    HIPCHK(hipMalloc((void **)&d, 4 * n * sizeof(double)));
+    HIPCHK(hipMemcpy(d, a, n * sizeof(double), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(d + n, b, n * sizeof(double), hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_div_sqrt, dim3(nblocks(n)), dim3(TPB), 0, 0, d, d + n, d + 2 * n, d + 3 * n, n);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpy(q, d + 2 * n, n * sizeof(double), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(r, d + 3 * n, n * sizeof(double), hipMemcpyDeviceToHost));
     HIPCHK(hipFree(d));
     return 0;
 }

@@ -94,11 +94,16 @@ __host__ __device__ inline double div_r(double a, double b, double rb)
 // a / b and sqrt(x), correctly rounded, without the scaling that the compiler's sequences
 // carry for operands next to the ends of the exponent range: the reciprocal (square root)
 // estimate, two refinements and a corrected quotient (two corrected roots) by FMA residuals,
-// the very operations that the full sequences run where they do not scale.  Holds for |a|
-// = 0 or above 2^-960, |b| in 2^+-700 and a quotient in 2^+-700, for x = 0 or above 2^-767;
-// zeros, infinities and NaN come out as by IEEE division.  The kernels of the step are
-// bound by their FP64 instructions, of which divisions and roots were a third: 9
-// instructions for 11 and 12 for 17.
+// the very operations that the full sequences run where they do not scale (Markstein's
+// correction on the hardware's estimate).  Hold for |a| = 0 or above 2^-960, |b| in 2^+-700
+// and a quotient in 2^+-700, for x = 0 or above 2^-767; zero, infinite and NaN operands and
+// negative x give what IEEE gives.  Beyond that they do not: a denominator below 2^-1022
+// and a quotient that overflows give NaN, smaller numerators and quotients a last bit off.
+// So they stand where the operands are a state's own sizes and ratios; a quotient by a
+// squared velocity, by a fourth power or of a product of small fields is a plain division
+// (gnr_step, vsq_calc, u2p_recover_vel).  The kernels of the step are bound by their FP64
+// instructions, of which divisions and roots were a third: 9 instructions for 11 and 12
+// for 17.
 HD double fdiv(double a, double b)
 {
     double r = __builtin_amdgcn_rcp(b);
@@ -736,7 +741,7 @@ HD double vsq_calc(const U2P &s, double W)
 {
     double Wsq = W * W;
     double Xsq = (s.Bsq + W) * (s.Bsq + W);
-    return fdiv(Wsq * s.Qtsq + s.QdotBsq * (s.Bsq + 2. * W), Wsq * Xsq);
+    return (Wsq * s.Qtsq + s.QdotBsq * (s.Bsq + 2. * W)) / (Wsq * Xsq);  // W^4: plain (fdiv)
 }
 
 // utoprim_2d.c:562-624 with the Gamma-law EOS of utoprim_2d.c:645-678
@@ -799,7 +804,11 @@ HD void gnr_step(const U2P &s, Gnr2 &g)
     g.x0 += dx0;
     g.x1 += dx1;
     g.errx = (g.x0 == 0.) ? fabs(dx0) : fabs(fdiv(dx0, g.x0));
-    g.errx += (g.x1 == 0.) ? fabs(dx1) : fabs(fdiv(dx1, g.x1));
+    // v^2 may be anything above 0 and dx1 is of its size or below 1: plain where fdiv ends
+    if (__builtin_expect(fabs(g.x1) < 0x1p-700, 0))
+        g.errx += (g.x1 == 0.) ? fabs(dx1) : fabs(dx1 / g.x1);
+    else
+        g.errx += fabs(fdiv(dx1, g.x1));
     g.x0 = fabs(g.x0);
     g.x0 = (g.x0 > W_TOO_BIG) ? xo0 : g.x0;
     g.x1 = (g.x1 < 0.) ? 0. : g.x1;
@@ -853,7 +862,7 @@ HD void u2p_recover_vel(const U2P &s, const double *Bcon, const double *Qcon, co
 #pragma unroll
     for (int i = 1; i < 4; i++) {
         double Qtcon = Qcon[i] + ncon[i] * s.Qdotn;
-        prim[U1 + i - 1] = fdiv(gamma, W + s.Bsq) * (Qtcon + fdiv(QdotB * Bcon[i], W));
+        prim[U1 + i - 1] = fdiv(gamma, W + s.Bsq) * (Qtcon + QdotB * Bcon[i] / W);
     }
 }
 

@@ -209,6 +209,9 @@ int harm_debug_fixup(harm_ctx *c);
 /* The device pow used by the Font-fix solvers (correctly rounded), on host arrays;
  * for tests against the host libm pow the reference calls. */
 int harm_debug_pow(const double *x, const double *y, double *out, size_t n);
+/* The short division a / b and root sqrt(a) of the step's kernels, on host arrays;
+ * for tests against IEEE over the exponents that they are stated for. */
+int harm_debug_div_sqrt(const double *a, const double *b, double *q, double *r, size_t n);
 /* A plain device-to-device copy of nbytes (1 + repeats launches): the reference
  * reading for the HBM traffic counters and the achievable copy bandwidth. */
 int harm_debug_copy(size_t nbytes, int repeats, double *ms_per_copy);
