@@ -2964,13 +2964,16 @@ __global__ void __launch_bounds__(TPB) k_dump_cols(DGrid g, const double *__rest
 // (all lanes take part in the wave-level forward pass, so there is no early exit).
 // FONT: the Font fix where the inversion fails; its solvers would double the
 // registers of the others (2 and 1 wavefronts a SIMD), so they have kernels without it.
-// WIDE: the network's operands in LDS and registers for 3 wavefronts a SIMD, for batches
-// of more than one (C2P_WIDE zones, a block on each of 256 CUs); a smaller one has no use
-// for them and keeps the operands where it reads them (20,000 gated zones 33 us, WIDE 41;
-// 200,000 from the seed on every zone 84 us, WIDE 65).
+// WIDE: the network's operands in LDS, for 3 wavefronts a SIMD from the seed on every zone
+// and 2 gated (which keeps the paused Newton state over the network: 34 spills at 3), for
+// batches of more than one (C2P_WIDE zones, a block on each of 256 CUs); a smaller one has no
+// use for them and keeps the operands where it reads them.  us a call, narrow / WIDE: every
+// zone 65,536 45.0 / 46.8, 65,537 58.8 / 52.8, 2^23 2520 / 1728; gated where every wavefront
+// asks 65,536 51.3 / 54.3, 65,537 54.6 / 53.6, 2^23 3324 / 2711, where none does 65,536 36.6 /
+// 37.5, 2^23 1645 / 1198 (at 3 wavefronts 1801).
 constexpr size_t C2P_WIDE = 256 * TPB;
 template <int GUESS, bool FONT, bool WIDE>
-__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(FONT ? 1 : GUESS == 0 ? 4 : WIDE ? 3 : 1, 8))) k_c2p_batch(const double *__restrict__ U, const double *__restrict__ gcov,
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(FONT ? 1 : GUESS == 0 ? 4 : WIDE ? (GUESS == 1 ? 3 : 2) : 1, 8))) k_c2p_batch(const double *__restrict__ U, const double *__restrict__ gcov,
                                                    const double *__restrict__ gcon, const double *__restrict__ gdet,
                                                    double *__restrict__ prim, int8_t *__restrict__ ret,
                                                    uint8_t *__restrict__ iters, uint8_t *__restrict__ kconv, size_t n,
