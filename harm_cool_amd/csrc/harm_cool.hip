@@ -1114,10 +1114,13 @@ __device__ __forceinline__ unsigned upd_tiled_row(unsigned b, unsigned G, unsign
 // falls back to the pi guess where the seeded solve fails.
 // FUSED forms the flux divergence in place (flux_div) instead of reading S.
 // The wave-uniform UPD_GATED update is held to the plain one's 4 waves per SIMD
-// (its seed-list store would otherwise take it past 128 VGPRs); every other
-// instance keeps the compiler's choice.
+// (its seed-list store would otherwise take it past 128 VGPRs), the wave-uniform
+// UPD_LEARNED one to 3 (a 128^3 step 1560 us, 1655 with the 127 VGPRs and 4 AGPRs of the
+// compiler's choice); every other instance keeps the compiler's choice (the learned
+// update of other grids spills 18 registers at 3: a 160x128x96 step 2257 us, now 1954;
+// 128x128 234 -> 187).
 template <bool UNI, int MODE, bool TAB, bool FUSED>
-__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu((UNI && MODE == UPD_GATED) ? 4 : MODE == UPD_LEARNED ? 3 : 1, 8)))
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(!UNI ? 1 : MODE == UPD_GATED ? 4 : MODE == UPD_LEARNED ? 3 : 1, 8)))
 k_update(DGrid g, const double *__restrict__ pi, const double *__restrict__ pb, double *__restrict__ pf,
          int8_t *__restrict__ pflag, const double *__restrict__ S, DivArgs dv, const double *__restrict__ tstate,
          double dtfac, int pi_is_pb, FontList fl, unsigned long long *__restrict__ cpart, UpdateExtra ex)
