@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -25,7 +26,11 @@ struct harm_cache {
     int whole;
     double *vx = nullptr, *vy = nullptr, *vz = nullptr, *values = nullptr;
     uint8_t *counted = nullptr;
-    double *tab = nullptr;  // the splines along y of every component (harm_cache.hpp), or null
+    // the splines along y of every component (harm_cache.hpp), or null: formed by the first
+    // lookup or solve that reads them (lookup_table)
+    mutable std::mutex tab_mu;
+    mutable bool tab_tried = false;
+    mutable double *tab = nullptr;
     int device = 0;
 };
 
@@ -200,26 +205,56 @@ size_t axes_lds(const harm_cache_desc &d)
     return b <= 16 * 1024 ? b : 0;
 }
 
-// Tables of at most 1 GiB (12 times the values' size); larger caches, and those whose
-// table finds no memory, are looked up from their values.
+// Tables of at most 1 GiB (12 times the values' size) that leave an eighth of the device's
+// memory free; larger caches, and those whose table finds no room, are looked up from their
+// values.  Formed by the first lookup, not with the cache: the step's caches (one per radius,
+// hundreds of them) are never looked up and keep tables of e and p alone with the context.
 constexpr size_t TAB_MAX = (size_t)1 << 30;
 
-int build_table(harm_cache *c)
+int form_table(const harm_cache *c, hipStream_t s)
 {
     const harm_cache_desc &d = c->desc;
     const size_t planes = (size_t)d.z * d.d, bytes = planes * harm::cache_tab_plane(d.x, d.y) * sizeof(double);
-    if (bytes > TAB_MAX || planes > 65535) return 0;
-    if (hipMalloc(&c->tab, bytes) != hipSuccess) {
+    size_t room = 0, all = 0;
+    int dev = -1;
+    if (bytes > TAB_MAX || planes > 65535 || hipGetDevice(&dev) != hipSuccess || dev != c->device) return 0;
+    if (hipMemGetInfo(&room, &all) != hipSuccess || room < bytes + all / 8) {
         (void)hipGetLastError();
-        c->tab = nullptr;
+        return 0;
+    }
+    // another thread's stream capture may not be broken by this thread's allocation
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    CCHK(hipThreadExchangeStreamCaptureMode(&mode));
+    double *t = nullptr;
+    const hipError_t e = hipMalloc(&t, bytes);
+    CCHK(hipThreadExchangeStreamCaptureMode(&mode));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
         return 0;
     }
     const size_t per = (size_t)d.x * d.y;
-    hipLaunchKernelGGL(k_cache_table, dim3((unsigned)((per + TPB_C - 1) / TPB_C), (unsigned)planes), dim3(TPB_C), 0, 0,
-                       view_of(c), c->tab);
-    CCHK(hipGetLastError());
-    CCHK(hipStreamSynchronize(0));
+    hipLaunchKernelGGL(k_cache_table, dim3((unsigned)((per + TPB_C - 1) / TPB_C), (unsigned)planes), dim3(TPB_C), 0, s,
+                       view_of(c), t);
+    // finished before another thread's stream may read it
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) {
+        (void)hipFree(t);
+        return harm_host::set_error("the cache's lookup table could not be formed", 2);
+    }
+    c->tab = t;
     return 0;
+}
+
+// The cache's table, formed on the caller's stream if this is its first use; null: none.
+int lookup_table(const harm_cache *c, hipStream_t s, const double *&tab)
+{
+    std::lock_guard<std::mutex> lk(c->tab_mu);
+    int rc = 0;
+    if (!c->tab_tried) {
+        rc = form_table(c, s);
+        c->tab_tried = rc == 0;
+    }
+    tab = c->tab;
+    return rc;
 }
 
 }  // namespace
@@ -392,7 +427,7 @@ harm_cache *harm_cache_create(const harm_cache_desc *desc, const double *vx, con
     for (size_t i = 0; i < np; i++) ones += counted[i] == 1;
     // a file that says it is whole is taken at its word, as the reference does
     c->whole = d.wholecachecalculated || ones == np;
-    if (cache_upload(c, vx, vy, vz, values, counted) || build_table(c)) {
+    if (cache_upload(c, vx, vy, vz, values, counted)) {
         harm_cache_free(c);
         return nullptr;
     }
@@ -447,12 +482,14 @@ int harm_cache_lookup(const harm_cache *c, int mode, const int *dimmask, const d
     const harm::CacheView v = view_of(c);
     hipStream_t s = (hipStream_t)stream;
     const dim3 grid((unsigned)((n + TPB_C - 1) / TPB_C)), block(TPB_C);
-    const bool tab = c->tab && mode == HARM_INTERP_SPLINE && zindex;
+    const double *tab = nullptr;
+    if (mode == HARM_INTERP_SPLINE && zindex)
+        if (const int rc = lookup_table(c, s, tab)) return rc;
     if (tab) {
         const size_t lds = axes_lds(c->desc);
         auto *k = dery ? (lds ? k_lookup_tab<true, true> : k_lookup_tab<true, false>)
                        : (lds ? k_lookup_tab<false, true> : k_lookup_tab<false, false>);
-        hipLaunchKernelGGL(k, grid, block, lds, s, v, c->tab, mask, x, y, z, zindex, out, dery, status, n);
+        hipLaunchKernelGGL(k, grid, block, lds, s, v, tab, mask, x, y, z, zindex, out, dery, status, n);
         CCHK(hipGetLastError());
     }
     if (!tab || c->desc.z >= 3) {
@@ -484,15 +521,17 @@ int harm_cache_solve_T(const harm_cache *c, const double *rho, const double *e, 
     const harm::CacheView v = view_of(c);
     hipStream_t s = (hipStream_t)stream;
     const dim3 grid((unsigned)((n + TPB_C - 1) / TPB_C)), block(TPB_C);
-    if (c->tab) {
+    const double *tab = nullptr;
+    if (const int rc = lookup_table(c, s, tab)) return rc;
+    if (tab) {
         const size_t lds = axes_lds(c->desc);
-        hipLaunchKernelGGL(lds ? k_solve_tab<true> : k_solve_tab<false>, grid, block, lds, s, v, c->tab, rho, e, zindex,
+        hipLaunchKernelGGL(lds ? k_solve_tab<true> : k_solve_tab<false>, grid, block, lds, s, v, tab, rho, e, zindex,
                            T, Tlo, Thi, ntrial, tolf, berr, ret, n);
         CCHK(hipGetLastError());
     }
-    if (!c->tab || (zindex && c->desc.z >= 3)) {
+    if (!tab || (zindex && c->desc.z >= 3)) {
         hipLaunchKernelGGL(k_cache_solve_T, grid, block, 0, s, v, rho, e, zindex, T, Tlo, Thi, ntrial, tolf, berr, ret,
-                           n, !c->tab);
+                           n, !tab);
     }
     CCHK(hipGetLastError());
     CCHK(hipStreamSynchronize(s));

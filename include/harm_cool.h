@@ -511,7 +511,10 @@ void harm_cache_free(harm_cache *c);
  * and -1 interpolates in z; out[d][n]; dery[d][n] (may be NULL) the derivative
  * along y (spline only); status[n] (may be NULL) HARM_CACHE_*.  dimmask (host,
  * d ints, may be NULL = all) selects the components the spline computes; the
- * others, like every output of a point whose status is not 1, are not written. */
+ * others, like every output of a point whose status is not 1, are not written.
+ * The first spline lookup with zindex, or temperature solve, of a cache forms a table
+ * of its splines along y (12 times the values' size, at most 1 GiB, kept with the
+ * cache; none where that would not leave an eighth of the device's memory free). */
 int harm_cache_lookup(const harm_cache *c, int mode, const int *dimmask, const double *x, const double *y,
                       const double *z, const int *zindex, double *out, double *dery, int *status, size_t n,
                       void *stream);
