@@ -123,7 +123,7 @@ __device__ __forceinline__ void stage_axes(const harm::CacheView &c, double *ax,
 // One query per thread, its windows found once and then the components one after
 // another.  Bound by the FP64 VALU: 22 divisions and about 300 other operations a
 // component with the derivative (2^21 points of a 200x200 table, six values and their
-// derivatives: 418 us a call; with every spline fitted per query, 4300 us).
+// derivatives: 283 us, 319 a call; with every spline fitted per query, 4300 us a call).
 template <bool DER, bool AX>
 __global__ void __launch_bounds__(TPB_C) k_lookup_tab(harm::CacheView c, const double *__restrict__ tab, uint64_t mask,
                                                       const double *__restrict__ x, const double *__restrict__ y,
@@ -156,8 +156,8 @@ __global__ void __launch_bounds__(TPB_C) k_lookup_tab(harm::CacheView c, const d
     }
 }
 
-// One solve per thread, about four trials each (2^21 solves from starts 5% off: 290 us a
-// call; with every spline fitted per trial, 1350 us).
+// One solve per thread, about four trials each (2^21 solves from starts 5% off: 237 us, 256
+// a call; with every spline fitted per trial, 1350 us a call).
 template <bool AX>
 __global__ void __launch_bounds__(TPB_C) k_solve_tab(harm::CacheView c, const double *__restrict__ tab,
                                                      const double *__restrict__ rho, const double *__restrict__ e,

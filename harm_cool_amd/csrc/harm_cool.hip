@@ -899,10 +899,11 @@ __device__ __forceinline__ void flux_div(const DGrid &g, const DivArgs &a, int i
     }
 }
 
-// flux_div with 32-bit zone offsets (nz < OFF32_MAX_ZONES, N3 > 2); the same
-// operations in the same order.  The twelve corner EMFs it needs are formed
-// here from the face B-fluxes with k_emf's expressions (step_ch.c:773-781), so
-// the fused update needs no EMF pass.
+// flux_div with 32-bit zone offsets (nz < OFF32_MAX_ZONES); the same operations
+// in the same order.  The twelve corner EMFs it needs (four in two dimensions,
+// which only the grids that are not wave-uniform can have) are formed here from
+// the face B-fluxes with k_emf's expressions (step_ch.c:773-781), so the fused
+// update needs no EMF pass.
 template <bool UNI>
 __device__ __forceinline__ void flux_div32(const DGrid &g, const DivArgs &a, int i, int j, int h, double *d)
 {
@@ -1319,7 +1320,9 @@ k_update(DGrid g, const double *__restrict__ pi, const double *__restrict__ pb, 
 // ---------------------------------------------------------------------------
 
 // Wavefronts a SIMD of the cache-EOS kernels: two for the inversion's 256 registers,
-// three for the solves of faces and zones (165).
+// three for the solves of faces and zones (165; with resolved derivative steps, five solves
+// a state, 24-31 of 168 spill, which still is no slower: a 96^3 step 5.70 ms and a 128x128 one
+// 1.01, at two 5.81 and 0.99).
 constexpr int CEOS_WPE = 2, CEOS_EOS_WPE = 3;
 
 // The tables of the splines along T of e and p of cache blockIdx.y (cache_tab_fill): one
@@ -3760,8 +3763,9 @@ int advance(harm_ctx *c, double *pi, double *pb, double *pf, double dtfac, int f
         c->cap_phase = (int)((ph + 7919) % (size_t)c->cap_stride);
     }
     const DivArgs dv = {c->F1, c->F2, c->F3, c->e1, c->e2, c->e3};
-    // the plain wave-uniform update forms the EMFs and the divergence itself; the
-    // others read S, which k_div forms from the EMF arrays
+    // the update forms the EMFs and the divergence itself; in the capture of pairs and in
+    // the learned start of grids that are not wave-uniform, and on grids beyond 32-bit
+    // offsets, it reads S, which k_div forms from the EMF arrays
     const bool fused = c->nz < OFF32_MAX_ZONES &&
                        (c->eos_kind == 1 || (c->uniform ? mode != UPD_CAPTURE : mode == UPD_PLAIN || mode == UPD_GATED));
     if ((rc = fluxes_and_emf(c, pb, fullstep, !fused))) return rc;

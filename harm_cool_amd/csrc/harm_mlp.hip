@@ -68,9 +68,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // coming from LDS (rows of TR_LD floats: 16-byte reads along a row and 4-byte reads
 // across rows both touch every bank once).  A weight gradient contracts over the batch
 // rows, for which D would have to be rows x neurons: each layer's h and dZ pass
-// through LDS once and are read back in that order.  The 8 + 128 accumulator tiles of
-// a wavefront (dW1 with db1 as its ninth column, dW2, dW3) stay in registers over all
-// its rows.
+// through LDS once and are read back in that order.  The 36 accumulator tiles of a
+// wavefront (dW1 with db1 as its ninth column, dW2, dW3: 144 registers) are kept over all
+// its rows; with the products' operands 60 of its registers go to scratch (136 B a lane).
 //
 // Bound by the FP32 matrix cores: 408 MFMA of 32 cycles per 16 rows.  Two wavefronts
 // a SIMD (256 registers each) let one's 48 tanhf a lane run beside the other's
@@ -162,9 +162,9 @@ __device__ __forceinline__ void tr_wgrad(const float *dz, const float *h, int q,
 
 // tanh without a branch (the library's takes one of two per lane, so a wavefront runs
 // both and the loads around them wait): an odd polynomial below 0.9, fitted there to a
-// relative error of 1.1e-9, and 1 - 2 / (exp(2|x|) + 1) above.  Against 64 bits over 4e6
-// arguments in [-12, 12]: 2.1e-8 rms, 1.8e-7 at most (the library's: 2.0e-8, 1.4e-7; the
-// trained parameters' error is the same).
+// relative error of 6e-9, and 1 - 2 / (exp(2|x|) + 1) above.  Relative error against 64 bits
+// over 4e6 arguments in [-12, 12]: 1.73e-8 rms, 1.06e-7 at most (the library's: 1.76e-8,
+// 1.42e-7); over 4e6 in [1e-30, 1] 8.9e-9 and 1.06e-7 (9.2e-9 and 1.41e-7).
 __device__ __forceinline__ float tr_tanhf(float x)
 {
     const float ax = __builtin_fabsf(x), y = x * x;

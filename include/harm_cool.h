@@ -61,7 +61,10 @@ enum {
     HARM_NCOUNTERS
 };
 
-/* Kernel classes timed with HIP events when timing is enabled. */
+/* Kernel classes timed with HIP events when timing is enabled.  Grids whose phi rows are
+ * no multiple of 64 take the fluxes of every direction in one launch, counted under
+ * HARM_K_FLUX1 (the cache EOS excepted); EMF and DIV are launches of their own only where
+ * the update does not form them. */
 enum {
     HARM_K_FLUX1 = 0, HARM_K_FLUX2, HARM_K_FLUX3, HARM_K_EMF, HARM_K_UPDATE,
     HARM_K_BOUND, HARM_K_FIXUTOPRIM, HARM_K_STEPEND, HARM_K_C2P_BATCH, HARM_K_MLP, HARM_K_FONTFIX,
