@@ -59,7 +59,7 @@ ALG_BYTES = {
 # One wave instruction per CU per cycle: 256 CUs at 2.4 GHz (FP64 FMA is full rate).
 VALU_PEAK_WAVE_INSTR_PER_S = 256 * 2.4e9
 PROFILED_KERNEL = {"flux1": "k_flux_strip<1, false, 0>", "flux2": "k_flux_strip<2, false, 0>",
-                   "flux3": "k_flux<3, true, false, 0, true>", "update": "k_update<true, 0, false, true>"}
+                   "flux3": "k_flux<3, false, 0, true>", "update": "k_update<true, 0, false, true>"}
 
 
 def measured_valu(kernel: str, n1: int, n2: int, n3: int):
